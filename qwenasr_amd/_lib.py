@@ -136,11 +136,25 @@ def lib() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Call entry point ``name``; raise QasrError on a non-zero status."""
-    so = lib()
-    rc = getattr(so, name)(*args)
+    rc = getattr(lib(), name)(*args)
     if rc != QASR_OK:
-        msg = so.qasr_last_error().decode(errors="replace")
-        raise QasrError(name, rc, msg)
+        raise_status(name, rc)
+
+
+def raise_status(name: str, rc: int) -> None:
+    raise QasrError(name, rc, lib().qasr_last_error().decode(errors="replace"))
+
+
+def bind(need, dtypes: tuple) -> dict:
+    """The entry points as functions of the binding extension (csrc/binding.cpp),
+    by name; ``need`` raises what is wrong with a tensor argument."""
+    so = lib()
+    try:
+        from . import _binding
+    except ImportError as e:
+        raise QasrLibraryMissing(
+            f"qwenasr_amd/_binding.so cannot be loaded ({e}): build it with `python -m qwenasr_amd.build`") from e
+    return _binding.setup(lambda name: ctypes.cast(getattr(so, name), c_void_p).value, need, raise_status, dtypes)
 
 
 def version() -> tuple[int, int, int]:

@@ -3,6 +3,8 @@
 Compiles every ``csrc/*.hip`` with hipcc for gfx950 and produces, in-tree:
 
 * ``qwenasr_amd/libqasr_hip.so`` -- shared library the Python and C++ hosts load;
+* ``qwenasr_amd/_binding.so``     -- the Python extension through which ``kernels.py``
+  calls it (host code only, against torch's headers);
 * ``qwenasr_amd/libqasr_hip.a``  -- static archive for a host that links it
   statically (a Rust ``build.rs`` would add ``cargo:rustc-link-lib=static=qasr_hip``
   plus ``amdhip64``).
@@ -15,6 +17,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -22,6 +25,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 SO = PKG / "libqasr_hip.so"
+BINDING = PKG / "_binding.so"
 ARCHIVE = PKG / "libqasr_hip.a"
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 
@@ -59,6 +63,20 @@ def _run(cmd: list[str]) -> None:
         raise RuntimeError(f"command failed ({r.returncode}): {' '.join(cmd)}")
 
 
+def binding_command(out: Path) -> list[str]:
+    """The compile line of the Python binding: plain host C++ that calls the
+    entry points by address, so it links torch but not the kernel library."""
+    import torch
+
+    t = Path(torch.__file__).resolve().parent
+    incs = [t / "include", t / "include" / "torch" / "csrc" / "api" / "include", ROCM / "include",
+            Path(sysconfig.get_paths()["include"])]
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *[f"-I{i}" for i in incs], str(CSRC / "binding.cpp"), "-o", str(out),
+            f"-L{t / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+
+
 def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
@@ -77,9 +95,18 @@ def build(verbose: bool = False) -> Path:
             print(" ".join(cmd), flush=True)
         _run(cmd)
 
+    binding = BUILD / "_binding.so"
+
+    def compile_binding(_):
+        _run(binding_command(binding))
+
     workers = min(len(srcs), max(1, (os.cpu_count() or 4)))
     with ThreadPoolExecutor(max_workers=workers) as ex:
-        list(ex.map(compile_one, zip(srcs, objs)))
+        jobs = [ex.submit(compile_binding, None)]
+        jobs += [ex.submit(compile_one, pair) for pair in zip(srcs, objs)]
+        for j in jobs:
+            j.result()
+    os.replace(binding, BINDING)
 
     tmp_so = SO.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp_so),

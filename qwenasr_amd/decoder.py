@@ -151,8 +151,9 @@ class DecoderInt8:
         x = self.px
         x[:T * H].copy_(embeds[:T * H])
         layers = self.w["layers"]
+        k_blocks, v_blocks = self.kv.layer_blocks()
         for l, lw in enumerate(layers):
-            kb, vb = self.kv.k_layer_block(l), self.kv.v_layer_block(l)
+            kb, vb = k_blocks[l], v_blocks[l]
             if fold and l > 0 and fused_heads:  # input norm: h * gain and the sums of squares from down
                 K.rms_norm_qkv_heads_int8(self.pq, kb, vb, self.kv.max_seq, lw["wq"], lw["wk"], lw["wv"], self.pxn,
                                           self.pss, eps, self.pxn, T, H, nq, nk, hd, lw["q_norm"], lw["k_norm"],
@@ -162,7 +163,7 @@ class DecoderInt8:
                     K.rms_norm(self.pxn, x, lw["input_norm"], T, H, eps)
                 else:  # previous layer's residual add (decoder.rs:837-838) + this layer's input norm
                     K.add_rms_norm(x, self.pffn, lw["input_norm"], self.pxn, T, H, eps)
-                self._prefill_qkv(l, lw, T, start_pos, fused_heads)
+                self._prefill_qkv(kb, vb, lw, T, start_pos, fused_heads)
             K.causal_attention(self.pattn, self.pq, kb, vb, T, total, nq, nk, hd, self.scale, start_pos)
             wo, dn = lw["wo"], lw["down"]
             if fold:
@@ -181,11 +182,10 @@ class DecoderInt8:
             K.add_inplace(x, self.pffn, T * H)
         self.kv.len = total
 
-    def _prefill_qkv(self, l: int, lw: dict, T: int, start_pos: int, fused_heads: bool) -> None:
+    def _prefill_qkv(self, kb, vb, lw: dict, T: int, start_pos: int, fused_heads: bool) -> None:
         """q/k/v of the normalised rows in ``self.pxn`` with the head norms, RoPE
-        and the layer's cache rows (decoder.rs:795-810)."""
+        and the layer's cache rows in ``kb`` / ``vb`` (decoder.rs:795-810)."""
         nq, nk, hd, eps, H = self.nq, self.nk, self.hd, self.eps, self.H
-        kb, vb = self.kv.k_layer_block(l), self.kv.v_layer_block(l)
         if fused_heads:
             K.qkv_heads_int8(self.pq, kb, vb, self.kv.max_seq, lw["wq"], lw["wk"], lw["wv"], self.pxn, T, H,
                              nq, nk, hd, lw["q_norm"], lw["k_norm"], self.rope, start_pos, eps)
@@ -239,6 +239,7 @@ class DecoderInt8:
         H, I, nq, nk, hd, eps = self.H, self.I, self.nq, self.nk, self.hd, self.eps
         h, h2 = self.x, self.x2
         h.copy_(embed)
+        k_blocks, v_blocks = self.kv.layer_blocks()
         for l, lw in enumerate(self.w["layers"]):
             qkv_w = [lw["wq"], lw["wk"], lw["wv"]]
             if l == 0:
@@ -249,8 +250,7 @@ class DecoderInt8:
                                                         lw["input_norm"], H, eps)
                 h, h2 = h2, h
             K.decode_attention(self.attn, self.q, self.k, self.v, lw["q_norm"], lw["k_norm"], self.rope, pos,
-                               nq, nk, hd, eps, self.scale, self.kv.k_layer_block(l), self.kv.v_layer_block(l),
-                               self.kv.max_seq, self.attn_ws)
+                               nq, nk, hd, eps, self.scale, k_blocks[l], v_blocks[l], self.kv.max_seq, self.attn_ws)
             wo = lw["wo"]
             K.linear_nobias_int8(self.proj, self.attn, wo.data, wo.scales, 1, nq * hd, H)
             K.add_rms_norm_gate_up_swiglu_int8(self.ffn, h2, h, self.proj, lw["post_attn_norm"], lw["gate_up"],
@@ -370,10 +370,9 @@ class DecoderInt8Batched:
         if lm_head_w8a8:
             self.lm_packed = K.pack_w8a8_tiles(self.lm)
 
-    def _layer_w8a8(self, l: int, lw: dict) -> None:
+    def _layer_w8a8(self, l: int, lw: dict, kb, vb) -> None:
         H, I, B, nq, nk, hd, eps = self.H, self.I, self.B, self.nq, self.nk, self.hd, self.eps
         pk = self.packed[l]
-        kb, vb = self.k[l], self.v[l]
         K.add_rms_norm_quant(self.x, None if l == 0 else self.down, lw["input_norm"], None, self.xq, self.xs,
                              B, H, eps)
         K.qkv_heads_w8a8_packed(self.q, kb, vb, self.rows, pk["qkv"], self.xq, self.xs, lw["q_norm"],
@@ -394,9 +393,11 @@ class DecoderInt8Batched:
         H, I, B, nq, nk, hd, eps = self.H, self.I, self.B, self.nq, self.nk, self.hd, self.eps
         self.x.copy_(embeds[:B * H])
         K.batched_decode_order(self.order, self.positions, B, self.rows)
+        k_blocks, v_blocks = self.k.unbind(0), self.v.unbind(0)
         for l, lw in enumerate(self.w["layers"]):
+            kb, vb = k_blocks[l], v_blocks[l]
             if self.w8a8:
-                self._layer_w8a8(l, lw)
+                self._layer_w8a8(l, lw, kb, vb)
                 continue
             if l == 0:
                 K.rms_norm(self.x_norm, self.x, lw["input_norm"], B, H, eps)
@@ -404,7 +405,6 @@ class DecoderInt8Batched:
                 K.add_rms_norm(self.x, self.down, lw["input_norm"], self.x_norm, B, H, eps)
             K.linear_nobias_int8_multi([self.q, self.kk, self.vv], [lw["wq"], lw["wk"], lw["wv"]],
                                        self.x_norm, B, H)
-            kb, vb = self.k[l], self.v[l]
             K.head_rms_norm_rope_kv(self.q, self.kk, self.vv, lw["q_norm"], lw["k_norm"], self.rope,
                                     self.positions, 0, B, nq, nk, hd, eps, kb, vb, self.rows)
             K.batched_decode_attention(self.attn, self.q, kb, vb, self.rows, self.positions, B, nq, nk, hd,

@@ -58,33 +58,40 @@ def _need(t: torch.Tensor, dtype: torch.dtype, n: int, name: str) -> None:
 F32, I8, I32, U16 = torch.float32, torch.int8, torch.int32, torch.int16
 
 
+class _Calls:
+    """The entry points as functions of the binding extension: a tensor argument
+    is followed by the element count it must hold (checked as ``_need`` does),
+    and the stream is the current one. Bound on first use, all at once."""
+
+    def __getattr__(self, name: str):
+        if name.startswith("__"):
+            raise AttributeError(name)
+        self.__dict__.update(_lib.bind(_need, (F32, I8, I32, U16)))
+        if name not in self.__dict__:
+            raise AttributeError(name)
+        return self.__dict__[name]
+
+
+_call = _Calls()
+
+
 # ---------------------------------------------------------------------------
 # Basic / normalisation (kernels/mod.rs)
 # ---------------------------------------------------------------------------
 def add_inplace(a: torch.Tensor, b: torch.Tensor, n: int) -> None:
     """``a[i] += b[i]`` for i < n (kernels/mod.rs:486-488)."""
-    _need(a, F32, n, "a")
-    _need(b, F32, n, "b")
-    _lib.call("qasr_add_inplace_f32", _ptr(a), _ptr(b), n, _stream())
+    _call.qasr_add_inplace_f32(a, n, b, n, n)
 
 
 def rms_norm(out, x, weight, seq_len: int, hidden: int, eps: float) -> None:
     """Row RMSNorm (kernels/mod.rs:897-918)."""
-    _need(out, F32, seq_len * hidden, "out")
-    _need(x, F32, seq_len * hidden, "x")
-    _need(weight, F32, hidden, "weight")
-    _lib.call("qasr_rms_norm_f32", _ptr(out), _ptr(x), _ptr(weight), seq_len, hidden, eps, _stream())
+    _call.qasr_rms_norm_f32(out, seq_len * hidden, x, seq_len * hidden, weight, hidden, seq_len, hidden, eps)
 
 
 def add_rms_norm(x, delta, weight, out, seq_len: int, hidden: int, eps: float) -> None:
     """Fused ``add_inplace(x, delta)`` + ``rms_norm(out, x)`` (decoder.rs:908+910)."""
     n = seq_len * hidden
-    _need(x, F32, n, "x")
-    _need(delta, F32, n, "delta")
-    _need(weight, F32, hidden, "weight")
-    _need(out, F32, n, "out")
-    _lib.call("qasr_add_rms_norm_f32", _ptr(x), _ptr(delta), _ptr(weight), _ptr(out), seq_len,
-              hidden, eps, _stream())
+    _call.qasr_add_rms_norm_f32(x, n, delta, n, weight, hidden, out, n, seq_len, hidden, eps)
 
 
 def add_rms_norm_quant(x, delta, weight, out, q, q_scales, seq_len: int, hidden: int,
@@ -93,26 +100,14 @@ def add_rms_norm_quant(x, delta, weight, out, q, q_scales, seq_len: int, hidden:
     per-row int8 quantization of y into ``q``/``q_scales``; ``out`` (may be None)
     receives y."""
     n = seq_len * hidden
-    _need(x, F32, n, "x")
-    if delta is not None:
-        _need(delta, F32, n, "delta")
-    _need(weight, F32, hidden, "weight")
-    if out is not None:
-        _need(out, F32, n, "out")
-    _need(q, I8, n, "q")
-    _need(q_scales, F32, seq_len, "q_scales")
-    _lib.call("qasr_add_rms_norm_quant_f32", _ptr(x), _ptr(delta), _ptr(weight), _ptr(out),
-              _ptr(q), _ptr(q_scales), seq_len, hidden, eps, _stream())
+    _call.qasr_add_rms_norm_quant_f32(x, n, delta, n, weight, hidden, out, n, q, n, q_scales, seq_len, seq_len, hidden,
+                                      eps)
 
 
 def layer_norm(out, x, weight, bias, seq_len: int, hidden: int, eps: float) -> None:
     """Row LayerNorm (kernels/mod.rs:866-895)."""
-    _need(out, F32, seq_len * hidden, "out")
-    _need(x, F32, seq_len * hidden, "x")
-    _need(weight, F32, hidden, "weight")
-    _need(bias, F32, hidden, "bias")
-    _lib.call("qasr_layer_norm_f32", _ptr(out), _ptr(x), _ptr(weight), _ptr(bias), seq_len,
-              hidden, eps, _stream())
+    _call.qasr_layer_norm_f32(out, seq_len * hidden, x, seq_len * hidden, weight, hidden, bias, hidden, seq_len, hidden,
+                              eps)
 
 
 
@@ -122,30 +117,18 @@ def add_layer_norm(x, delta, weight, bias, out, seq_len: int, hidden: int, eps: 
     next (encoder.rs:389-390, 370-371, 401-402); equal to ``add_inplace`` +
     ``layer_norm`` bit for bit."""
     n = seq_len * hidden
-    _need(x, F32, n, "x")
-    _need(delta, F32, n, "delta")
-    _need(weight, F32, hidden, "weight")
-    _need(bias, F32, hidden, "bias")
-    _need(out, F32, n, "out")
-    _lib.call("qasr_add_layer_norm_f32", _ptr(x), _ptr(delta), _ptr(weight), _ptr(bias), _ptr(out),
-              seq_len, hidden, eps, _stream())
+    _call.qasr_add_layer_norm_f32(x, n, delta, n, weight, hidden, bias, hidden, out, n, seq_len, hidden, eps)
 
 
 def rms_norm_per_head(x, weight, seq_len: int, n_heads: int, head_dim: int, eps: float) -> None:
     """In-place per-head RMSNorm (kernels/mod.rs:920-935)."""
-    _need(x, F32, seq_len * n_heads * head_dim, "x")
-    _need(weight, F32, head_dim, "weight")
-    _lib.call("qasr_rms_norm_per_head_f32", _ptr(x), _ptr(weight), seq_len, n_heads, head_dim,
-              eps, _stream())
+    _call.qasr_rms_norm_per_head_f32(x, seq_len * n_heads * head_dim, weight, head_dim, seq_len, n_heads, head_dim, eps)
 
 
 def apply_rope_neox(x, cos_vals, sin_vals, seq: int, n_heads: int, head_dim: int) -> None:
     """In-place NeoX RoPE, row s uses cos/sin row s (kernels/mod.rs:1247-1267)."""
-    _need(x, F32, seq * n_heads * head_dim, "x")
-    _need(cos_vals, F32, seq * head_dim, "cos_vals")
-    _need(sin_vals, F32, seq * head_dim, "sin_vals")
-    _lib.call("qasr_apply_rope_neox_f32", _ptr(x), _ptr(cos_vals), _ptr(sin_vals), seq, n_heads,
-              head_dim, _stream())
+    _call.qasr_apply_rope_neox_f32(x, seq * n_heads * head_dim, cos_vals, seq * head_dim, sin_vals, seq * head_dim, seq,
+                                   n_heads, head_dim)
 
 
 def head_rms_norm_rope(q, k, q_norm_w, k_norm_w, cos_tab, sin_tab, positions, seq: int,
@@ -156,21 +139,13 @@ def head_rms_norm_rope(q, k, q_norm_w, k_norm_w, cos_tab, sin_tab, positions, se
     position s). ``cos_tab``/``sin_tab`` are RopeCache tables; a position outside
     the table poisons that row with NaN.
     """
-    if n_heads:
-        _need(q, F32, seq * n_heads * head_dim, "q")
-        _need(q_norm_w, F32, head_dim, "q_norm_w")
-    if n_kv_heads:
-        _need(k, F32, seq * n_kv_heads * head_dim, "k")
-        _need(k_norm_w, F32, head_dim, "k_norm_w")
-    _need(cos_tab, F32, head_dim, "cos_tab")
-    _need(sin_tab, F32, cos_tab.numel(), "sin_tab")
-    if positions is not None:
-        _need(positions, I32, seq, "positions")
     rows = cos_tab.numel() // head_dim
-    _lib.call("qasr_head_rms_norm_rope_f32", _ptr(q if n_heads else None),
-              _ptr(k if n_kv_heads else None), _ptr(q_norm_w if n_heads else None),
-              _ptr(k_norm_w if n_kv_heads else None), _ptr(cos_tab), _ptr(sin_tab),
-              _ptr(positions), seq, n_heads, n_kv_heads, head_dim, rows, eps, _stream())
+    _call.qasr_head_rms_norm_rope_f32(q if n_heads else None, seq * n_heads * head_dim,
+                                      k if n_kv_heads else None, seq * n_kv_heads * head_dim,
+                                      q_norm_w if n_heads else None, head_dim,
+                                      k_norm_w if n_kv_heads else None, head_dim, cos_tab, head_dim,
+                                      sin_tab, cos_tab.numel(), positions, seq, seq, n_heads, n_kv_heads, head_dim,
+                                      rows, eps)
 
 
 def head_rms_norm_rope_kv(q, k, v, q_norm_w, k_norm_w, rope: "RopeCache", positions, start_pos: int,
@@ -186,37 +161,25 @@ def head_rms_norm_rope_kv(q, k, v, q_norm_w, k_norm_w, rope: "RopeCache", positi
     k and v are read only; q is rotated in place.
     """
     kv_dim = n_kv_heads * head_dim
-    if n_heads:
-        _need(q, F32, seq * n_heads * head_dim, "q")
-        _need(q_norm_w, F32, head_dim, "q_norm_w")
-    if n_kv_heads:
-        _need(k, F32, seq * kv_dim, "k")
-        _need(v, F32, seq * kv_dim, "v")
-        _need(k_norm_w, F32, head_dim, "k_norm_w")
-        streams = seq if positions is not None else 1
-        _need(k_cache, F32, streams * cache_rows * kv_dim, "k_cache")
-        _need(v_cache, F32, streams * cache_rows * kv_dim, "v_cache")
-    if positions is not None:
-        _need(positions, I32, seq, "positions")
     if rope.head_dim != head_dim:
         raise ValueError("RopeCache head_dim does not match")
-    _lib.call("qasr_head_rms_norm_rope_kv_f32", _ptr(q if n_heads else None), _ptr(k), _ptr(v),
-              _ptr(q_norm_w if n_heads else None), _ptr(k_norm_w), _ptr(rope.cos), _ptr(rope.sin),
-              _ptr(positions), start_pos, seq, n_heads, n_kv_heads, head_dim, rope.cap, eps,
-              _ptr(k_cache), _ptr(v_cache), cache_rows, _stream())
+    heads, kv = n_heads != 0, n_kv_heads != 0
+    cache = (seq if positions is not None else 1) * cache_rows * kv_dim
+    _call.qasr_head_rms_norm_rope_kv_f32(q if heads else None, seq * n_heads * head_dim, k if kv else None,
+                                         seq * kv_dim, v if kv else None, seq * kv_dim, q_norm_w if heads else None,
+                                         head_dim, k_norm_w if kv else None, head_dim, rope.cos, 0, rope.sin, 0,
+                                         positions, seq, start_pos, seq, n_heads, n_kv_heads, head_dim, rope.cap,
+                                         eps, k_cache if kv else None, cache, v_cache if kv else None, cache,
+                                         cache_rows)
 
 
 def causal_attention(out, q, k, v, seq_q: int, seq_k: int, n_heads: int, n_kv_heads: int,
                      head_dim: int, scale: float, q_offset: int) -> None:
     """Causal GQA attention over a KV block (kernels/mod.rs:1124-1207)."""
-    _need(out, F32, seq_q * n_heads * head_dim, "out")
-    _need(q, F32, seq_q * n_heads * head_dim, "q")
-    if seq_k:
-        _need(k, F32, seq_k * n_kv_heads * head_dim, "k")
-        _need(v, F32, seq_k * n_kv_heads * head_dim, "v")
-    _lib.call("qasr_causal_attention_f32", _ptr(out), _ptr(q), _ptr(k if seq_k else None),
-              _ptr(v if seq_k else None), seq_q, seq_k, n_heads, n_kv_heads, head_dim, scale,
-              q_offset, _stream())
+    _call.qasr_causal_attention_f32(out, seq_q * n_heads * head_dim, q, seq_q * n_heads * head_dim,
+                                    k if seq_k else None, seq_k * n_kv_heads * head_dim,
+                                    v if seq_k else None, seq_k * n_kv_heads * head_dim, seq_q, seq_k, n_heads,
+                                    n_kv_heads, head_dim, scale, q_offset)
 
 
 def batched_decode_workspace(batch: int, n_heads: int, head_dim: int, cache_rows: int,
@@ -230,9 +193,7 @@ def batched_decode_workspace(batch: int, n_heads: int, head_dim: int, cache_rows
 def batched_decode_order(order, positions, batch: int, cache_rows: int) -> None:
     """order (int32 [2 * batch]) = (stream, position) pairs, the streams with the
     most keys first, for batched_decode_attention's ``order``."""
-    _need(order, I32, 2 * batch, "order")
-    _need(positions, I32, batch, "positions")
-    _lib.call("qasr_batched_decode_order_i32", _ptr(order), _ptr(positions), batch, cache_rows, _stream())
+    _call.qasr_batched_decode_order_i32(order, 2 * batch, positions, batch, batch, cache_rows)
 
 
 def batched_decode_attention(out, q, k_cache, v_cache, cache_rows: int, positions, batch: int, n_heads: int,
@@ -245,25 +206,14 @@ def batched_decode_attention(out, q, k_cache, v_cache, cache_rows: int, position
     one workgroup per (stream, kv head) walks all of its keys. ``out_q`` /
     ``out_scales`` (int8 [batch * n_heads * head_dim], f32 [batch]) also get each
     stream's row quantized per row, as quantize_rows_i8 would on ``out``."""
-    if workspace is not None:
-        _need(workspace, F32, 1, "workspace")
     if (out_q is None) != (out_scales is None):
         raise ValueError("out_q and out_scales go together")
-    if out_q is not None:
-        _need(out_q, I8, batch * n_heads * head_dim, "out_q")
-        _need(out_scales, F32, batch, "out_scales")
-    if order is not None:
-        _need(order, I32, 2 * batch, "order")
     kv = n_kv_heads * head_dim
-    _need(out, F32, batch * n_heads * head_dim, "out")
-    _need(q, F32, batch * n_heads * head_dim, "q")
-    _need(k_cache, F32, batch * cache_rows * kv, "k_cache")
-    _need(v_cache, F32, batch * cache_rows * kv, "v_cache")
-    _need(positions, I32, batch, "positions")
-    _lib.call("qasr_batched_decode_attention_f32", _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), cache_rows,
-              _ptr(positions), batch, n_heads, n_kv_heads, head_dim, scale, _ptr(workspace),
-              0 if workspace is None else workspace.numel(), _ptr(out_q), _ptr(out_scales), _ptr(order),
-              _stream())
+    _call.qasr_batched_decode_attention_f32(out, batch * n_heads * head_dim, q, batch * n_heads * head_dim,
+                                            k_cache, batch * cache_rows * kv, v_cache, batch * cache_rows * kv,
+                                            cache_rows, positions, batch, batch, n_heads, n_kv_heads, head_dim, scale,
+                                            workspace, 1, 0 if workspace is None else workspace.numel(),
+                                            out_q, batch * n_heads * head_dim, out_scales, batch, order, 2 * batch)
 
 
 def attention_workspace(seq_q: int, n_heads: int, head_dim: int, device="cuda") -> torch.Tensor:
@@ -277,15 +227,10 @@ def causal_attention_split(out, q, k, v, seq_q: int, seq_k: int, n_heads: int, n
                            head_dim: int, scale: float, q_offset: int, workspace) -> None:
     """causal_attention with the keys split over workgroups (decode shape);
     partials go to ``workspace`` (see attention_workspace)."""
-    _need(out, F32, seq_q * n_heads * head_dim, "out")
-    _need(q, F32, seq_q * n_heads * head_dim, "q")
-    if seq_k:
-        _need(k, F32, seq_k * n_kv_heads * head_dim, "k")
-        _need(v, F32, seq_k * n_kv_heads * head_dim, "v")
-    _need(workspace, F32, 0, "workspace")
-    _lib.call("qasr_causal_attention_split_f32", _ptr(out), _ptr(q), _ptr(k if seq_k else None),
-              _ptr(v if seq_k else None), seq_q, seq_k, n_heads, n_kv_heads, head_dim, scale,
-              q_offset, _ptr(workspace), workspace.numel(), _stream())
+    _call.qasr_causal_attention_split_f32(out, seq_q * n_heads * head_dim, q, seq_q * n_heads * head_dim,
+                                          k if seq_k else None, seq_k * n_kv_heads * head_dim,
+                                          v if seq_k else None, seq_k * n_kv_heads * head_dim, seq_q, seq_k, n_heads,
+                                          n_kv_heads, head_dim, scale, q_offset, workspace, 0, workspace.numel())
 
 
 def decode_attention(out, q, k, v, q_norm_w, k_norm_w, rope: "RopeCache", pos: int, n_heads: int,
@@ -297,28 +242,17 @@ def decode_attention(out, q, k, v, q_norm_w, k_norm_w, rope: "RopeCache", pos: i
     the keys split over workgroups it is one attention launch; ``q`` is scratch
     (it may come back normalised and rotated)."""
     kv_dim = n_kv_heads * head_dim
-    _need(out, F32, n_heads * head_dim, "out")
-    _need(q, F32, n_heads * head_dim, "q")
-    _need(k, F32, kv_dim, "k")
-    _need(v, F32, kv_dim, "v")
-    _need(q_norm_w, F32, head_dim, "q_norm_w")
-    _need(k_norm_w, F32, head_dim, "k_norm_w")
-    _need(k_cache, F32, cache_rows * kv_dim, "k_cache")
-    _need(v_cache, F32, cache_rows * kv_dim, "v_cache")
-    _need(workspace, F32, 0, "workspace")
     if rope.head_dim != head_dim:
         raise ValueError("RopeCache head_dim does not match")
-    _lib.call("qasr_decode_attention_f32", _ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(q_norm_w),
-              _ptr(k_norm_w), _ptr(rope.cos), _ptr(rope.sin), rope.cap, pos, n_heads, n_kv_heads,
-              head_dim, eps, scale, _ptr(k_cache), _ptr(v_cache), cache_rows, _ptr(workspace),
-              workspace.numel(), _stream())
+    _call.qasr_decode_attention_f32(out, n_heads * head_dim, q, n_heads * head_dim, k, kv_dim, v, kv_dim,
+                                    q_norm_w, head_dim, k_norm_w, head_dim, rope.cos, 0, rope.sin, 0, rope.cap, pos,
+                                    n_heads, n_kv_heads, head_dim, eps, scale, k_cache, cache_rows * kv_dim,
+                                    v_cache, cache_rows * kv_dim, cache_rows, workspace, 0, workspace.numel())
 
 
 def argmax_rows(idx, x, rows: int, cols: int) -> None:
     """Per-row argmax with the lm_head loop's semantics (decoder.rs:941-949)."""
-    _need(idx, I32, rows, "idx")
-    _need(x, F32, rows * cols, "x")
-    _lib.call("qasr_argmax_rows_f32", _ptr(idx), _ptr(x), rows, cols, _stream())
+    _call.qasr_argmax_rows_f32(idx, rows, x, rows * cols, rows, cols)
 
 
 def lm_head_workspace(vocab: int, device="cuda") -> torch.Tensor:
@@ -331,14 +265,9 @@ def lm_head_int8_argmax(idx, logits, x, w: QuantWeight, rows: int, in_dim: int, 
                         workspace: torch.Tensor | None = None) -> None:
     """INT8 lm_head logits + greedy argmax (decoder.rs:935-963). With a
     ``lm_head_workspace`` and one row the argmax is reduced inside the matvec."""
-    _need(idx, I32, rows, "idx")
-    _need(logits, F32, rows * vocab, "logits")
-    _need(x, F32, rows * in_dim, "x")
-    _need(w.data, I8, vocab * in_dim, "w")
-    _need(w.scales, F32, vocab, "scales")
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    _lib.call("qasr_lm_head_int8_argmax_f32", _ptr(idx), _ptr(logits), _ptr(x), _ptr(w.data),
-              _ptr(w.scales), rows, in_dim, vocab, _ptr(workspace), ws_bytes, _stream())
+    _call.qasr_lm_head_int8_argmax_f32(idx, rows, logits, rows * vocab, x, rows * in_dim, w.data, vocab * in_dim,
+                                       w.scales, vocab, rows, in_dim, vocab, workspace, ws_bytes)
 
 
 class KvCache:
@@ -374,6 +303,11 @@ class KvCache:
     def v_layer_block(self, layer: int) -> torch.Tensor:
         off = layer * self.max_seq * self.kv_dim
         return self.v[off:off + self.max_seq * self.kv_dim]
+
+    def layer_blocks(self) -> tuple:
+        """Every layer's k block and v block: one torch call for all layers."""
+        n = max(self.max_seq * self.kv_dim, 1)
+        return self.k.split(n), self.v.split(n)
 
     def k_layer(self, layer: int) -> torch.Tensor:
         return self.k_layer_block(layer)[: self.len * self.kv_dim]
@@ -438,44 +372,34 @@ class RopeCache:
 # ---------------------------------------------------------------------------
 def swiglu_multiply(out, gate_up, seq_len: int, intermediate: int) -> None:
     """SwiGLU on the row-interleaved gate/up buffer (kernels/mod.rs:965-985)."""
-    _need(out, F32, seq_len * intermediate, "out")
-    _need(gate_up, F32, seq_len * 2 * intermediate, "gate_up")
-    _lib.call("qasr_swiglu_multiply_f32", _ptr(out), _ptr(gate_up), seq_len, intermediate,
-              _stream())
+    _call.qasr_swiglu_multiply_f32(out, seq_len * intermediate, gate_up, seq_len * 2 * intermediate, seq_len,
+                                   intermediate)
 
 
 def swiglu_multiply_inplace(gate, up) -> None:
     """``gate = silu(gate) * up`` (kernels/mod.rs:988-994)."""
     n = gate.numel()
-    _need(gate, F32, n, "gate")
-    _need(up, F32, n, "up")
-    _lib.call("qasr_swiglu_split_f32", _ptr(gate), _ptr(gate), _ptr(up), n, _stream())
+    _call.qasr_swiglu_split_f32(gate, n, gate, n, up, n, n)
 
 
 def swiglu_split(out, gate, up, n: int) -> None:
     """``out = silu(gate) * up`` on split buffers (decode SwiGLU, decoder.rs:916-921)."""
-    _need(out, F32, n, "out")
-    _need(gate, F32, n, "gate")
-    _need(up, F32, n, "up")
-    _lib.call("qasr_swiglu_split_f32", _ptr(out), _ptr(gate), _ptr(up), n, _stream())
+    _call.qasr_swiglu_split_f32(out, n, gate, n, up, n, n)
 
 
 def silu(x, n: int) -> None:
     """In-place SiLU (kernels/mod.rs:941-946)."""
-    _need(x, F32, n, "x")
-    _lib.call("qasr_silu_f32", _ptr(x), n, _stream())
+    _call.qasr_silu_f32(x, n, n)
 
 
 def gelu(x, n: int) -> None:
     """In-place tanh-approximation GELU, reference arithmetic (kernels/mod.rs:948-963)."""
-    _need(x, F32, n, "x")
-    _lib.call("qasr_gelu_tanh_f32", _ptr(x), n, _stream())
+    _call.qasr_gelu_tanh_f32(x, n, n)
 
 
 def gelu_erf(x, n: int) -> None:
     """In-place exact GELU 0.5*x*(1+erf(x/sqrt(2)))."""
-    _need(x, F32, n, "x")
-    _lib.call("qasr_gelu_erf_f32", _ptr(x), n, _stream())
+    _call.qasr_gelu_erf_f32(x, n, n)
 
 
 # ---------------------------------------------------------------------------
@@ -489,9 +413,7 @@ def sinusoidal_pe(pe, n_pos: int, d_model: int) -> None:
 
 def pe_add(x, pe, rows: int, d_model: int, n_pos: int) -> None:
     """``x[r] += pe[r % n_pos]`` (encoder.rs:340-343 with the table reused)."""
-    _need(x, F32, rows * d_model, "x")
-    _need(pe, F32, n_pos * d_model, "pe")
-    _lib.call("qasr_pe_add_f32", _ptr(x), _ptr(pe), rows, d_model, n_pos, _stream())
+    _call.qasr_pe_add_f32(x, rows * d_model, pe, n_pos * d_model, rows, d_model, n_pos)
 
 
 def pe_add_layer_norm(x, pe, out, weight, bias, rows: int, d_model: int, n_pos: int,
@@ -499,13 +421,8 @@ def pe_add_layer_norm(x, pe, out, weight, bias, rows: int, d_model: int, n_pos: 
     """``x[r] += pe[r % n_pos]`` then ``out = layer_norm(x)`` in one pass: the
     encoder's PE add (encoder.rs:341-343) and layer 0's LayerNorm of the same
     rows (encoder.rs:370-371); equal to ``pe_add`` + ``layer_norm`` bit for bit."""
-    _need(x, F32, rows * d_model, "x")
-    _need(pe, F32, n_pos * d_model, "pe")
-    _need(out, F32, rows * d_model, "out")
-    _need(weight, F32, d_model, "weight")
-    _need(bias, F32, d_model, "bias")
-    _lib.call("qasr_pe_add_layer_norm_f32", _ptr(x), _ptr(pe), _ptr(out), _ptr(weight), _ptr(bias),
-              rows, d_model, n_pos, eps, _stream())
+    _call.qasr_pe_add_layer_norm_f32(x, rows * d_model, pe, n_pos * d_model, out, rows * d_model, weight, d_model,
+                                     bias, d_model, rows, d_model, n_pos, eps)
 
 
 # ---------------------------------------------------------------------------
@@ -522,32 +439,19 @@ class QuantWeight:
 
 
 def embed_gather_f32(out, table, ids, n: int, dim: int) -> None:
-    _need(out, F32, n * dim, "out")
-    _need(table, F32, dim, "table")
-    _need(ids, I32, n, "ids")
-    _lib.call("qasr_embed_gather_f32", _ptr(out), _ptr(table), _ptr(ids), n, dim,
-              table.numel() // dim, _stream())
+    _call.qasr_embed_gather_f32(out, n * dim, table, dim, ids, n, n, dim, table.numel() // dim)
 
 
 def embed_gather_bf16(out, table, ids, n: int, dim: int) -> None:
     """Batched tok_embed_bf16_to_f32; ``table`` holds bf16 bits as int16 or bfloat16."""
-    _need(out, F32, n * dim, "out")
     if table.dtype == torch.bfloat16:
         table = table.view(U16)
-    _need(table, U16, dim, "table")
-    _need(ids, I32, n, "ids")
-    _lib.call("qasr_embed_gather_bf16", _ptr(out), _ptr(table), _ptr(ids), n, dim,
-              table.numel() // dim, _stream())
+    _call.qasr_embed_gather_bf16(out, n * dim, table, dim, ids, n, n, dim, table.numel() // dim)
 
 
 def embed_gather_i8(out, w: QuantWeight, ids, n: int, dim: int) -> None:
     """Batched tok_embed_int8_to_f32."""
-    _need(out, F32, n * dim, "out")
-    _need(w.data, I8, w.out_dim * dim, "w.data")
-    _need(w.scales, F32, w.out_dim, "w.scales")
-    _need(ids, I32, n, "ids")
-    _lib.call("qasr_embed_gather_i8", _ptr(out), _ptr(w.data), _ptr(w.scales), _ptr(ids), n, dim,
-              w.out_dim, _stream())
+    _call.qasr_embed_gather_i8(out, n * dim, w.data, w.out_dim * dim, w.scales, w.out_dim, ids, n, n, dim, w.out_dim)
 
 
 def _one_id(token_id: int, device) -> torch.Tensor:
@@ -573,10 +477,7 @@ def tok_embed_int8_to_f32(dst, w: QuantWeight, token_id: int, dim: int) -> None:
 # ---------------------------------------------------------------------------
 def quantize_rows_i8(q, scales, x, rows: int, cols: int) -> None:
     """Per-row int8 quantization into caller buffers (quantize.rs:633-662)."""
-    _need(q, I8, rows * cols, "q")
-    _need(scales, F32, rows, "scales")
-    _need(x, F32, rows * cols, "x")
-    _lib.call("qasr_quantize_rows_i8", _ptr(q), _ptr(scales), _ptr(x), rows, cols, _stream())
+    _call.qasr_quantize_rows_i8(q, rows * cols, scales, rows, x, rows * cols, rows, cols)
 
 
 def quantize_f32_to_int8(f32_data, out_dim: int, in_dim: int):
@@ -589,30 +490,14 @@ def quantize_f32_to_int8(f32_data, out_dim: int, in_dim: int):
 
 def linear_nobias_int8(y, x, w_int8, scales, seq_len: int, in_dim: int, out_dim: int) -> None:
     """W8A32 ``y = scale * (W_int8 @ x)`` (kernels/mod.rs:650-661)."""
-    _need(y, F32, seq_len * out_dim, "y")
-    _need(x, F32, seq_len * in_dim, "x")
-    _need(w_int8, I8, out_dim * in_dim, "w_int8")
-    _need(scales, F32, out_dim, "scales")
-    _lib.call("qasr_linear_nobias_int8_f32", _ptr(y), _ptr(x), _ptr(w_int8), _ptr(scales),
-              seq_len, in_dim, out_dim, _stream())
+    _call.qasr_linear_nobias_int8_f32(y, seq_len * out_dim, x, seq_len * in_dim, w_int8, out_dim * in_dim,
+                                      scales, out_dim, seq_len, in_dim, out_dim)
 
 
 def linear_nobias_int8_multi(ys, ws: list, x, seq_len: int, in_dim: int) -> None:
     """Several W8A32 projections of the same x in one launch (q/k/v, decoder.rs:881-886);
     ``ws`` are QuantWeights, ``ys[m]`` gets ``seq_len * ws[m].out_dim`` floats."""
-    if len(ys) != len(ws):
-        raise ValueError("one output per weight")
-    for y, w in zip(ys, ws):
-        _need(y, F32, seq_len * w.out_dim, "y")
-        _need(w.data, I8, w.out_dim * in_dim, "w")
-        _need(w.scales, F32, w.out_dim, "scales")
-    _need(x, F32, seq_len * in_dim, "x")
-    n = len(ws)
-    arr = ctypes.c_void_p * max(n, 1)
-    _lib.call("qasr_linear_nobias_int8_multi_f32", n, arr(*[y.data_ptr() for y in ys]),
-              arr(*[w.data.data_ptr() for w in ws]), arr(*[w.scales.data_ptr() for w in ws]),
-              (ctypes.c_size_t * max(n, 1))(*[w.out_dim for w in ws]), _ptr(x), seq_len, in_dim,
-              _stream())
+    _call.qasr_linear_nobias_int8_multi_f32(ys, ws, x, seq_len * in_dim, seq_len, in_dim)
 
 
 def qkv_heads_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeight, wk: QuantWeight, wv: QuantWeight,
@@ -623,22 +508,14 @@ def qkv_heads_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeight, wk: Qu
     ``linear_nobias_int8_multi`` followed by ``head_rms_norm_rope_kv`` (positions
     None); ``k_cache``/``v_cache`` are the layer's ``[cache_rows, kv_dim]`` blocks.
     head_dim 128, seq_len >= 8 and in_dim % 64 == 0 (else the library raises)."""
-    kv = n_kv_heads * head_dim
-    _need(q, F32, seq_len * n_heads * head_dim, "q")
-    _need(k_cache, F32, cache_rows * kv, "k_cache")
-    _need(v_cache, F32, cache_rows * kv, "v_cache")
-    for w, rows, name in ((wq, n_heads * head_dim, "wq"), (wk, kv, "wk"), (wv, kv, "wv")):
-        _need(w.data, I8, rows * in_dim, name)
-        _need(w.scales, F32, rows, name + ".scales")
-    _need(x, F32, seq_len * in_dim, "x")
-    _need(q_norm_w, F32, head_dim, "q_norm_w")
-    _need(k_norm_w, F32, head_dim, "k_norm_w")
+    qd, kv = n_heads * head_dim, n_kv_heads * head_dim
     if rope.head_dim != head_dim:
         raise ValueError("RopeCache head_dim does not match")
-    _lib.call("qasr_qkv_heads_int8_f32", _ptr(q), _ptr(k_cache), _ptr(v_cache), cache_rows, _ptr(wq.data),
-              _ptr(wq.scales), _ptr(wk.data), _ptr(wk.scales), _ptr(wv.data), _ptr(wv.scales), _ptr(x), seq_len,
-              in_dim, n_heads, n_kv_heads, head_dim, _ptr(q_norm_w), _ptr(k_norm_w), _ptr(rope.cos),
-              _ptr(rope.sin), rope.cap, start_pos, eps, _stream())
+    _call.qasr_qkv_heads_int8_f32(q, seq_len * qd, k_cache, cache_rows * kv, v_cache, cache_rows * kv, cache_rows,
+                                  wq.data, qd * in_dim, wq.scales, qd, wk.data, kv * in_dim, wk.scales, kv,
+                                  wv.data, kv * in_dim, wv.scales, kv, x, seq_len * in_dim, seq_len, in_dim, n_heads,
+                                  n_kv_heads, head_dim, q_norm_w, head_dim, k_norm_w, head_dim, rope.cos, 0,
+                                  rope.sin, 0, rope.cap, start_pos, eps)
 
 
 def norm_slices(hidden: int) -> int:
@@ -654,19 +531,11 @@ def linear_int8_residual(h, ss, x, w: QuantWeight, seq_len: int, in_dim: int, ou
     ``ss[t, s]`` = the sum of squares of the updated ``h[t, 64s:64s+64]``, and
     with ``hg``/``gain`` also ``hg = h * gain`` -- what the next folded RMSNorm
     reads. seq_len >= 8 and in_dim % 64 == 0 (else the library raises)."""
-    _need(h, F32, seq_len * out_dim, "h")
-    _need(ss, F32, seq_len * norm_slices(out_dim), "ss")
-    _need(x, F32, seq_len * in_dim, "x")
-    _need(w.data, I8, out_dim * in_dim, "w")
-    _need(w.scales, F32, out_dim, "scales")
     if (hg is None) != (gain is None):
         raise ValueError("linear_int8_residual: hg and gain go together")
-    if hg is not None:
-        _need(hg, F32, seq_len * out_dim, "hg")
-        _need(gain, F32, out_dim, "gain")
-    _lib.call("qasr_linear_int8_residual_f32", _ptr(h), _ptr(ss), _ptr(hg) if hg is not None else None,
-              _ptr(gain) if gain is not None else None, _ptr(x), _ptr(w.data), _ptr(w.scales), seq_len, in_dim,
-              out_dim, _stream())
+    _call.qasr_linear_int8_residual_f32(h, seq_len * out_dim, ss, seq_len * norm_slices(out_dim), hg, seq_len * out_dim,
+                                        gain, out_dim, x, seq_len * in_dim, w.data, out_dim * in_dim, w.scales, out_dim,
+                                        seq_len, in_dim, out_dim)
 
 
 def rms_norm_gate_up_swiglu_multiply_int8(out, hg, ss, eps: float, x_norm, w: QuantWeight, seq_len: int,
@@ -676,15 +545,10 @@ def rms_norm_gate_up_swiglu_multiply_int8(out, hg, ss, eps: float, x_norm, w: Qu
     ``linear_int8_residual``; each token's outputs are multiplied by its 1 / rms.
     ``x_norm`` ([seq_len, in_dim], may be ``hg``) receives the normalised rows
     only on shapes the folded kernel does not take."""
-    _need(out, F32, seq_len * intermediate, "out")
-    _need(hg, F32, seq_len * in_dim, "hg")
-    _need(ss, F32, seq_len * norm_slices(in_dim), "ss")
-    _need(x_norm, F32, seq_len * in_dim, "x_norm")
-    _need(w.data, I8, 2 * intermediate * in_dim, "w")
-    _need(w.scales, F32, 2 * intermediate, "scales")
-    _lib.call("qasr_rms_norm_gate_up_swiglu_multiply_int8_f32", _ptr(out), _ptr(hg), _ptr(ss),
-              norm_slices(in_dim), eps, _ptr(x_norm), _ptr(w.data), _ptr(w.scales), seq_len, in_dim,
-              intermediate, _stream())
+    _call.qasr_rms_norm_gate_up_swiglu_multiply_int8_f32(out, seq_len * intermediate, hg, seq_len * in_dim,
+                                                         ss, seq_len * norm_slices(in_dim), norm_slices(in_dim), eps,
+                                                         x_norm, seq_len * in_dim, w.data, 2 * intermediate * in_dim,
+                                                         w.scales, 2 * intermediate, seq_len, in_dim, intermediate)
 
 
 def rms_norm_qkv_heads_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeight, wk: QuantWeight,
@@ -694,36 +558,24 @@ def rms_norm_qkv_heads_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeigh
     """``qkv_heads_int8`` on the layer-input RMSNorm folded in: ``hg`` = h *
     input_norm and ``ss`` from ``linear_int8_residual`` (decoder.rs:789-810);
     ``x_norm`` as in ``rms_norm_gate_up_swiglu_multiply_int8``."""
-    kv = n_kv_heads * head_dim
-    _need(q, F32, seq_len * n_heads * head_dim, "q")
-    _need(k_cache, F32, cache_rows * kv, "k_cache")
-    _need(v_cache, F32, cache_rows * kv, "v_cache")
-    for w, rows, name in ((wq, n_heads * head_dim, "wq"), (wk, kv, "wk"), (wv, kv, "wv")):
-        _need(w.data, I8, rows * in_dim, name)
-        _need(w.scales, F32, rows, name + ".scales")
-    _need(hg, F32, seq_len * in_dim, "hg")
-    _need(ss, F32, seq_len * norm_slices(in_dim), "ss")
-    _need(x_norm, F32, seq_len * in_dim, "x_norm")
-    _need(q_norm_w, F32, head_dim, "q_norm_w")
-    _need(k_norm_w, F32, head_dim, "k_norm_w")
+    qd, kv = n_heads * head_dim, n_kv_heads * head_dim
     if rope.head_dim != head_dim:
         raise ValueError("RopeCache head_dim does not match")
-    _lib.call("qasr_rms_norm_qkv_heads_int8_f32", _ptr(q), _ptr(k_cache), _ptr(v_cache), cache_rows,
-              _ptr(wq.data), _ptr(wq.scales), _ptr(wk.data), _ptr(wk.scales), _ptr(wv.data), _ptr(wv.scales),
-              _ptr(hg), _ptr(ss), norm_slices(in_dim), norm_eps, _ptr(x_norm), seq_len, in_dim, n_heads,
-              n_kv_heads, head_dim, _ptr(q_norm_w), _ptr(k_norm_w), _ptr(rope.cos), _ptr(rope.sin), rope.cap,
-              start_pos, eps, _stream())
+    _call.qasr_rms_norm_qkv_heads_int8_f32(q, seq_len * qd, k_cache, cache_rows * kv, v_cache, cache_rows * kv,
+                                           cache_rows, wq.data, qd * in_dim, wq.scales, qd, wk.data, kv * in_dim,
+                                           wk.scales, kv, wv.data, kv * in_dim, wv.scales, kv, hg, seq_len * in_dim,
+                                           ss, seq_len * norm_slices(in_dim), norm_slices(in_dim), norm_eps,
+                                           x_norm, seq_len * in_dim, seq_len, in_dim, n_heads, n_kv_heads, head_dim,
+                                           q_norm_w, head_dim, k_norm_w, head_dim, rope.cos, 0, rope.sin, 0, rope.cap,
+                                           start_pos, eps)
 
 
 def gate_up_swiglu_int8(out, x, w: QuantWeight, seq_len: int, in_dim: int, intermediate: int) -> None:
     """W8A32 gate/up projection on the interleaved weight + the decode loop's
     SwiGLU (decoder.rs:912-921), one launch; gate/up values are not stored."""
-    _need(out, F32, seq_len * intermediate, "out")
-    _need(x, F32, seq_len * in_dim, "x")
-    _need(w.data, I8, 2 * intermediate * in_dim, "w")
-    _need(w.scales, F32, 2 * intermediate, "scales")
-    _lib.call("qasr_gate_up_swiglu_int8_f32", _ptr(out), _ptr(x), _ptr(w.data), _ptr(w.scales),
-              seq_len, in_dim, intermediate, _stream())
+    _call.qasr_gate_up_swiglu_int8_f32(out, seq_len * intermediate, x, seq_len * in_dim,
+                                       w.data, 2 * intermediate * in_dim, w.scales, 2 * intermediate, seq_len, in_dim,
+                                       intermediate)
 
 
 def add_rms_norm_linear_nobias_int8_multi(ys, ws: list, h_out, x, delta, norm_w, in_dim: int,
@@ -733,24 +585,8 @@ def add_rms_norm_linear_nobias_int8_multi(ys, ws: list, h_out, x, delta, norm_w,
     then 881-886). ``h_out`` (None: not written) gets h and must be a different
     buffer from x and delta; ``ys[m]`` equals add_rms_norm + linear_nobias_int8_multi
     bit for bit."""
-    if len(ys) != len(ws):
-        raise ValueError("one output per weight")
-    for y, w in zip(ys, ws):
-        _need(y, F32, w.out_dim, "y")
-        _need(w.data, I8, w.out_dim * in_dim, "w")
-        _need(w.scales, F32, w.out_dim, "scales")
-    _need(x, F32, in_dim, "x")
-    _need(norm_w, F32, in_dim, "norm_w")
-    if delta is not None:
-        _need(delta, F32, in_dim, "delta")
-    if h_out is not None:
-        _need(h_out, F32, in_dim, "h_out")
-    n = len(ws)
-    arr = ctypes.c_void_p * max(n, 1)
-    _lib.call("qasr_add_rms_norm_linear_nobias_int8_multi_f32", n, arr(*[y.data_ptr() for y in ys]),
-              arr(*[w.data.data_ptr() for w in ws]), arr(*[w.scales.data_ptr() for w in ws]),
-              (ctypes.c_size_t * max(n, 1))(*[w.out_dim for w in ws]), _ptr(h_out), _ptr(x),
-              _ptr(delta), _ptr(norm_w), in_dim, eps, _stream())
+    _call.qasr_add_rms_norm_linear_nobias_int8_multi_f32(ys, ws, h_out, in_dim, x, in_dim, delta, in_dim, norm_w, in_dim,
+                                                         in_dim, eps)
 
 
 def add_rms_norm_gate_up_swiglu_int8(out, h_out, x, delta, norm_w, w: QuantWeight, in_dim: int,
@@ -758,40 +594,23 @@ def add_rms_norm_gate_up_swiglu_int8(out, h_out, x, delta, norm_w, w: QuantWeigh
     """One decode token: the post-attention add + RMSNorm, the gate/up projection
     and the decode SwiGLU in one launch (decoder.rs:908-921); equals add_rms_norm
     followed by gate_up_swiglu_int8 bit for bit."""
-    _need(out, F32, intermediate, "out")
-    _need(x, F32, in_dim, "x")
-    _need(norm_w, F32, in_dim, "norm_w")
-    if delta is not None:
-        _need(delta, F32, in_dim, "delta")
-    if h_out is not None:
-        _need(h_out, F32, in_dim, "h_out")
-    _need(w.data, I8, 2 * intermediate * in_dim, "w")
-    _need(w.scales, F32, 2 * intermediate, "scales")
-    _lib.call("qasr_add_rms_norm_gate_up_swiglu_int8_f32", _ptr(out), _ptr(h_out), _ptr(x), _ptr(delta),
-              _ptr(norm_w), _ptr(w.data), _ptr(w.scales), in_dim, intermediate, eps, _stream())
+    _call.qasr_add_rms_norm_gate_up_swiglu_int8_f32(out, intermediate, h_out, in_dim, x, in_dim, delta, in_dim,
+                                                    norm_w, in_dim, w.data, 2 * intermediate * in_dim,
+                                                    w.scales, 2 * intermediate, in_dim, intermediate, eps)
 
 
 def gate_up_swiglu_multiply_int8(out, x, w: QuantWeight, seq_len: int, in_dim: int, intermediate: int) -> None:
     """The prefill's W8A32 gate/up projection on the interleaved weight + swiglu_multiply
     (decoder.rs:831-834; the fast_exp SwiGLU), one launch; gate/up values are not stored."""
-    _need(out, F32, seq_len * intermediate, "out")
-    _need(x, F32, seq_len * in_dim, "x")
-    _need(w.data, I8, 2 * intermediate * in_dim, "w")
-    _need(w.scales, F32, 2 * intermediate, "scales")
-    _lib.call("qasr_gate_up_swiglu_multiply_int8_f32", _ptr(out), _ptr(x), _ptr(w.data), _ptr(w.scales),
-              seq_len, in_dim, intermediate, _stream())
+    _call.qasr_gate_up_swiglu_multiply_int8_f32(out, seq_len * intermediate, x, seq_len * in_dim,
+                                                w.data, 2 * intermediate * in_dim, w.scales, 2 * intermediate, seq_len,
+                                                in_dim, intermediate)
 
 
 def linear_int8(y, x, w_int8, scales, bias, seq_len: int, in_dim: int, out_dim: int) -> None:
     """W8A32 linear with optional bias (kernels/mod.rs:664-673)."""
-    _need(y, F32, seq_len * out_dim, "y")
-    _need(x, F32, seq_len * in_dim, "x")
-    _need(w_int8, I8, out_dim * in_dim, "w_int8")
-    _need(scales, F32, out_dim, "scales")
-    if bias is not None:
-        _need(bias, F32, out_dim, "bias")
-    _lib.call("qasr_linear_int8_f32", _ptr(y), _ptr(x), _ptr(w_int8), _ptr(scales), _ptr(bias),
-              seq_len, in_dim, out_dim, _stream())
+    _call.qasr_linear_int8_f32(y, seq_len * out_dim, x, seq_len * in_dim, w_int8, out_dim * in_dim, scales, out_dim,
+                               bias, out_dim, seq_len, in_dim, out_dim)
 
 
 def interleave_gate_up(gate: QuantWeight, up: QuantWeight) -> QuantWeight:
@@ -813,23 +632,15 @@ def interleave_gate_up(gate: QuantWeight, up: QuantWeight) -> QuantWeight:
 def gate_up_swiglu_w8a8(out, w: QuantWeight, xq, x_scales, batch: int, in_dim: int,
                         intermediate: int) -> None:
     """W8A8 gate/up projection + SwiGLU on the interleaved weight (int32-exact dots)."""
-    _need(out, F32, batch * intermediate, "out")
-    _need(w.data, I8, 2 * intermediate * in_dim, "w.data")
-    _need(w.scales, F32, 2 * intermediate, "w.scales")
-    _need(xq, I8, batch * in_dim, "xq")
-    _need(x_scales, F32, batch, "x_scales")
-    _lib.call("qasr_gate_up_swiglu_w8a8", _ptr(out), _ptr(w.data), _ptr(w.scales), _ptr(xq),
-              _ptr(x_scales), batch, in_dim, intermediate, _stream())
+    _call.qasr_gate_up_swiglu_w8a8(out, batch * intermediate, w.data, 2 * intermediate * in_dim,
+                                   w.scales, 2 * intermediate, xq, batch * in_dim, x_scales, batch, batch, in_dim,
+                                   intermediate)
 
 
 def gate_up_swiglu_w8a8_f32in(out, w: QuantWeight, x, in_dim: int, intermediate: int) -> None:
     """Batch-1 W8A8 gate/up + SwiGLU quantizing the fp32 input vector in-kernel."""
-    _need(out, F32, intermediate, "out")
-    _need(w.data, I8, 2 * intermediate * in_dim, "w.data")
-    _need(w.scales, F32, 2 * intermediate, "w.scales")
-    _need(x, F32, in_dim, "x")
-    _lib.call("qasr_gate_up_swiglu_w8a8_f32in", _ptr(out), _ptr(w.data), _ptr(w.scales), _ptr(x),
-              in_dim, intermediate, _stream())
+    _call.qasr_gate_up_swiglu_w8a8_f32in(out, intermediate, w.data, 2 * intermediate * in_dim,
+                                         w.scales, 2 * intermediate, x, in_dim, in_dim, intermediate)
 
 
 def pack_w8a8_tiles(w: QuantWeight) -> QuantWeight:
@@ -842,13 +653,8 @@ def pack_w8a8_tiles(w: QuantWeight) -> QuantWeight:
 
 def linear_w8a8_packed(y, w_packed: QuantWeight, xq, x_scales, batch: int, in_dim: int, out_dim: int) -> None:
     """Batched W8A8 projection: y[m, n] = ((f32)dot * x_scales[m]) * scales[n]."""
-    _need(y, F32, batch * out_dim, "y")
-    _need(w_packed.data, I8, out_dim * in_dim, "w.data")
-    _need(w_packed.scales, F32, out_dim, "w.scales")
-    _need(xq, I8, batch * in_dim, "xq")
-    _need(x_scales, F32, batch, "x_scales")
-    _lib.call("qasr_linear_w8a8_packed", _ptr(y), _ptr(w_packed.data), _ptr(w_packed.scales), _ptr(xq),
-              _ptr(x_scales), batch, in_dim, out_dim, _stream())
+    _call.qasr_linear_w8a8_packed(y, batch * out_dim, w_packed.data, out_dim * in_dim, w_packed.scales, out_dim,
+                                  xq, batch * in_dim, x_scales, batch, batch, in_dim, out_dim)
 
 
 def qkv_heads_w8a8_packed(q_out, k_cache, v_cache, cache_rows: int, w_packed: QuantWeight, xq, x_scales,
@@ -859,30 +665,16 @@ def qkv_heads_w8a8_packed(q_out, k_cache, v_cache, cache_rows: int, w_packed: Qu
     stream). ``k_cache``/``v_cache``: [batch, cache_rows, n_kv_heads * head_dim]."""
     n = (n_heads + 2 * n_kv_heads) * head_dim
     kv = n_kv_heads * head_dim
-    _need(q_out, F32, batch * n_heads * head_dim, "q_out")
-    _need(k_cache, F32, batch * cache_rows * kv, "k_cache")
-    _need(v_cache, F32, batch * cache_rows * kv, "v_cache")
-    _need(w_packed.data, I8, n * in_dim, "w.data")
-    _need(w_packed.scales, F32, n, "w.scales")
-    _need(xq, I8, batch * in_dim, "xq")
-    _need(x_scales, F32, batch, "x_scales")
-    _need(q_norm_w, F32, head_dim, "q_norm_w")
-    _need(k_norm_w, F32, head_dim, "k_norm_w")
-    _need(positions, I32, batch, "positions")
-    _lib.call("qasr_qkv_heads_w8a8_packed", _ptr(q_out), _ptr(k_cache), _ptr(v_cache), cache_rows,
-              _ptr(w_packed.data), _ptr(w_packed.scales), _ptr(xq), _ptr(x_scales), _ptr(q_norm_w),
-              _ptr(k_norm_w), _ptr(rope.cos), _ptr(rope.sin), rope.cap, _ptr(positions), batch, in_dim,
-              n_heads, n_kv_heads, head_dim, eps, _stream())
+    _call.qasr_qkv_heads_w8a8_packed(q_out, batch * n_heads * head_dim, k_cache, batch * cache_rows * kv,
+                                     v_cache, batch * cache_rows * kv, cache_rows, w_packed.data, n * in_dim,
+                                     w_packed.scales, n, xq, batch * in_dim, x_scales, batch, q_norm_w, head_dim,
+                                     k_norm_w, head_dim, rope.cos, 0, rope.sin, 0, rope.cap, positions, batch, batch,
+                                     in_dim, n_heads, n_kv_heads, head_dim, eps)
 
 
 def gate_up_swiglu_w8a8_packed(out, w_packed: QuantWeight, xq, x_scales, batch: int, in_dim: int,
                                intermediate: int) -> None:
     """gate_up_swiglu_w8a8 on a pack_w8a8_tiles weight (same results)."""
-    _need(out, F32, batch * intermediate, "out")
-    _need(w_packed.data, I8, 2 * intermediate * in_dim, "w.data")
-    _need(w_packed.scales, F32, 2 * intermediate, "w.scales")
-    _need(xq, I8, batch * in_dim, "xq")
-    _need(x_scales, F32, batch, "x_scales")
-    _lib.call("qasr_gate_up_swiglu_w8a8_packed", _ptr(out), _ptr(w_packed.data),
-              _ptr(w_packed.scales), _ptr(xq), _ptr(x_scales), batch, in_dim, intermediate,
-              _stream())
+    _call.qasr_gate_up_swiglu_w8a8_packed(out, batch * intermediate, w_packed.data, 2 * intermediate * in_dim,
+                                          w_packed.scales, 2 * intermediate, xq, batch * in_dim, x_scales, batch, batch,
+                                          in_dim, intermediate)
