@@ -878,8 +878,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
           sv[b][r] = key < k_lim ? sacc[b][r] * scale : -__builtin_inff();
           mx = fmaxf(mx, sv[b][r]);
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = fmaxf(mx, lane_xor<16>(mx));
+      mx = fmaxf(mx, lane_xor<32>(mx));
       const float m_new = fmaxf(m_run, mx);
       const float corr = expf(m_run - m_new);
       float sum = 0.0f;
@@ -890,8 +890,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
           sv[b][r] = sv[b][r] == -__builtin_inff() ? 0.0f : expf(sv[b][r] - m_new);
           sum += sv[b][r];
         }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
+      sum += lane_xor<16>(sum);
+      sum += lane_xor<32>(sum);
       l_run = __builtin_fmaf(l_run, corr, sum);
       m_run = m_new;
       // The tile's P V goes into a zeroed accumulator and is added to the

@@ -24,29 +24,69 @@ constexpr int kWave = 64;
 // Cross-lane reductions
 // ---------------------------------------------------------------------------
 
-// Sum over groups of WIDTH consecutive lanes (WIDTH a power of two <= 64).
-// Every lane of a group ends with the same value.
-template <int WIDTH>
-QASR_DEV float group_sum(float v) {
-#pragma unroll
-  for (int m = WIDTH / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
-  return v;
+// The value of lane (lane ^ M) of a wave with every lane active. On the vector
+// ALU alone (DPP moves; permlane swaps for M = 16 and 32): __shfl_xor goes
+// through the LDS pipe, ~100 cycles a step and six steps one after another in
+// a wave-wide sum, which a one-token kernel or an attention tile waits for
+// (four 1.7B decode layers + lm_head at position 1801: 178.8 -> 170.8 us).
+// M == 4 is two moves, or one rotation where lanes 8 apart already hold the
+// same value (PERIODIC, as in a reduction after its M == 8 step).
+template <int M, bool PERIODIC = false>
+QASR_DEV int lane_xor(int v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8 || M == 16 || M == 32, "one bit of the lane index");
+  if constexpr (M == 32) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (int)(s[0] ^ s[1]) ^ v;  // {lower half twice, upper half twice}: the half that is not ours
+  } else if constexpr (M == 16) {
+    const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (int)(s[0] ^ s[1]) ^ v;
+  } else if constexpr (M == 8) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);  // row_ror:8
+  } else if constexpr (M == 4 && PERIODIC) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, true);  // row_ror:4
+  } else if constexpr (M == 4) {
+    const int up = __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xa, false);  // row_shr:4 into lanes 4-7, 12-15
+    return __builtin_amdgcn_update_dpp(up, v, 0x104, 0xf, 0x5, false);         // row_shl:4 into lanes 0-3, 8-11
+  } else if constexpr (M == 2) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);  // quad_perm [2,3,0,1]
+  } else {
+    return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);  // quad_perm [1,0,3,2]
+  }
+}
+template <int M, bool PERIODIC = false>
+QASR_DEV float lane_xor(float v) {
+  return __int_as_float(lane_xor<M, PERIODIC>(__float_as_int(v)));
 }
 
-template <int WIDTH>
-QASR_DEV float group_max(float v) {
-#pragma unroll
-  for (int m = WIDTH / 2; m >= 1; m >>= 1) {
-    float o = __shfl_xor(v, m, kWave);
-    v = o > v ? o : v;
+// Reductions over groups of WIDTH consecutive lanes (WIDTH a power of two
+// <= 64), from the farthest partner to the nearest, every lane active. Every
+// lane of a group ends with the same value.
+template <int WIDTH, int M = WIDTH / 2>
+QASR_DEV float group_sum(float v) {
+  if constexpr (M >= 1) {
+    v += lane_xor<M, (WIDTH > 8)>(v);
+    v = group_sum<WIDTH, M / 2>(v);
   }
   return v;
 }
 
-template <int WIDTH>
+template <int WIDTH, int M = WIDTH / 2>
+QASR_DEV float group_max(float v) {
+  if constexpr (M >= 1) {
+    // not PERIODIC: a NaN stays in its lane (o > v is false), so lanes 8 apart may differ
+    const float o = lane_xor<M>(v);
+    v = o > v ? o : v;
+    v = group_max<WIDTH, M / 2>(v);
+  }
+  return v;
+}
+
+template <int WIDTH, int M = WIDTH / 2>
 QASR_DEV int group_sum_i32(int v) {
-#pragma unroll
-  for (int m = WIDTH / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
+  if constexpr (M >= 1) {
+    v += lane_xor<M, (WIDTH > 8)>(v);
+    v = group_sum_i32<WIDTH, M / 2>(v);
+  }
   return v;
 }
 

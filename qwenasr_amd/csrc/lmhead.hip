@@ -25,18 +25,21 @@ namespace {
 constexpr int kArgmaxBlock = 1024;
 constexpr int kArgmaxLoads = 8;  // loads in flight per thread
 
+template <int M>
+QASR_DEV void wave_argmax(float& bv, int& bi) {
+  const float ov = lane_xor<M>(bv);
+  const int oi = lane_xor<M>(bi);
+  if (argmax_better(ov, oi, bv, bi)) {
+    bv = ov;
+    bi = oi;
+  }
+  if constexpr (M > 1) wave_argmax<M / 2>(bv, bi);
+}
+
 QASR_DEV void block_argmax(float& bv, int& bi) {
   __shared__ float sv[kArgmaxBlock / kWave];
   __shared__ int si[kArgmaxBlock / kWave];
-#pragma unroll
-  for (int m = kWave / 2; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(bv, m, kWave);
-    const int oi = __shfl_xor(bi, m, kWave);
-    if (argmax_better(ov, oi, bv, bi)) {
-      bv = ov;
-      bi = oi;
-    }
-  }
+  wave_argmax<kWave / 2>(bv, bi);
   const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   if (lane == 0) {
     sv[w] = bv;
