@@ -537,7 +537,7 @@ int qasr_causal_attention_split_f32(float* out, const float* q, const float* k, 
  * start_pos = pos, seq = 1, ...) followed by
  * qasr_causal_attention_split_f32(out, q, k_cache, v_cache, 1, pos + 1, ...,
  * q_offset = pos, workspace, ...). When the keys are split over workgroups
- * (workspace large enough, pos >= 255, head_dim 128 with n_heads/n_kv_heads
+ * (workspace large enough, head_dim 128 with n_heads/n_kv_heads
  * <= 2 or head_dim 64 with <= 4) it is a single attention launch (+ merge):
  * every workgroup normalises and rotates its q heads itself and the one
  * holding key pos writes the cache rows; q is then left as given. Otherwise

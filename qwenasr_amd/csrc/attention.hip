@@ -1022,7 +1022,7 @@ bool dispatch_group(int G, float* out, const float* q, const float* k, const flo
                     hipStream_t st) {
 #define QASR_ATTN_CASE(GG)                                                                       \
   case GG:                                                                                       \
-    if (sp.nsplit > 1)                                                                           \
+    if (sp.nsplit > 0)                                                                           \
       launch_attention_split<HD, GG>(out, q, k, v, seq_q, seq_k, nk, scale, q_offset, sp.nsplit, \
                                      sp.keys_per_split, sp.ws_o, sp.ws_ml, st);                 \
     else                                                                                         \
@@ -1040,7 +1040,14 @@ bool dispatch_group(int G, float* out, const float* q, const float* k, const flo
 
 // Key-split plan: workgroups of whole 64-key tiles, aiming at about 1024
 // workgroups, at most kMaxSplits splits; nothing to gain when there are
-// already many (row, kv head) pairs or few keys. Workspace layout: the
+// already many (row, kv head) pairs, or few keys for several rows. One row
+// always takes it, also with one split of up to 64 keys: its tiles load all
+// their keys at once where the unsplit kernel walks them, and the decode step
+// folds the head norm, RoPE and cache store into it (12 layers of the 1.7B
+// shape + lm_head, position 20: 408 -> 363 us, 200: 465 -> 368). The split
+// count is the number of 64-key tiles rounded up: rounded down, every length
+// but whole multiples of 64 got splits of 128 keys, half the workgroups (0.6B
+// at 404 keys: 4 splits, 7.7 us a layer). Workspace layout: the
 // partial outputs [seq_q][n_heads][nsplit][head_dim], then the (max, sum)
 // pairs [seq_q][n_heads][nsplit][2]. (Merging in the last-finishing
 // workgroup instead of a second kernel needs an agent-scope fence per
@@ -1052,12 +1059,12 @@ SplitPlan plan_split(size_t seq_q, size_t seq_k, size_t nk, size_t q_offset, siz
   SplitPlan p;
   const size_t k_max = seq_k < q_offset + seq_q ? seq_k : q_offset + seq_q;
   const size_t pairs = seq_q * nk;
-  if (!workspace || pairs >= 512 || k_max < 256) return p;
+  if (!workspace || pairs >= 512 || k_max == 0 || (seq_q > 1 && k_max < 256)) return p;
   size_t want = (1024 + pairs - 1) / pairs;
-  const size_t by_len = k_max / 64;
+  const size_t by_len = (k_max + 63) / 64;
   if (want > by_len) want = by_len;
   if (want > (size_t)kMaxSplits) want = kMaxSplits;
-  if (want < 2) return p;
+  if (want < 2 && seq_q > 1) return p;
   const size_t need = seq_q * n_heads * want * (head_dim + 2);
   if (need > workspace_floats) return p;
   p.nsplit = (int)want;
@@ -1142,7 +1149,7 @@ extern "C" int qasr_decode_attention_f32(float* out, float* q, const float* k, c
                        aligned16(q_norm_w) && aligned16(k_norm_w) && aligned16(cos_tab) &&
                        aligned16(sin_tab) && aligned16(k_cache) && aligned16(v_cache) &&
                        (!workspace || aligned16(workspace));
-  if (sp.nsplit > 1 && fused_shape && aligned) {
+  if (sp.nsplit > 0 && fused_shape && aligned) {
     DecodePre pre{k, v, q_norm_w, k_norm_w, cos_tab + pos * head_dim, sin_tab + pos * head_dim,
                   k_cache + pos * kv_dim, v_cache + pos * kv_dim, eps};
     hipStream_t st = as_stream(stream);

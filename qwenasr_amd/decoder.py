@@ -7,8 +7,7 @@ Per layer, in the reference's order:
   causal attention over the layer's cache block (one launch with the keys
   split over workgroups, then the merge), o projection, residual add +
   post-attention RMSNorm + gate/up projection + SwiGLU (one launch), down
-  projection: 6 launches (7 below 256 cached keys, where attention does not
-  split and the head norm runs as its own launch).
+  projection: 6 launches.
 The fused add + RMSNorm + projection launches normalise the row inside every
 workgroup, in the element order of the standalone add_rms_norm kernel, so the
 results equal the unfused sequence (``fuse_norms=False``: add_rms_norm, then
