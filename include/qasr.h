@@ -598,6 +598,13 @@ int qasr_batched_decode_order_i32(int32_t* order, const int32_t* positions, size
 size_t qasr_batched_decode_attention_workspace_floats(size_t batch, size_t n_heads, size_t head_dim,
                                                       size_t cache_rows);
 
+/* Workspace floats with which qasr_batched_decode_attention_f32 cuts a small
+ * batch's keys into shorter chunks than 512 (64 or more, by batch, heads and
+ * cache_rows), so that a few streams give the whole GPU work; never less than
+ * qasr_batched_decode_attention_workspace_floats(). */
+size_t qasr_batched_decode_attention_split_workspace_floats(size_t batch, size_t n_heads, size_t head_dim,
+                                                            size_t cache_rows);
+
 /* Workspace floats qasr_causal_attention_split_f32 can use for these sizes. */
 size_t qasr_causal_attention_workspace_floats(size_t seq_q, size_t n_heads, size_t head_dim);
 

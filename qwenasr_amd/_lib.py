@@ -104,6 +104,7 @@ SIGNATURES: dict[str, list] = {
 SIZE_QUERIES = {
     "qasr_causal_attention_workspace_floats": [ctypes.c_size_t] * 3,
     "qasr_batched_decode_attention_workspace_floats": [ctypes.c_size_t] * 4,
+    "qasr_batched_decode_attention_split_workspace_floats": [ctypes.c_size_t] * 4,
     "qasr_lm_head_argmax_workspace_bytes": [ctypes.c_size_t],
 }
 

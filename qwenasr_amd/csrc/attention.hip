@@ -1182,6 +1182,37 @@ static size_t batched_chunk_keys(size_t cache_rows) {
   return r > 512 ? r : 512;
 }
 
+// Keys per chunk when the caller's workspace has room for shorter chunks: with
+// few streams, 512-key chunks leave most CUs idle and each walk is a chain of
+// eight 64-key tiles (11 streams of the 0.6B shape, 768 rows: 22 us a layer on
+// 176 workgroups). So as many 64-key tiles a chunk as give the chip about 1024
+// workgroups at 2 query heads a workgroup and half-full caches, at most 64
+// chunks a row. From batch * n_heads = 1024 on (64 streams of 16 heads) the
+// streams alone fill it and the second launch only costs: 100 streams of 400
+// rows 523 us a step unchunked, 559 us in chunks of 192.
+// Four 0.6B layers + lm_head, before -> after: 11 streams of 768 rows
+// 387 -> 345 us, 2 of 1200 rows 326 -> 273; 30 of 1500 rows, 1.7B 644 -> 633.
+static size_t batched_split_keys(size_t batch, size_t n_heads, size_t cache_rows) {
+  constexpr size_t kWork = 4096;  // (query head, cache row) pairs per workgroup and key of its chunk
+  const size_t most = batched_chunk_keys(cache_rows);
+  if (most > 512 || batch >= 1024 || n_heads >= 1024 || batch * n_heads >= 1024) return most;
+  const size_t work = batch * n_heads * cache_rows;
+  const size_t by_work = (work + 64 * kWork - 1) / (64 * kWork) * 64;
+  const size_t by_slots = (cache_rows + 64 * kMaxSplits - 1) / (64 * kMaxSplits) * 64;
+  const size_t keys = by_work > by_slots ? by_work : by_slots;
+  return keys < most ? keys : most;
+}
+
+// Floats of the partials of chunks of `keys` keys: 0 for one chunk, or when the
+// size would overflow (such a call is rejected anyway).
+static size_t chunk_floats(size_t batch, size_t n_heads, size_t head_dim, size_t cache_rows, size_t keys) {
+  const size_t nchunk = (cache_rows + keys - 1) / keys;
+  size_t n = 0;
+  if (nchunk <= 1 || !mul_ok(batch, n_heads, &n) || !mul_ok(n, nchunk, &n) || !mul_ok(n, head_dim + 2, &n))
+    return 0;
+  return n;
+}
+
 namespace qasr {
 namespace {
 // order[r] = (stream, position) of the stream of rank r when the streams are
@@ -1239,15 +1270,16 @@ extern "C" int qasr_batched_decode_order_i32(int32_t* order, const int32_t* posi
   return launch_status("batched_decode_order");
 }
 
-// 0 also when the size would overflow (such a call is rejected anyway).
 extern "C" size_t qasr_batched_decode_attention_workspace_floats(size_t batch, size_t n_heads, size_t head_dim,
                                                                  size_t cache_rows) {
   if (cache_rows == 0 || cache_rows >= 0x40000000u) return 0;
-  const size_t nchunk = (cache_rows + batched_chunk_keys(cache_rows) - 1) / batched_chunk_keys(cache_rows);
-  size_t n = 0;
-  if (nchunk <= 1 || !mul_ok(batch, n_heads, &n) || !mul_ok(n, nchunk, &n) || !mul_ok(n, head_dim + 2, &n))
-    return 0;
-  return n;
+  return chunk_floats(batch, n_heads, head_dim, cache_rows, batched_chunk_keys(cache_rows));
+}
+
+extern "C" size_t qasr_batched_decode_attention_split_workspace_floats(size_t batch, size_t n_heads,
+                                                                       size_t head_dim, size_t cache_rows) {
+  if (cache_rows == 0 || cache_rows >= 0x40000000u) return 0;
+  return chunk_floats(batch, n_heads, head_dim, cache_rows, batched_split_keys(batch, n_heads, cache_rows));
 }
 
 extern "C" int qasr_batched_decode_attention_f32(float* out, const float* q, const float* k_cache,
@@ -1280,8 +1312,12 @@ extern "C" int qasr_batched_decode_attention_f32(float* out, const float* q, con
   QASR_REQUIRE(!out_q == !out_scales, "batched_decode_attention: out_q and out_scales go together");
   QASR_REQUIRE(!out_q || n_heads * head_dim * 4 <= 65536,
                "batched_decode_attention: a quantized row must fit 64 KiB of LDS");
-  const bool chunked = workspace && need > 0;
-  const int kpc = chunked ? (int)batched_chunk_keys(cache_rows) : (int)cache_rows;
+  const size_t split = qasr_batched_decode_attention_split_workspace_floats(batch, n_heads, head_dim, cache_rows);
+  const bool fine = workspace && split > need && workspace_floats >= split;
+  const bool chunked = workspace && (fine || need > 0);  // the shorter chunks where they fit the workspace
+  const int kpc = fine      ? (int)batched_split_keys(batch, n_heads, cache_rows)
+                  : chunked ? (int)batched_chunk_keys(cache_rows)
+                            : (int)cache_rows;
   const int nchunk = (int)((cache_rows + kpc - 1) / kpc);
   const size_t rows_heads = batch * n_heads;
   float* ws_o = chunked ? workspace : nullptr;

@@ -343,7 +343,8 @@ class DecoderInt8Batched:
         # cut into chunks (merged in a second launch) to give the GPU work.
         if attn_chunked is None:
             attn_chunked = B * n_kv_heads < 1024
-        self.attn_ws = K.batched_decode_workspace(B, n_heads, head_dim, cache_rows, device) if attn_chunked else None
+        self.attn_ws = K.batched_decode_split_workspace(B, n_heads, head_dim, cache_rows,
+                                                          device) if attn_chunked else None
         self.order = torch.empty(2 * B, dtype=torch.int32, device=device)
         self.w8a8 = w8a8
         if w8a8:

@@ -190,6 +190,14 @@ def batched_decode_workspace(batch: int, n_heads: int, head_dim: int, cache_rows
     return torch.empty(n, dtype=F32, device=device) if n else None
 
 
+def batched_decode_split_workspace(batch: int, n_heads: int, head_dim: int, cache_rows: int,
+                                   device="cuda") -> torch.Tensor | None:
+    """As batched_decode_workspace, large enough for a small batch's shorter
+    chunks (None if the cache is one chunk all the same)."""
+    n = _lib.lib().qasr_batched_decode_attention_split_workspace_floats(batch, n_heads, head_dim, cache_rows)
+    return torch.empty(n, dtype=F32, device=device) if n else None
+
+
 def batched_decode_order(order, positions, batch: int, cache_rows: int) -> None:
     """order (int32 [2 * batch]) = (stream, position) pairs, the streams with the
     most keys first, for batched_decode_attention's ``order``."""

@@ -1,5 +1,6 @@
-"""How the decode attentions cut their keys, against the oracle at the fp32
-tolerance of the other attention tests."""
+"""How the decode attentions cut their keys: one token's 64-key splits at every
+edge of a tile, and a small batch's shorter chunks (a larger workspace), against
+the oracle at the fp32 tolerance of the other attention tests."""
 from __future__ import annotations
 
 import numpy as np
@@ -27,3 +28,54 @@ def test_one_token_split_edges(dev, pos):
                              K.attention_workspace(1, NQ, HD, dev))
     ref = oracle.causal_attention(q, k, v, 1, pos + 1, NQ, NK, HD, HD ** -0.5, pos)
     np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=1e-5)
+
+
+def test_split_workspace_sizes():
+    from qwenasr_amd import _lib
+
+    split = _lib.lib().qasr_batched_decode_attention_split_workspace_floats
+    whole = _lib.lib().qasr_batched_decode_attention_workspace_floats
+    assert split(11, 16, 128, 768) == 11 * 16 * 12 * 130   # chunks of 64 keys
+    assert split(30, 16, 128, 1500) == 30 * 16 * 8 * 130   # of 192
+    assert split(1, 16, 128, 64) == 0                      # one chunk
+    assert split(1, 16, 128, 10000) == 16 * 53 * 130       # of 192: at most 64 chunks
+    for b, h, rows in ((64, 16, 1024), (256, 16, 2048), (1 << 40, 16, 2048), (3, 1 << 62, 100), (1, 16, 40000),
+                       (2, 16, 0), (2, 16, 1 << 31)):
+        assert split(b, h, 128, rows) == whole(b, h, 128, rows)
+    for b in (1, 2, 7, 20, 63, 64, 200):
+        for rows in (1, 65, 300, 513, 2048, 32768, 32769):
+            assert split(b, 16, 128, rows) >= whole(b, 16, 128, rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nq,nk,hd,rows", [(16, 8, 128, 130), (16, 8, 128, 768), (8, 8, 128, 300), (16, 4, 64, 500)])
+def test_short_chunks(dev, nq, nk, hd, rows):
+    from qwenasr_amd import _lib, kernels as K
+
+    kv, pos = nk * hd, [0, 63, 64, rows - 1, rows // 2, rows]
+    B = len(pos)
+    r = np.random.default_rng([82, nq, rows])
+    q = r.standard_normal((B, nq * hd)).astype(np.float32)
+    k, v = (r.standard_normal((B, rows, kv)).astype(np.float32) for _ in range(2))
+    d = lambda a: torch.from_numpy(a).to(dev).reshape(-1)  # noqa: E731
+    p = d(np.array(pos, np.int32))
+    ws = K.batched_decode_split_workspace(B, nq, hd, rows, dev)
+    assert ws.numel() > _lib.lib().qasr_batched_decode_attention_workspace_floats(B, nq, hd, rows)
+    order = torch.empty(2 * B, dtype=torch.int32, device=dev)
+    K.batched_decode_order(order, p, B, rows)
+    out, oq = torch.full((B * nq * hd,), 9.0, device=dev), torch.empty(B * nq * hd, dtype=torch.int8, device=dev)
+    osc = torch.empty(B, device=dev)
+    dq, dk, dv = d(q), d(k), d(v)
+    for quant in (False, True):
+        ws.fill_(7.0)
+        K.batched_decode_attention(out, dq, dk, dv, rows, p, B, nq, nk, hd, hd ** -0.5, ws, oq if quant else None,
+                                   osc if quant else None, order)
+        got = out.view(B, -1).cpu().numpy()
+        assert np.isnan(got[-1]).all()  # a position outside the cache
+        for m in range(B - 1):
+            n = pos[m] + 1
+            ref = oracle.causal_attention(q[m], k[m, :n].ravel(), v[m, :n].ravel(), 1, n, nq, nk, hd, hd ** -0.5, n - 1)
+            np.testing.assert_allclose(got[m], ref, rtol=1e-5, atol=1e-5, err_msg=f"stream {m}")
+    rq, rs = torch.empty_like(oq), torch.empty_like(osc)
+    K.quantize_rows_i8(rq, rs, out, B, nq * hd)
+    assert torch.equal(oq, rq) and torch.equal(osc, rs)
