@@ -552,6 +552,45 @@ int qasr_decode_attention_f32(float* out, float* q, const float* k, const float*
                               float* k_cache, float* v_cache, size_t cache_rows, float* workspace,
                               size_t workspace_floats, void* stream);
 
+/* Digit rows: a row of fp32 activations as fixed-point numbers under the row's
+ * own power of two, x = 2^exps[r] * I with |I| <= 2^30, each I as four signed
+ * base-256 digits: plane d of digits ([4][rows][cols] int8) holds digit d, the
+ * lowest first. The *_digits_* projections take such rows: their int8 weights
+ * meet the digits on the int8 matrix cores with exact integer sums, so they
+ * round less than an fp32 accumulation of the same dot product. A row with an
+ * infinity or NaN gives NaN outputs. cols a multiple of 4, at most 8192.
+ * No reference counterpart (its INT8 linears multiply in fp32). */
+int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
+                        void* stream);
+/* x += delta (nullable), then the digit rows of its RMSNorm (kernels/mod.rs:897-918);
+ * x_norm (nullable) receives the normalised rows too. */
+int qasr_add_rms_norm_digits_f32(float* x, const float* delta, const float* weight, float* x_norm,
+                                 int8_t* digits, int32_t* exps, size_t rows, size_t cols, float eps,
+                                 void* stream);
+/* W8A32 projections (kernels/mod.rs:650-661) of digit rows, 1 to 3 matrices of
+ * the same input in one launch; residual != 0: y += projection. in_dim a
+ * multiple of 256, out_dims multiples of 4, 16-byte aligned buffers. */
+int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
+                                const float* const* scales, const size_t* out_dims, const int8_t* digits,
+                                const int32_t* exps, size_t seq, size_t in_dim, size_t residual,
+                                void* stream);
+/* The interleaved gate/up projection of digit rows with the SwiGLU: the decode
+ * loop's (decoder.rs:916-921, libm exp) or, prefill != 0, swiglu_multiply's
+ * (kernels/mod.rs:965-985). */
+int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_gate_up, const float* scales,
+                                        const int8_t* digits, const int32_t* exps, size_t seq, size_t in_dim,
+                                        size_t inter, size_t prefill, void* stream);
+/* As qasr_qkv_heads_int8_f32, from digit rows: the q/k/v projections of a
+ * prefill chunk, q/k head RMSNorm + RoPE at start_pos + t, K/V rows into the
+ * layer's cache blocks (decoder.rs:795-810). head_dim 128. */
+int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v_cache, size_t cache_rows,
+                                   const int8_t* wq, const float* sq, const int8_t* wk, const float* sk,
+                                   const int8_t* wv, const float* sv, const int8_t* digits,
+                                   const int32_t* exps, size_t seq, size_t in_dim, size_t n_heads,
+                                   size_t n_kv_heads, size_t head_dim, const float* q_norm_w,
+                                   const float* k_norm_w, const float* cos_tab, const float* sin_tab,
+                                   size_t table_rows, size_t start_pos, float eps, void* stream);
+
 /* Decode attention of `batch` streams, each over its own cache block
  * (decoder.rs:900-903 per stream): for stream m at pos = positions[m], out[m]
  * = causal attention of q[m] (n_heads*head_dim, already normalised and

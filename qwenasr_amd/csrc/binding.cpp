@@ -249,6 +249,11 @@ QASR_BIND(qasr_gate_up_swiglu_w8a8_packed, "out", "w.data", "w.scales", "xq", "x
 QASR_BIND(qasr_linear_w8a8_packed, "y", "w.data", "w.scales", "xq", "x_scales")
 QASR_BIND(qasr_qkv_heads_w8a8_packed, "q_out", "k_cache", "v_cache", "w.data", "w.scales", "xq", "x_scales",
           "q_norm_w", "k_norm_w", "cos", "sin", "positions")
+QASR_BIND(qasr_digit_rows_f32, "digits", "exps", "x")
+QASR_BIND(qasr_add_rms_norm_digits_f32, "x", "?delta", "weight", "?x_norm", "digits", "exps")
+QASR_BIND(qasr_gate_up_swiglu_digits_int8_f32, "out", "w.data", "w.scales", "digits", "exps")
+QASR_BIND(qasr_qkv_heads_digits_int8_f32, "q", "k_cache", "v_cache", "wq", "wq.scales", "wk", "wk.scales", "wv",
+          "wv.scales", "digits", "exps", "q_norm_w", "k_norm_w", "cos", "sin")
 QASR_BIND(qasr_causal_attention_f32, "out", "q", "?k", "?v")
 QASR_BIND(qasr_causal_attention_split_f32, "out", "q", "?k", "?v", "workspace")
 QASR_BIND(qasr_decode_attention_f32, "out", "q", "k", "v", "q_norm_w", "k_norm_w", "cos", "sin", "k_cache", "v_cache",
@@ -304,6 +309,7 @@ Mats take_mats(Args& a, PyObject* rows, PyObject* in_dim) {
 
 struct Tag_multi {};
 struct Tag_norm_multi {};
+struct Tag_digits {};
 
 // (ys, ws, x, n_x, seq_len, in_dim)
 PyObject* py_multi(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -360,6 +366,32 @@ PyObject* py_norm_multi(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
+// (ys, ws, digits, n, exps, n, seq_len, in_dim, residual)
+PyObject* py_digits(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    static const char* const names[] = {"digits", "exps"};
+    const char* fn = "qasr_linear_digits_int8_f32";
+    Args a{args, n, names, fn};
+    if (n != 9) {
+      PyErr_Format(PyExc_TypeError, "%s: takes 9 arguments", fn);
+      throw PyError();
+    }
+    const Mats m = take_mats(a, args[6], args[7]);
+    const int8_t* digits = take<const int8_t*, false>(a);
+    const int32_t* exps = take<const int32_t*, false>(a);
+    const size_t seq = size_arg(a.next()), in_dim = size_arg(a.next()), residual = size_arg(a.next());
+    void* st = take<void*, true>(a);
+    int rc;
+    {
+      PyThreadState* ts = PyEval_SaveThread();
+      rc = reinterpret_cast<decltype(&qasr_linear_digits_int8_f32)>(Entry<Tag_digits>::address)(
+          (size_t)m.n, m.y.data(), m.w.data(), m.s.data(), m.out.data(), digits, exps, seq, in_dim, residual, st);
+      PyEval_RestoreThread(ts);
+    }
+    return finish(fn, rc);
+  });
+}
+
 struct Bound {
   const char* name;
   PyCFunction fn;
@@ -405,6 +437,10 @@ Bound g_bound[] = {
     QASR_ENTRY(qasr_gate_up_swiglu_w8a8_packed),
     QASR_ENTRY(qasr_linear_w8a8_packed),
     QASR_ENTRY(qasr_qkv_heads_w8a8_packed),
+    QASR_ENTRY(qasr_digit_rows_f32),
+    QASR_ENTRY(qasr_add_rms_norm_digits_f32),
+    QASR_ENTRY(qasr_gate_up_swiglu_digits_int8_f32),
+    QASR_ENTRY(qasr_qkv_heads_digits_int8_f32),
     QASR_ENTRY(qasr_causal_attention_f32),
     QASR_ENTRY(qasr_causal_attention_split_f32),
     QASR_ENTRY(qasr_decode_attention_f32),
@@ -415,6 +451,7 @@ Bound g_bound[] = {
     {"qasr_linear_nobias_int8_multi_f32", (PyCFunction)(void (*)(void))py_multi, &Entry<Tag_multi>::address},
     {"qasr_add_rms_norm_linear_nobias_int8_multi_f32", (PyCFunction)(void (*)(void))py_norm_multi,
      &Entry<Tag_norm_multi>::address},
+    {"qasr_linear_digits_int8_f32", (PyCFunction)(void (*)(void))py_digits, &Entry<Tag_digits>::address},
 };
 constexpr size_t kBound = sizeof(g_bound) / sizeof(g_bound[0]);
 PyMethodDef g_defs[kBound];

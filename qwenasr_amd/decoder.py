@@ -100,6 +100,8 @@ class DecoderInt8:
         self.pgate = torch.empty(T * I, **f32)
         self.pffn = torch.empty(T * H, **f32)
         self.pss = torch.empty(T * K.norm_slices(H), **f32)  # per-token partial sums of squares
+        self.pdigits = torch.empty(4 * T * max(H, I, q_dim), dtype=torch.int8, device=self.x.device)
+        self.pexps = torch.empty(T, dtype=torch.int32, device=self.x.device)
         self._pcap = T
 
     def _check_pos(self, pos: int | None, what: str) -> int:
@@ -137,6 +139,38 @@ class DecoderInt8:
         fits = T >= 8 and self.H % 64 == 0 and (self.nq * self.hd) % 64 == 0 and self.I % 64 == 0
         return fits and self.fuse_prefill_norms is not False
 
+    def prefill_digits(self, T: int) -> bool:
+        """Whether a prefill of T tokens runs its projections from digit rows (exact
+        integer products on the int8 matrix cores; ``K.linear_digits_int8``), the default
+        wherever it is the faster one: from 5 tokens on, except where a hidden size of
+        1024 meets a q/k/v grid of exactly one workgroup per CU (449 to 512 tokens),
+        for which the folded bf16-split launches are tuned (two 0.6B layers, 512 tokens
+        213 us against 224; 430 tokens 240 against 217, 64 tokens 143 against 123, 2
+        tokens 89 against 99; 1.7B, 1473 tokens 1377 against 1099)."""
+        q_dim = self.nq * self.hd
+        fits = (self.hd == 128 and max(self.H, self.I, q_dim) <= 8192
+                and self.H % 256 == 0 and self.I % 256 == 0 and q_dim % 256 == 0)
+        one_wave = self.H <= 1024 and (self.nq + 2 * self.nk) * ((T + 63) // 64) == 256
+        return (fits and self.fuse_prefill_heads is None and self.fuse_prefill_norms is None and T >= 5
+                and not one_wave)
+
+    def _prefill_digits(self, T: int, start_pos: int) -> None:
+        H, I, nq, nk, hd, eps = self.H, self.I, self.nq, self.nk, self.hd, self.eps
+        x, dg, ex, rows = self.px, self.pdigits, self.pexps, self.kv.max_seq
+        k_blocks, v_blocks = self.kv.layer_blocks()
+        for l, lw in enumerate(self.w["layers"]):
+            kb, vb = k_blocks[l], v_blocks[l]
+            K.add_rms_norm_digits(x, None, lw["input_norm"], None, dg, ex, T, H, eps)
+            K.qkv_heads_digits_int8(self.pq, kb, vb, rows, lw["wq"], lw["wk"], lw["wv"], dg, ex, T, H, nq, nk, hd,
+                                    lw["q_norm"], lw["k_norm"], self.rope, start_pos, eps)
+            K.causal_attention(self.pattn, self.pq, kb, vb, T, start_pos + T, nq, nk, hd, self.scale, start_pos)
+            K.digit_rows(dg, ex, self.pattn, T, nq * hd)
+            K.linear_digits_int8([x], [lw["wo"]], dg, ex, T, nq * hd, residual=True)
+            K.add_rms_norm_digits(x, None, lw["post_attn_norm"], None, dg, ex, T, H, eps)
+            K.gate_up_swiglu_digits_int8(self.pgate, lw["gate_up"], dg, ex, T, H, I, prefill=True)
+            K.digit_rows(dg, ex, self.pgate, T, I)
+            K.linear_digits_int8([x], [lw["down"]], dg, ex, T, I, residual=True)
+
     def prefill(self, embeds: torch.Tensor, T: int, start_pos: int | None = None) -> None:
         """T tokens at positions start_pos.. (decoder.rs:751-847): writes cache rows
         start_pos..start_pos+T-1 of every layer; ``self.px[:T*H]`` receives the
@@ -149,6 +183,10 @@ class DecoderInt8:
         fold = self.prefill_norms_folded(T)
         x = self.px
         x[:T * H].copy_(embeds[:T * H])
+        if self.prefill_digits(T):
+            self._prefill_digits(T, start_pos)
+            self.kv.len = total
+            return
         layers = self.w["layers"]
         k_blocks, v_blocks = self.kv.layer_blocks()
         for l, lw in enumerate(layers):
@@ -360,6 +398,15 @@ class DecoderInt8Batched:
                 self.packed.append({k: K.pack_w8a8_tiles(w) for k, w in
                                     (("qkv", qkv), ("wo", lw["wo"]), ("gate_up", lw["gate_up"]),
                                      ("down", lw["down"]))})
+        # from two streams on the W8A32 projections run from digit rows (exact integer
+        # products on the int8 matrix cores): two 0.6B layers + lm_head, 2 streams 178 ->
+        # 151 us, 64 streams 292 -> 279; 1.7B, 5 streams 603 -> 237, 64 streams 412 -> 370
+        q_dim = n_heads * head_dim
+        self.digits = (not w8a8 and B >= 2 and max(hidden, intermediate, q_dim) <= 8192
+                       and hidden % 256 == 0 and intermediate % 256 == 0 and q_dim % 256 == 0)
+        if self.digits:
+            self.dg = torch.empty(4 * B * max(hidden, intermediate, q_dim), dtype=torch.int8, device=device)
+            self.dg_exps = torch.empty(B, dtype=torch.int32, device=device)
         fits = self.vocab % 128 == 0 and self.vocab == self.lm.out_dim and hidden in (1024, 2048, 3072, 4096, 6144)
         if lm_head_w8a8 is None:
             lm_head_w8a8 = w8a8 and fits
@@ -385,6 +432,22 @@ class DecoderInt8Batched:
         K.quantize_rows_i8(self.fq, self.fs, self.ffn, B, I)
         K.linear_w8a8_packed(self.down, pk["down"], self.fq, self.fs, B, I, H)
 
+    def _layer_digits(self, l: int, lw: dict, kb, vb) -> None:
+        H, I, B, nq, nk, hd, eps = self.H, self.I, self.B, self.nq, self.nk, self.hd, self.eps
+        dg, ex = self.dg, self.dg_exps
+        K.add_rms_norm_digits(self.x, None if l == 0 else self.down, lw["input_norm"], None, dg, ex, B, H, eps)
+        K.linear_digits_int8([self.q, self.kk, self.vv], [lw["wq"], lw["wk"], lw["wv"]], dg, ex, B, H)
+        K.head_rms_norm_rope_kv(self.q, self.kk, self.vv, lw["q_norm"], lw["k_norm"], self.rope, self.positions, 0, B,
+                                nq, nk, hd, eps, kb, vb, self.rows)
+        K.batched_decode_attention(self.attn, self.q, kb, vb, self.rows, self.positions, B, nq, nk, hd, self.scale,
+                                   self.attn_ws, order=self.order)
+        K.digit_rows(dg, ex, self.attn, B, nq * hd)
+        K.linear_digits_int8([self.proj], [lw["wo"]], dg, ex, B, nq * hd)
+        K.add_rms_norm_digits(self.x, self.proj, lw["post_attn_norm"], None, dg, ex, B, H, eps)
+        K.gate_up_swiglu_digits_int8(self.ffn, lw["gate_up"], dg, ex, B, H, I)
+        K.digit_rows(dg, ex, self.ffn, B, I)
+        K.linear_digits_int8([self.down], [lw["down"]], dg, ex, B, I)
+
     def decode(self, embeds: torch.Tensor) -> None:
         """One token for every stream (``embeds``: [batch, hidden]) at its
         position: ``tokens`` receives each stream's greedy next token,
@@ -398,6 +461,9 @@ class DecoderInt8Batched:
             kb, vb = k_blocks[l], v_blocks[l]
             if self.w8a8:
                 self._layer_w8a8(l, lw, kb, vb)
+                continue
+            if self.digits:
+                self._layer_digits(l, lw, kb, vb)
                 continue
             if l == 0:
                 K.rms_norm(self.x_norm, self.x, lw["input_norm"], B, H, eps)
@@ -418,6 +484,11 @@ class DecoderInt8Batched:
         if self.lm_head_w8a8:
             K.add_rms_norm_quant(self.x, self.down, self.w["norm"], self.x_norm, self.xq, self.xs, B, H, eps)
             K.linear_w8a8_packed(self.logits, self.lm_packed, self.xq, self.xs, B, H, self.vocab)
+            K.argmax_rows(self.tokens, self.logits, B, self.vocab)
+            return
+        if self.digits and self.vocab % 4 == 0:
+            K.add_rms_norm_digits(self.x, self.down, self.w["norm"], self.x_norm, self.dg, self.dg_exps, B, H, eps)
+            K.linear_digits_int8([self.logits], [self.lm], self.dg, self.dg_exps, B, H)
             K.argmax_rows(self.tokens, self.logits, B, self.vocab)
             return
         K.add_rms_norm(self.x, self.down, self.w["norm"], self.x_norm, B, H, eps)

@@ -508,6 +508,51 @@ def linear_nobias_int8_multi(ys, ws: list, x, seq_len: int, in_dim: int) -> None
     _call.qasr_linear_nobias_int8_multi_f32(ys, ws, x, seq_len * in_dim, seq_len, in_dim)
 
 
+def digit_rows(digits, exps, x, rows: int, cols: int) -> None:
+    """Rows of x as four int8 digit planes (``digits`` [4 * rows * cols]) and a power of
+    two per row (``exps``, int32), for the ``*_digits`` projections."""
+    _call.qasr_digit_rows_f32(digits, 4 * rows * cols, exps, rows, x, rows * cols, rows, cols)
+
+
+def add_rms_norm_digits(x, delta, weight, x_norm, digits, exps, rows: int, cols: int, eps: float) -> None:
+    """x += delta (None: not), then the digit rows of its RMSNorm; ``x_norm`` (or None)
+    receives the normalised rows too."""
+    n = rows * cols
+    _call.qasr_add_rms_norm_digits_f32(x, n, delta, n, weight, cols, x_norm, n, digits, 4 * n, exps, rows, rows, cols,
+                                       eps)
+
+
+def linear_digits_int8(ys, ws: list, digits, exps, seq_len: int, in_dim: int, residual: bool = False) -> None:
+    """W8A32 projections of the same digit rows in one launch (up to 3 QuantWeights);
+    with ``residual`` each is added to its y."""
+    _call.qasr_linear_digits_int8_f32(ys, ws, digits, 4 * seq_len * in_dim, exps, seq_len, seq_len, in_dim,
+                                      int(residual))
+
+
+def gate_up_swiglu_digits_int8(out, w: QuantWeight, digits, exps, seq_len: int, in_dim: int, intermediate: int,
+                               prefill: bool = False) -> None:
+    """The interleaved gate/up projection of digit rows with the decode loop's SwiGLU, or
+    swiglu_multiply's (``prefill``)."""
+    _call.qasr_gate_up_swiglu_digits_int8_f32(out, seq_len * intermediate, w.data, 2 * intermediate * in_dim, w.scales,
+                                              2 * intermediate, digits, 4 * seq_len * in_dim, exps, seq_len, seq_len,
+                                              in_dim, intermediate, int(prefill))
+
+
+def qkv_heads_digits_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeight, wk: QuantWeight, wv: QuantWeight,
+                          digits, exps, seq_len: int, in_dim: int, n_heads: int, n_kv_heads: int, head_dim: int,
+                          q_norm_w, k_norm_w, rope: "RopeCache", start_pos: int, eps: float) -> None:
+    """``qkv_heads_int8`` from digit rows."""
+    qd, kv = n_heads * head_dim, n_kv_heads * head_dim
+    if rope.head_dim != head_dim:
+        raise ValueError("RopeCache head_dim does not match")
+    _call.qasr_qkv_heads_digits_int8_f32(q, seq_len * qd, k_cache, cache_rows * kv, v_cache, cache_rows * kv,
+                                         cache_rows, wq.data, qd * in_dim, wq.scales, qd, wk.data, kv * in_dim,
+                                         wk.scales, kv, wv.data, kv * in_dim, wv.scales, kv, digits,
+                                         4 * seq_len * in_dim, exps, seq_len, seq_len, in_dim, n_heads, n_kv_heads,
+                                         head_dim, q_norm_w, head_dim, k_norm_w, head_dim, rope.cos, 0, rope.sin, 0,
+                                         rope.cap, start_pos, eps)
+
+
 def qkv_heads_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeight, wk: QuantWeight, wv: QuantWeight,
                    x, seq_len: int, in_dim: int, n_heads: int, n_kv_heads: int, head_dim: int, q_norm_w,
                    k_norm_w, rope: "RopeCache", start_pos: int, eps: float) -> None:

@@ -1,0 +1,186 @@
+"""The digit-row projections (csrc/gemm_digits.hip): the digits themselves, and every
+tile and epilogue at its edges, against 64-bit evaluations.
+
+Bounds: a digit row is x to 2^-31 of its largest element, and the dot products are exact;
+what is left are at most ten fp32 roundings of sums of the digits' size, so an output is
+within 10 * 2^-24 of sum |w| |x| * scale plus that fixed-point step."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _digits(x, dev):
+    from qwenasr_amd import kernels as K
+
+    rows, cols = x.shape
+    dg = torch.empty(4 * rows * cols, dtype=torch.int8, device=dev)
+    ex = torch.empty(rows, dtype=torch.int32, device=dev)
+    K.digit_rows(dg, ex, x.reshape(-1), rows, cols)
+    return dg, ex
+
+
+def _weight(n, k, dev, seed):
+    from qwenasr_amd import kernels as K
+
+    g = torch.Generator(device=dev).manual_seed(seed)
+    w = torch.randint(-128, 128, (n * k,), generator=g, device=dev, dtype=torch.int32).to(torch.int8)
+    return K.QuantWeight(w, torch.rand(n, generator=g, device=dev) + 0.5, n, k)
+
+
+def _product(x, w):
+    q = w.data.view(w.out_dim, w.in_dim).double().cpu()
+    s = w.scales.double().cpu()
+    x = x.double().cpu()
+    return (x @ q.t()) * s, (x.abs() @ q.abs().t()) * s * (10 * 2.0 ** -24) + 1e-30
+
+
+def _near(got, ref, bound):
+    assert ((got.double().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("cols", [4, 1000, 1024, 1028, 3072, 5000, 8192])
+def test_digit_rows_give_the_row_back(dev, cols):
+    r = np.random.default_rng([91, cols])
+    x = r.standard_normal((9, cols)).astype(np.float32)
+    x[1] *= 1e30
+    x[2] *= 1e-42          # subnormal
+    x[3] = 0.0
+    x[4, 0], x[5, -1], x[6, cols // 2] = np.inf, -np.inf, np.nan
+    x[7] = np.round(x[7] * 1000) * np.float32(2.0 ** 20)  # exact multiples of a power of two
+    x[8, 0] = 1e6          # an outlier
+    dg, ex = (t.cpu().numpy() for t in _digits(torch.from_numpy(x).to(dev), dev))
+    value = (dg.reshape(4, 9, cols).astype(np.float64) * 256.0 ** np.arange(4)[:, None, None]).sum(0)
+    for i in (0, 1, 2, 3, 7, 8):
+        got = np.ldexp(value[i], ex[i])
+        step = np.abs(x[i]).max().astype(np.float64) * 2.0 ** -29
+        assert np.abs(got - x[i]).max() <= step / 2
+    np.testing.assert_array_equal(np.ldexp(value[7], ex[7]), x[7])
+    assert (ex[4:7] == -0x40000000).all() and not dg.reshape(4, 9, cols)[:, 4:7].any()
+
+
+@pytest.mark.parametrize("T,K_,N", [(1, 256, 4), (2, 1024, 1024), (31, 512, 36), (32, 1024, 132), (33, 2048, 1000),
+                                    (65, 1024, 4096), (70, 512, 33028), (300, 1024, 12292), (1000, 3072, 1028)])
+def test_linear_digits(dev, T, K_, N):
+    from qwenasr_amd import kernels as K
+
+    x = torch.randn(T, K_, device=dev, generator=torch.Generator(device=dev).manual_seed(T + N))
+    x[:, 3] *= 100.0
+    x[T // 2] *= 1e-20
+    w = _weight(N, K_, dev, N)
+    dg, ex = _digits(x, dev)
+    y = torch.full((T * N,), 9.0, device=dev)
+    K.linear_digits_int8([y], [w], dg, ex, T, K_)
+    ref, bound = _product(x, w)
+    _near(y.view(T, N), ref, bound)
+    z = torch.ones(T * N, device=dev)
+    K.linear_digits_int8([z], [w], dg, ex, T, K_, residual=True)
+    assert torch.equal(z, y + 1.0)
+
+
+def test_three_matrices_and_a_bad_row(dev):
+    from qwenasr_amd import kernels as K
+
+    T, K_, dims = 40, 1024, (2048, 1024, 1028)
+    x = torch.randn(T, K_, device=dev)
+    x[5, 17], x[39, 0] = float("inf"), float("nan")
+    ws = [_weight(n, K_, dev, n) for n in dims]
+    dg, ex = _digits(x, dev)
+    ys = [torch.empty(T * n, device=dev) for n in dims]
+    K.linear_digits_int8(ys, ws, dg, ex, T, K_)
+    good = [i for i in range(T) if i not in (5, 39)]
+    for y, w in zip(ys, ws):
+        got = y.view(T, -1)
+        assert got[[5, 39]].isnan().all()
+        ref, bound = _product(x[good], w)
+        _near(got[good], ref, bound)
+
+
+@pytest.mark.parametrize("T,H,inter", [(3, 1024, 3072), (40, 256, 18), (70, 1024, 8200), (600, 2048, 6144)])
+def test_gate_up_swiglu_digits(dev, T, H, inter):
+    from qwenasr_amd import kernels as K
+
+    w = _weight(2 * inter, H, dev, inter)
+    w.scales.mul_(2e-4)
+    x = torch.randn(T, H, device=dev)
+    dg, ex = _digits(x, dev)
+    gu = torch.empty(T * 2 * inter, device=dev)
+    K.linear_digits_int8([gu], [w], dg, ex, T, H)
+    out, ref = (torch.full((T * inter,), 9.0, device=dev) for _ in range(2))
+    K.gate_up_swiglu_digits_int8(out, w, dg, ex, T, H, inter, prefill=True)
+    K.swiglu_multiply(ref, gu, T, inter)  # the tiles' K groups may differ: a last bit of the gates and ups
+    torch.testing.assert_close(out, ref, rtol=1e-6, atol=1e-6)
+    K.gate_up_swiglu_digits_int8(out, w, dg, ex, T, H, inter)
+    g, u = gu.view(T, inter, 2).double().unbind(-1)
+    torch.testing.assert_close(out.view(T, inter).double(), g / (1 + (-g).exp()) * u, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("T,start,rows", [(5, 0, 5), (33, 7, 64), (40, 24, 64), (200, 100, 300)])
+def test_qkv_heads_digits_equals_the_two_launches(dev, T, start, rows):
+    """The projections followed by head_rms_norm_rope_kv (their tiles may add K in another
+    number of parts); rows that do not fit the cache are refused."""
+    from qwenasr_amd import kernels as K
+
+    H, nq, nk, hd = 1024, 16, 8, 128
+    ws = [_weight(n * hd, H, dev, n + i) for i, n in enumerate((nq, nk, nk))]
+    for w in ws:
+        w.scales.mul_(1e-3)
+    dg, ex = _digits(torch.randn(T, H, device=dev), dev)
+    qw, kw = torch.rand(hd, device=dev) + 0.5, torch.rand(hd, device=dev) + 0.5
+    rope = K.RopeCache(dev)
+    rope.ensure(start + T, hd, 1e6)
+    q1, k1, v1 = (torch.empty(T * n * hd, device=dev) for n in (nq, nk, nk))
+    caches = [torch.full((rows * nk * hd,), 5.0, device=dev) for _ in range(4)]
+    q2 = torch.empty_like(q1)
+    K.qkv_heads_digits_int8(q2, caches[2], caches[3], rows, *ws, dg, ex, T, H, nq, nk, hd, qw, kw, rope, start, 1e-6)
+    with pytest.raises(K.QasrError):
+        K.qkv_heads_digits_int8(q2, caches[2], caches[3], start + T - 1, *ws, dg, ex, T, H, nq, nk, hd, qw, kw, rope,
+                                start, 1e-6)
+    K.linear_digits_int8([q1, k1, v1], ws, dg, ex, T, H)
+    K.head_rms_norm_rope_kv(q1, k1, v1, qw, kw, rope, None, start, T, nq, nk, hd, 1e-6, caches[0], caches[1], rows)
+    for a, b in ((q1, q2), (caches[0], caches[2]), (caches[1], caches[3])):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
+def test_add_rms_norm_digits(dev):
+    from qwenasr_amd import kernels as K
+
+    for rows, cols in ((1, 1024), (7, 2048), (3, 1500), (2, 8192)):
+        x, d = torch.randn(rows * cols, device=dev), torch.randn(rows * cols, device=dev)
+        g = torch.rand(cols, device=dev) + 0.5
+        for delta in (None, d):
+            a, b = x.clone(), x.clone()
+            xn, ref = torch.empty_like(x), torch.empty_like(x)
+            dg = torch.empty(4 * rows * cols, dtype=torch.int8, device=dev)
+            ex = torch.empty(rows, dtype=torch.int32, device=dev)
+            K.add_rms_norm_digits(a, delta, g, xn, dg, ex, rows, cols, 1e-6)
+            if delta is None:
+                K.rms_norm(ref, b, g, rows, cols, 1e-6)
+            else:
+                K.add_rms_norm(b, delta, g, ref, rows, cols, 1e-6)
+            assert torch.equal(a, b)
+            # each sums the squares through at most 42 additions (half of that in the row) and rounds 3 times
+            torch.testing.assert_close(xn, ref, rtol=2 * 24 * 2.0 ** -24, atol=0)
+            dg2, ex2 = _digits(xn.view(rows, cols), dev)
+            assert torch.equal(dg, dg2) and torch.equal(ex, ex2)
+
+
+def test_refusals(dev):
+    from qwenasr_amd import _lib, kernels as K
+
+    x = torch.zeros(4 * 512, device=dev)
+    dg, ex = torch.zeros(4 * 4 * 512, dtype=torch.int8, device=dev), torch.zeros(4, dtype=torch.int32, device=dev)
+    w = _weight(8, 512, dev, 1)
+    y = torch.zeros(64, device=dev)
+    for call in (lambda: K.linear_digits_int8([y], [w], dg, ex, 4, 384),               # in_dim not a multiple of 256
+                 lambda: K.linear_digits_int8([y], [K.QuantWeight(w.data, w.scales, 6, 512)], dg, ex, 4, 512),
+                 lambda: K.digit_rows(dg, ex, x, 4, 510),
+                 lambda: K.digit_rows(dg[1:], ex, x, 1, 512)):
+        with pytest.raises(K.QasrError) as e:
+            call()
+        assert e.value.code == _lib.QASR_ERR_UNSUPPORTED
+    with pytest.raises(IndexError):
+        K.linear_digits_int8([y[:31]], [w], dg, ex, 4, 512)
