@@ -799,10 +799,14 @@ QASR_DEV void ld_v_block(float (&dst)[32], const float* vbase, size_t kv_stride,
   }
 }
 
-template <int G, int NW>
+// SPLIT: workgroup (item, z) walks key tiles [z * tiles_per_split, ...) of its
+// item only and leaves its unnormalised row and (max, sum) in the workspace,
+// slot z of gridDim.y per (row, head), for attention_combine_kernel.
+template <int G, int NW, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_prefill_mfma_kernel(
     float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k,
-    const float* __restrict__ v, int seq_q, int seq_k, int nk, float scale, int q_offset) {
+    const float* __restrict__ v, int seq_q, int seq_k, int nk, float scale, int q_offset,
+    int tiles_per_split = 0, float* __restrict__ ws_o = nullptr, float* __restrict__ ws_ml = nullptr) {
   constexpr int HD = 128;
   constexpr int R = 16 / G;  // query rows per block
   __shared__ float ml[NW][16][2];
@@ -822,7 +826,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
   // keys [0, k_hi) cover every row of the block
   const int k_hi = min(q_offset + min(i0 + R, seq_q), seq_k);
-  const int ntiles = (k_hi + 63) / 64;
+  int ntiles = (k_hi + 63) / 64, first_tile = w;
+  if constexpr (SPLIT) {
+    first_tile += (int)blockIdx.y * tiles_per_split;
+    ntiles = min(ntiles, ((int)blockIdx.y + 1) * tiles_per_split);
+  }
   // this lane's QK column: row i0 + lo % R, head lo / R
   const int k_lim = min(q_offset + i0 + lo % R + 1, seq_k);
   const int last_key = seq_k > 0 ? seq_k - 1 : 0;
@@ -833,15 +841,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
   for (int jt = 0; jt < 8; ++jt) o[jt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-  if (w < ntiles) {
+  if (first_tile < ntiles) {
     float qf[32];
     ld_row32(qf, q + (size_t)min(i0 + lo % R, seq_q - 1) * q_stride + (size_t)(kh * G + lo / R) * HD + 4 * hi);
     const float* kbase = k + (size_t)kh * HD + 4 * hi;
     const float* vbase = v + (size_t)kh * HD + 4 * lo;
     float ka[32], kb1[32];
-    ld_row32(ka, kbase + (size_t)min(w * 64 + lo, last_key) * kv_stride);
-    ld_row32(kb1, kbase + (size_t)min(w * 64 + 16 + lo, last_key) * kv_stride);
-    for (int t = w; t < ntiles; t += NW) {
+    ld_row32(ka, kbase + (size_t)min(first_tile * 64 + lo, last_key) * kv_stride);
+    ld_row32(kb1, kbase + (size_t)min(first_tile * 64 + 16 + lo, last_key) * kv_stride);
+    for (int t = first_tile; t < ntiles; t += NW) {
       const int key0 = t * 64;
       // QK: key blocks 0 and 1 from the prefetched rows, 2 and 3 loaded meanwhile
       float kc[32], kd[32];
@@ -921,7 +929,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int jt = 0; jt < 8; ++jt) ot[jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[3][r], vd[8 * r + jt], ot[jt], 0, 0, 0);
-      if (t == w) {
+      if (t == first_tile) {
 #pragma unroll
         for (int jt = 0; jt < 8; ++jt) o[jt] = ot[jt];
       } else {
@@ -979,7 +987,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
       }
       const float inv = lsum > 0.0f ? 1.0f / lsum : 1.0f;  // no scaling when the sum is 0
       const int row = i0 + col % R, head = kh * G + col / R;
-      if (row < seq_q) {
+      if constexpr (SPLIT) {
+        if (row < seq_q) {
+          const size_t slot = ((size_t)row * nk * G + head) * gridDim.y + blockIdx.y;
+          float* dst = ws_o + slot * HD + 4 * lo;
+          st4(dst, 0, make_float4(acc[0], acc[1], acc[2], acc[3]));
+          st4(dst, 16, make_float4(acc[4], acc[5], acc[6], acc[7]));
+          if (lo == 0) {
+            ws_ml[2 * slot] = mx;
+            ws_ml[2 * slot + 1] = lsum;
+          }
+        }
+      } else if (row < seq_q) {
         float* dst = out + (size_t)row * q_stride + (size_t)head * HD + 4 * lo;
         st4(dst, 0, make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv));
         st4(dst, 16, make_float4(acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv));
@@ -1010,11 +1029,50 @@ void launch_attention(float* out, const float* q, const float* k, const float* v
   }
 }
 
+constexpr int kMaxSplits = 64;
+
 struct SplitPlan {
   int nsplit = 0, keys_per_split = 0;
   float* ws_o = nullptr;
   float* ws_ml = nullptr;
 };
+
+// Key split of a prefill chunk over a long cache: where the (row block, kv head)
+// items leave half of the CUs idle, workgroups of four or more 64-key tiles (one
+// per wave, the chain that a workgroup's time is made of), at most 512. With
+// more items the splits only queue up behind each other. Measured, 16/8 heads,
+// unsplit -> split: 77 rows at 610 24.8 -> 16.4 us, 20 at 1500 43.7 -> 15.4, 128
+// at 400 24.1 -> 22.1; 200 at 500 25.7 -> 34.6. A few rows over few keys are
+// better off with the one-row kernel's splits (plan_split): 8 rows at 610 12.5
+// us against 14.6, 20 at 300 12.9 against 13.6, but 20 at 1500 29.6 against 15.4.
+struct PrefillSplit {
+  int nsplit = 1, tiles_per_split = 0;
+};
+inline PrefillSplit plan_prefill_split(size_t seq_q, size_t seq_k, size_t nk, size_t G, size_t q_offset,
+                                       size_t workspace_floats) {
+  PrefillSplit p;
+  const size_t R = 16 / G, items = (seq_q + R - 1) / R * nk;
+  const size_t k_max = seq_k < q_offset + seq_q ? seq_k : q_offset + seq_q, tiles = (k_max + 63) / 64;
+  if (items > 128 || (seq_q * nk < 512 && seq_q * nk * k_max < 65536)) return p;
+  size_t want = (tiles + 3) / 4;
+  if (want > 512 / items) want = 512 / items;
+  if (want > (size_t)kMaxSplits) want = kMaxSplits;
+  if (want < 2 || seq_q * nk * G * want * 130 > workspace_floats) return p;
+  p.tiles_per_split = (int)((tiles + want - 1) / want);
+  p.nsplit = (int)((tiles + p.tiles_per_split - 1) / p.tiles_per_split);
+  return p;
+}
+
+template <int G>
+void launch_prefill_split(float* out, const float* q, const float* k, const float* v, int seq_q, int seq_k, int nk,
+                          float scale, int q_offset, const PrefillSplit& ps, float* workspace, hipStream_t st) {
+  const long long rows_heads = (long long)seq_q * nk * G;
+  float* ws_ml = workspace + rows_heads * ps.nsplit * 128;
+  const dim3 grid((unsigned)((seq_q + 16 / G - 1) / (16 / G)) * (unsigned)nk, (unsigned)ps.nsplit);
+  attention_prefill_mfma_kernel<G, kPrefillWaves, true><<<grid, 64 * kPrefillWaves, 0, st>>>(
+      out, q, k, v, seq_q, seq_k, nk, scale, q_offset, ps.tiles_per_split, workspace, ws_ml);
+  attention_combine_kernel<128><<<(unsigned)rows_heads, 64, 0, st>>>(out, workspace, ws_ml, rows_heads, ps.nsplit);
+}
 
 template <int HD>
 bool dispatch_group(int G, float* out, const float* q, const float* k, const float* v, int seq_q,
@@ -1052,7 +1110,6 @@ bool dispatch_group(int G, float* out, const float* q, const float* k, const flo
 // pairs [seq_q][n_heads][nsplit][2]. (Merging in the last-finishing
 // workgroup instead of a second kernel needs an agent-scope fence per
 // workgroup -- a whole-L2 writeback and invalidate -- and measured 2x slower.)
-constexpr int kMaxSplits = 64;
 
 SplitPlan plan_split(size_t seq_q, size_t seq_k, size_t nk, size_t q_offset, size_t head_dim,
                      size_t n_heads, float* workspace, size_t workspace_floats) {
@@ -1105,6 +1162,18 @@ static int attention_impl(float* out, const float* q, const float* k, const floa
   QASR_REQUIRE(!workspace || aligned16(workspace), "causal_attention: workspace must be 16-byte aligned");
   hipStream_t st = as_stream(stream);
   const int sq = (int)seq_q, sk = (int)seq_k, nk = (int)n_kv_heads, qo = (int)q_offset;
+  if (head_dim == 128 && seq_q >= 16 / G && workspace && seq_k > 0) {
+    const PrefillSplit ps = plan_prefill_split(seq_q, seq_k, n_kv_heads, G, q_offset, workspace_floats);
+    if (ps.nsplit > 1) {
+      switch (G) {
+        case 1: launch_prefill_split<1>(out, q, k, v, sq, sk, nk, scale, qo, ps, workspace, st); break;
+        case 2: launch_prefill_split<2>(out, q, k, v, sq, sk, nk, scale, qo, ps, workspace, st); break;
+        case 4: launch_prefill_split<4>(out, q, k, v, sq, sk, nk, scale, qo, ps, workspace, st); break;
+        default: launch_prefill_split<8>(out, q, k, v, sq, sk, nk, scale, qo, ps, workspace, st); break;
+      }
+      return launch_status("causal_attention");
+    }
+  }
   const SplitPlan sp = plan_split(seq_q, seq_k, n_kv_heads, q_offset, head_dim, n_heads, workspace,
                                   workspace_floats);
   if (head_dim == 64)

@@ -100,6 +100,8 @@ class DecoderInt8:
         self.pgate = torch.empty(T * I, **f32)
         self.pffn = torch.empty(T * H, **f32)
         self.pss = torch.empty(T * K.norm_slices(H), **f32)  # per-token partial sums of squares
+        # the partials of up to 512 workgroups of 16 (row, head) pairs: what a chunk's key splits use
+        self.pattn_ws = torch.empty(512 * 16 * (self.hd + 2), **f32)
         self.pdigits = torch.empty(4 * T * max(H, I, q_dim), dtype=torch.int8, device=self.x.device)
         self.pexps = torch.empty(T, dtype=torch.int32, device=self.x.device)
         self._pcap = T
@@ -163,7 +165,8 @@ class DecoderInt8:
             K.add_rms_norm_digits(x, None, lw["input_norm"], None, dg, ex, T, H, eps)
             K.qkv_heads_digits_int8(self.pq, kb, vb, rows, lw["wq"], lw["wk"], lw["wv"], dg, ex, T, H, nq, nk, hd,
                                     lw["q_norm"], lw["k_norm"], self.rope, start_pos, eps)
-            K.causal_attention(self.pattn, self.pq, kb, vb, T, start_pos + T, nq, nk, hd, self.scale, start_pos)
+            K.causal_attention_split(self.pattn, self.pq, kb, vb, T, start_pos + T, nq, nk, hd, self.scale, start_pos,
+                                     self.pattn_ws)
             K.digit_rows(dg, ex, self.pattn, T, nq * hd)
             K.linear_digits_int8([x], [lw["wo"]], dg, ex, T, nq * hd, residual=True)
             K.add_rms_norm_digits(x, None, lw["post_attn_norm"], None, dg, ex, T, H, eps)
@@ -201,7 +204,8 @@ class DecoderInt8:
                 else:  # previous layer's residual add (decoder.rs:837-838) + this layer's input norm
                     K.add_rms_norm(x, self.pffn, lw["input_norm"], self.pxn, T, H, eps)
                 self._prefill_qkv(kb, vb, lw, T, start_pos, fused_heads)
-            K.causal_attention(self.pattn, self.pq, kb, vb, T, total, nq, nk, hd, self.scale, start_pos)
+            K.causal_attention_split(self.pattn, self.pq, kb, vb, T, total, nq, nk, hd, self.scale, start_pos,
+                                     self.pattn_ws)
             wo, dn = lw["wo"], lw["down"]
             if fold:
                 K.linear_int8_residual(x, self.pss, self.pattn, wo, T, q_dim, H, self.pxn, lw["post_attn_norm"])

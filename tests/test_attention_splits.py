@@ -30,6 +30,34 @@ def test_one_token_split_edges(dev, pos):
     np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,start,nq,nk", [(77, 610, 16, 8), (128, 385, 16, 8), (16, 1000, 16, 8), (9, 3000, 16, 8),
+                                           (33, 400, 8, 8), (40, 2000, 16, 4), (20, 4200, 16, 2), (77, 179, 16, 8)])
+def test_prefill_key_splits(dev, T, start, nq, nk):
+    """A chunk over a cache in key splits (a last one with fewer tiles, rows whose causal
+    range ends before it) against the unsplit kernel; a workspace too small for them
+    gives the unsplit kernel's result bit for bit."""
+    from qwenasr_amd import kernels as K
+
+    n, kv = T + start, nk * HD
+    r = np.random.default_rng([83, T, start])
+    q = torch.from_numpy(r.standard_normal(T * nq * HD).astype(np.float32)).to(dev)
+    k, v = (torch.from_numpy(r.standard_normal(n * kv).astype(np.float32)).to(dev) for _ in range(2))
+    whole, out = torch.empty_like(q), torch.full_like(q, 9.0)
+    K.causal_attention(whole, q, k, v, T, n, nq, nk, HD, HD ** -0.5, start)
+    ws = torch.full((512 * 16 * (HD + 2),), float("nan"), device=dev)
+    K.causal_attention_split(out, q, k, v, T, n, nq, nk, HD, HD ** -0.5, start, ws)
+    torch.testing.assert_close(out, whole, rtol=1e-5, atol=1e-5)
+    K.causal_attention_split(out, q, k, v, T, n, nq, nk, HD, HD ** -0.5, start, ws[:64])
+    assert torch.equal(out, whole)
+    rows = [0, T // 2, T - 1]
+    for i in rows:
+        ref = oracle.causal_attention(q.view(T, -1)[i].cpu().numpy(), k.cpu().numpy()[:(start + i + 1) * kv],
+                                      v.cpu().numpy()[:(start + i + 1) * kv], 1, start + i + 1, nq, nk, HD, HD ** -0.5,
+                                      start + i)
+        np.testing.assert_allclose(whole.view(T, -1)[i].cpu().numpy(), ref, rtol=1e-5, atol=1e-5)
+
+
 def test_split_workspace_sizes():
     from qwenasr_amd import _lib
 
