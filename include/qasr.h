@@ -552,6 +552,21 @@ int qasr_decode_attention_f32(float* out, float* q, const float* k, const float*
                               float* k_cache, float* v_cache, size_t cache_rows, float* workspace,
                               size_t workspace_floats, void* stream);
 
+/* qasr_decode_attention_f32 followed by the o projection of its row
+ * (qasr_linear_nobias_int8_f32: y[out_dim] from w [out_dim][n_heads *
+ * head_dim], decoder.rs:906-907), bit for bit. Up to 512 cached keys of heads of
+ * 128 (n_heads * 128 = 1024 or 2048) the projection merges the attention's key
+ * splits itself and `out` is not written: treat it as scratch. w 16-byte
+ * aligned. */
+int qasr_decode_attention_linear_int8_f32(float* y, float* out, float* q, const float* k, const float* v,
+                                          const float* q_norm_w, const float* k_norm_w,
+                                          const float* cos_tab, const float* sin_tab, size_t table_rows,
+                                          size_t pos, size_t n_heads, size_t n_kv_heads, size_t head_dim,
+                                          float eps, float scale, float* k_cache, float* v_cache,
+                                          size_t cache_rows, float* workspace, size_t workspace_floats,
+                                          const int8_t* w, const float* scales, size_t out_dim,
+                                          void* stream);
+
 /* Digit rows: a row of fp32 activations as fixed-point numbers under the row's
  * own power of two, x = 2^exps[r] * I with |I| <= 2^30, each I as four signed
  * base-256 digits: plane d of digits ([4][rows][cols] int8) holds digit d, the

@@ -713,7 +713,7 @@ template <int HD, int G>
 void launch_attention_split(float* out, const float* q, const float* k, const float* v, int seq_q,
                             int seq_k, int nk, float scale, int q_offset, int nsplit,
                             int keys_per_split, float* ws_o, float* ws_ml, hipStream_t st,
-                            const DecodePre* pre = nullptr) {
+                            const DecodePre* pre = nullptr, bool merge = true) {
   const dim3 grid((unsigned)seq_q, (unsigned)nk, (unsigned)nsplit);
   if constexpr (G * HD <= 256) {  // the wave's loads fit the register file
     if (pre)
@@ -726,9 +726,9 @@ void launch_attention_split(float* out, const float* q, const float* k, const fl
     causal_attention_kernel<HD, G, 1, 1, true><<<grid, 64, 0, st>>>(
         out, q, k, v, seq_q, seq_k, nk, scale, q_offset, keys_per_split, ws_o, ws_ml);
   }
+  if (!merge) return;
   const long long rows_heads = (long long)seq_q * nk * G;
-  attention_combine_kernel<HD><<<(unsigned)rows_heads, 64, 0, st>>>(out, ws_o, ws_ml,
-                                                                               rows_heads, nsplit);
+  attention_combine_kernel<HD><<<(unsigned)rows_heads, 64, 0, st>>>(out, ws_o, ws_ml, rows_heads, nsplit);
 }
 
 // Prefill attention on the fp32 matrix cores (v_mfma_f32_16x16x4f32), for
@@ -1191,13 +1191,22 @@ extern "C" int qasr_causal_attention_f32(float* out, const float* q, const float
                         nullptr, 0, stream);
 }
 
-extern "C" int qasr_decode_attention_f32(float* out, float* q, const float* k, const float* v,
+// The o projection after the attention (qasr_decode_attention_linear_int8_f32).
+struct DecodeLinear {
+  float* y;
+  const int8_t* w;
+  const float* scales;
+  size_t out_dim;
+};
+
+static int decode_attention(float* out, float* q, const float* k, const float* v,
                                          const float* q_norm_w, const float* k_norm_w,
                                          const float* cos_tab, const float* sin_tab,
                                          size_t table_rows, size_t pos, size_t n_heads,
                                          size_t n_kv_heads, size_t head_dim, float eps, float scale,
                                          float* k_cache, float* v_cache, size_t cache_rows,
-                                         float* workspace, size_t workspace_floats, void* stream) {
+                                         float* workspace, size_t workspace_floats,
+                                         const DecodeLinear* lin, void* stream) {
   if (n_heads == 0) return QASR_OK;
   QASR_REQUIRE(out && q && k && v && q_norm_w && k_norm_w && cos_tab && sin_tab && k_cache && v_cache,
                "decode_attention: null pointer");
@@ -1223,11 +1232,22 @@ extern "C" int qasr_decode_attention_f32(float* out, float* q, const float* k, c
                   k_cache + pos * kv_dim, v_cache + pos * kv_dim, eps};
     hipStream_t st = as_stream(stream);
     const int nk = (int)n_kv_heads, sk = (int)pos + 1, qo = (int)pos;
+    // Few splits are merged by the projection itself. The line: the merge costs
+    // every one of its 256 workgroups 8 KB of reads a split (all 16 heads), the
+    // launch it replaces 2.7 us and as much again on the host.
+    const size_t q_dim = n_heads * head_dim;
+    const bool fold = lin && sp.nsplit <= kMergeSplits && head_dim == 128 && (q_dim == 1024 || q_dim == 2048);
 #define QASR_PRE(HD, GG)                                                                         \
   if (head_dim == HD && G == GG) {                                                               \
     launch_attention_split<HD, GG>(out, q, k_cache, v_cache, 1, sk, nk, scale, qo, sp.nsplit,    \
-                                   sp.keys_per_split, sp.ws_o, sp.ws_ml, st, &pre);             \
-    return launch_status("decode_attention");                                                    \
+                                   sp.keys_per_split, sp.ws_o, sp.ws_ml, st, &pre, !fold);       \
+    if (fold)                                                                                    \
+      launch_w8a32_merge(lin->y, sp.ws_o, sp.ws_ml, sp.nsplit, q_dim, lin->w, lin->scales,       \
+                         lin->out_dim, st);                                                      \
+    const int rc = launch_status("decode_attention");                                            \
+    if (rc != QASR_OK || !lin || fold) return rc;                                                \
+    return qasr_linear_nobias_int8_f32(lin->y, out, lin->w, lin->scales, 1, q_dim, lin->out_dim, \
+                                       stream);                                                  \
   }
     QASR_PRE(128, 1) QASR_PRE(128, 2) QASR_PRE(64, 1) QASR_PRE(64, 2) QASR_PRE(64, 4)
 #undef QASR_PRE
@@ -1237,9 +1257,46 @@ extern "C" int qasr_decode_attention_f32(float* out, float* q, const float* k, c
                                           n_heads, n_kv_heads, head_dim, table_rows, eps, k_cache,
                                           v_cache, cache_rows, stream);
   if (rc != QASR_OK) return rc;
-  return attention_impl(out, q, k_cache, v_cache, 1, pos + 1, n_heads, n_kv_heads, head_dim, scale, pos,
-                        workspace, workspace_floats, stream);
+  rc = attention_impl(out, q, k_cache, v_cache, 1, pos + 1, n_heads, n_kv_heads, head_dim, scale, pos, workspace,
+                      workspace_floats, stream);
+  if (rc != QASR_OK || !lin) return rc;
+  return qasr_linear_nobias_int8_f32(lin->y, out, lin->w, lin->scales, 1, n_heads * head_dim, lin->out_dim, stream);
 }
+
+extern "C" int qasr_decode_attention_f32(float* out, float* q, const float* k, const float* v,
+                                         const float* q_norm_w, const float* k_norm_w,
+                                         const float* cos_tab, const float* sin_tab,
+                                         size_t table_rows, size_t pos, size_t n_heads,
+                                         size_t n_kv_heads, size_t head_dim, float eps, float scale,
+                                         float* k_cache, float* v_cache, size_t cache_rows,
+                                         float* workspace, size_t workspace_floats, void* stream) {
+  return decode_attention(out, q, k, v, q_norm_w, k_norm_w, cos_tab, sin_tab, table_rows, pos, n_heads, n_kv_heads,
+                          head_dim, eps, scale, k_cache, v_cache, cache_rows, workspace, workspace_floats, nullptr,
+                          stream);
+}
+
+extern "C" int qasr_decode_attention_linear_int8_f32(float* y, float* out, float* q, const float* k, const float* v,
+                                                     const float* q_norm_w, const float* k_norm_w,
+                                                     const float* cos_tab, const float* sin_tab, size_t table_rows,
+                                                     size_t pos, size_t n_heads, size_t n_kv_heads, size_t head_dim,
+                                                     float eps, float scale, float* k_cache, float* v_cache,
+                                                     size_t cache_rows, float* workspace, size_t workspace_floats,
+                                                     const int8_t* w, const float* scales, size_t out_dim,
+                                                     void* stream) {
+  if (n_heads == 0 || out_dim == 0) return QASR_OK;
+  QASR_REQUIRE(y && w && scales, "decode_attention_linear: null pointer");
+  size_t n;
+  QASR_REQUIRE(out_dim <= 0x7fffffffu && n_heads <= 65536 && head_dim <= 4096 &&
+                   mul_ok(out_dim, n_heads * head_dim, &n),
+               "decode_attention_linear: size too large");
+  const DecodeLinear lin{y, w, scales, out_dim};
+  if (!aligned16(w))  // the unaligned projection's own kernel
+    return fail(QASR_ERR_UNSUPPORTED, "decode_attention_linear: w must be 16-byte aligned");
+  return decode_attention(out, q, k, v, q_norm_w, k_norm_w, cos_tab, sin_tab, table_rows, pos, n_heads, n_kv_heads,
+                          head_dim, eps, scale, k_cache, v_cache, cache_rows, workspace, workspace_floats, &lin,
+                          stream);
+}
+
 
 // Keys per chunk of the batched decode attention: 512 (a 2 MB stream-head
 // walk becomes at most 4 workgroups, which evens out streams at different

@@ -258,6 +258,8 @@ QASR_BIND(qasr_causal_attention_f32, "out", "q", "?k", "?v")
 QASR_BIND(qasr_causal_attention_split_f32, "out", "q", "?k", "?v", "workspace")
 QASR_BIND(qasr_decode_attention_f32, "out", "q", "k", "v", "q_norm_w", "k_norm_w", "cos", "sin", "k_cache", "v_cache",
           "workspace")
+QASR_BIND(qasr_decode_attention_linear_int8_f32, "y", "out", "q", "k", "v", "q_norm_w", "k_norm_w", "cos", "sin",
+          "k_cache", "v_cache", "workspace", "w", "scales")
 QASR_BIND(qasr_batched_decode_attention_f32, "out", "q", "k_cache", "v_cache", "positions", "?workspace", "?out_q",
           "?out_scales", "?order")
 QASR_BIND(qasr_batched_decode_order_i32, "order", "positions")
@@ -444,6 +446,7 @@ Bound g_bound[] = {
     QASR_ENTRY(qasr_causal_attention_f32),
     QASR_ENTRY(qasr_causal_attention_split_f32),
     QASR_ENTRY(qasr_decode_attention_f32),
+    QASR_ENTRY(qasr_decode_attention_linear_int8_f32),
     QASR_ENTRY(qasr_batched_decode_attention_f32),
     QASR_ENTRY(qasr_batched_decode_order_i32),
     QASR_ENTRY(qasr_argmax_rows_f32),

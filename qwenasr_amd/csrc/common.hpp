@@ -311,6 +311,13 @@ QASR_DEV void argmax_consider(float v, int i, float& bv, int& bi) {
   }
 }
 
+// One-token projection whose input row is a split attention's partials, merged
+// by every workgroup (int8.hip): in_dim / 128 heads of 1 to kMergeSplits splits,
+// in_dim 1024 or 2048. False, launching nothing, for another in_dim.
+constexpr int kMergeSplits = 8;
+bool launch_w8a32_merge(float* y, const float* ws_o, const float* ws_ml, int nsplit, size_t in_dim,
+                        const int8_t* w, const float* scales, size_t out_dim, hipStream_t st);
+
 // Logits of one token through the W8A32 decode kernel, which also writes one
 // (best value, index bits) pair per workgroup to `part` (int8.hip). Returns
 // false, launching nothing, when the shape has no such kernel; *n_part is the

@@ -139,11 +139,24 @@ struct RowNorm {
   float eps;
 };
 
-template <int KCH, int R, int EPI, bool NORM = false>
+// With MERGE the input row is the attention output of one token whose keys were
+// split: heads of 128, at most kMergeSplits partials each ([heads][nsplit][128],
+// (max, sum) pairs [heads][nsplit][2]). Every workgroup merges all heads into
+// its LDS row, wave w the heads w, w + 4, ..., in the arithmetic order of
+// attention_combine_kernel, while its weights arrive: the merge launch and its
+// round trip go, for 66 KB of L2 reads per workgroup at 8 splits.
+struct SplitMerge {
+  const float* ws_o;
+  const float* ws_ml;
+  int nsplit;
+};
+
+template <int KCH, int R, int EPI, bool NORM = false, bool MERGE = false>
 QASR_DEV void w8a32_rows_body(float* y, const float* x, const int8_t* w, const float* scales,
                               const float* bias, int in_dim, int out_dim, unsigned block,
-                              float2* part, const RowNorm& rn = RowNorm{}) {
+                              float2* part, const RowNorm& rn = RowNorm{}, const SplitMerge& sm = SplitMerge{}) {
   constexpr bool PART = EPI == kEpiArgmax;
+  static_assert(!MERGE || (!NORM && !PART && KCH <= 2), "merged heads feed the plain rows");
   static_assert(EPI != kEpiSwiglu || R % 2 == 0, "SwiGLU pairs sit in one wave");
   static_assert(!(NORM && PART), "no normalised input on the argmax path");
   const int lane = threadIdx.x & (kWave - 1);
@@ -152,8 +165,22 @@ QASR_DEV void w8a32_rows_body(float* y, const float* x, const int8_t* w, const f
   // the row statistics' inputs are loaded before the weights: the wait for
   // them then leaves the weight loads in flight
   float4 nx[NORM ? KCH : 1], nd[NORM ? KCH : 1], ng[NORM ? KCH : 1];
-  float4 xg[NORM ? 1 : KCH];
-  if constexpr (!NORM) {
+  [[maybe_unused]] float4 xg[NORM ? 1 : KCH];
+  constexpr int HW = MERGE ? 2 * KCH : 1;  // heads per wave
+  [[maybe_unused]] float2 mo[HW][kMergeSplits];
+  [[maybe_unused]] float mz[HW], lz[HW];
+  if constexpr (MERGE) {
+#pragma unroll
+    for (int j = 0; j < HW; ++j) {
+      const size_t head = threadIdx.x / kWave + 4 * j;
+      const float2* ob = reinterpret_cast<const float2*>(sm.ws_o + head * sm.nsplit * 128) + lane;
+#pragma unroll
+      for (int u = 0; u < kMergeSplits; ++u) mo[j][u] = ob[(size_t)min(u, sm.nsplit - 1) * 64];
+      const float2 t = reinterpret_cast<const float2*>(sm.ws_ml)[head * sm.nsplit + min(lane, sm.nsplit - 1)];
+      mz[j] = lane < sm.nsplit ? t.x : -__builtin_inff();
+      lz[j] = lane < sm.nsplit ? t.y : 0.0f;
+    }
+  } else if constexpr (!NORM) {
 #pragma unroll
     for (int i = 0; i < KCH; ++i) xg[i] = ld4(x, threadIdx.x + 256 * i);
   }
@@ -240,8 +267,29 @@ QASR_DEV void w8a32_rows_body(float* y, const float* x, const int8_t* w, const f
     // weight loads for a quarter of the bytes), once per workgroup. The
     // barrier waits for LDS only, so the weight loads stay in flight.
     __shared__ float4 xs[256 * KCH];
+    if constexpr (MERGE) {
 #pragma unroll
-    for (int i = 0; i < KCH; ++i) xs[threadIdx.x + 256 * i] = xg[i];
+      for (int j = 0; j < HW; ++j) {
+        const float mx = wave_max(mz[j]);
+        const float f = lane < sm.nsplit ? expf(mz[j] - mx) : 0.0f;
+        const float lsum = wave_sum(lz[j] * f);
+        float2 acc = make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int u = 0; u < kMergeSplits; ++u) {
+          if (u < sm.nsplit) {  // uniform
+            const float fz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), u));
+            acc.x = __builtin_fmaf(mo[j][u].x, fz, acc.x);
+            acc.y = __builtin_fmaf(mo[j][u].y, fz, acc.y);
+          }
+        }
+        const float inv = lsum > 0.0f ? 1.0f / lsum : 1.0f;
+        reinterpret_cast<float2*>(xs)[(threadIdx.x / kWave + 4 * j) * 64 + lane] =
+            make_float2(acc.x * inv, acc.y * inv);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < KCH; ++i) xs[threadIdx.x + 256 * i] = xg[i];
+    }
     lds_barrier();
 #pragma unroll
     for (int c = 0; c < KCH; ++c)
@@ -325,6 +373,13 @@ __global__ __launch_bounds__(256) void w8a32_rows_kernel(float* y, const float* 
                                                          int in_dim, int out_dim,
                                                          float2* part = nullptr, RowNorm rn = RowNorm{}) {
   w8a32_rows_body<KCH, R, EPI, NORM>(y, x, w, scales, bias, in_dim, out_dim, blockIdx.x, part, rn);
+}
+
+template <int KCH, int R>
+__global__ __launch_bounds__(256) void w8a32_rows_merge_kernel(float* y, const int8_t* w, const float* scales,
+                                                               int in_dim, int out_dim, SplitMerge sm) {
+  w8a32_rows_body<KCH, R, kEpiRows, false, true>(y, nullptr, w, scales, nullptr, in_dim, out_dim, blockIdx.x,
+                                                 nullptr, RowNorm{}, sm);
 }
 
 // Several matrices of the same input in one launch (the q/k/v projections):
@@ -2042,6 +2097,22 @@ static int launch_w8a32(float* y, const float* x, const int8_t* w, const float* 
 }
 
 namespace qasr {
+bool launch_w8a32_merge(float* y, const float* ws_o, const float* ws_ml, int nsplit, size_t in_dim, const int8_t* w,
+                        const float* scales, size_t out_dim, hipStream_t st) {
+  const int r = rows_per_wave(in_dim, out_dim), k = (int)in_dim, o = (int)out_dim;
+  const unsigned grid = (unsigned)((out_dim + 4 * r - 1) / (4 * r));
+  const SplitMerge sm{ws_o, ws_ml, nsplit};
+#define QASR_MERGE(KCH, R)                                                         \
+  if (in_dim == 1024 * KCH && r == R) {                                            \
+    w8a32_rows_merge_kernel<KCH, R><<<grid, 256, 0, st>>>(y, w, scales, k, o, sm); \
+    return true;                                                                   \
+  }
+  QASR_MERGE(1, 1) QASR_MERGE(1, 2) QASR_MERGE(1, 4) QASR_MERGE(1, 8)
+  QASR_MERGE(2, 1) QASR_MERGE(2, 2) QASR_MERGE(2, 4)
+#undef QASR_MERGE
+  return false;
+}
+
 bool launch_w8a32_argmax_partials(float* y, const float* x, const int8_t* w, const float* scales,
                                   size_t in_dim, size_t out_dim, float2* part, size_t part_cap,
                                   hipStream_t st, unsigned* n_part) {

@@ -290,10 +290,9 @@ class DecoderInt8:
                 K.add_rms_norm_linear_nobias_int8_multi([self.q, self.k, self.v], qkv_w, h2, h, self.down,
                                                         lw["input_norm"], H, eps)
                 h, h2 = h2, h
-            K.decode_attention(self.attn, self.q, self.k, self.v, lw["q_norm"], lw["k_norm"], self.rope, pos,
-                               nq, nk, hd, eps, self.scale, k_blocks[l], v_blocks[l], self.kv.max_seq, self.attn_ws)
-            wo = lw["wo"]
-            K.linear_nobias_int8(self.proj, self.attn, wo.data, wo.scales, 1, nq * hd, H)
+            K.decode_attention_linear_int8(self.proj, self.attn, self.q, self.k, self.v, lw["q_norm"], lw["k_norm"],
+                                           self.rope, pos, nq, nk, hd, eps, self.scale, k_blocks[l], v_blocks[l],
+                                           self.kv.max_seq, self.attn_ws, lw["wo"], H)
             K.add_rms_norm_gate_up_swiglu_int8(self.ffn, h2, h, self.proj, lw["post_attn_norm"], lw["gate_up"],
                                                H, I, eps)
             h, h2 = h2, h

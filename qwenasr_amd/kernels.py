@@ -258,6 +258,22 @@ def decode_attention(out, q, k, v, q_norm_w, k_norm_w, rope: "RopeCache", pos: i
                                     v_cache, cache_rows * kv_dim, cache_rows, workspace, 0, workspace.numel())
 
 
+def decode_attention_linear_int8(y, out, q, k, v, q_norm_w, k_norm_w, rope: "RopeCache", pos: int, n_heads: int,
+                                 n_kv_heads: int, head_dim: int, eps: float, scale: float, k_cache, v_cache,
+                                 cache_rows: int, workspace, w: QuantWeight, out_dim: int) -> None:
+    """``decode_attention`` and the o projection of its row into ``y``, bit for bit; ``out``
+    and ``q`` are scratch."""
+    kv_dim, q_dim = n_kv_heads * head_dim, n_heads * head_dim
+    if rope.head_dim != head_dim:
+        raise ValueError("RopeCache head_dim does not match")
+    _call.qasr_decode_attention_linear_int8_f32(y, out_dim, out, q_dim, q, q_dim, k, kv_dim, v, kv_dim, q_norm_w,
+                                                head_dim, k_norm_w, head_dim, rope.cos, 0, rope.sin, 0, rope.cap, pos,
+                                                n_heads, n_kv_heads, head_dim, eps, scale, k_cache,
+                                                cache_rows * kv_dim, v_cache, cache_rows * kv_dim, cache_rows,
+                                                workspace, 0, workspace.numel(), w.data, out_dim * q_dim, w.scales,
+                                                out_dim, out_dim)
+
+
 def argmax_rows(idx, x, rows: int, cols: int) -> None:
     """Per-row argmax with the lm_head loop's semantics (decoder.rs:941-949)."""
     _call.qasr_argmax_rows_f32(idx, rows, x, rows * cols, rows, cols)

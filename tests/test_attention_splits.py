@@ -107,3 +107,38 @@ def test_short_chunks(dev, nq, nk, hd, rows):
     rq, rs = torch.empty_like(oq), torch.empty_like(osc)
     K.quantize_rows_i8(rq, rs, out, B, nq * hd)
     assert torch.equal(oq, rq) and torch.equal(osc, rs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pos,nq,nk,hd,out_dim", [(0, 16, 8, 128, 1024), (63, 16, 8, 128, 2048), (64, 16, 8, 128, 1000),
+                                                  (403, 16, 8, 128, 1024), (511, 16, 8, 128, 8192),
+                                                  (512, 16, 8, 128, 1024), (300, 8, 8, 128, 4100), (300, 4, 4, 64, 100)])
+def test_decode_attention_linear_equals_the_two_calls(dev, pos, nq, nk, hd, out_dim):
+    """Bit for bit decode_attention and the o projection: 1 to 8 splits merged by the
+    projection, 9 (a merge launch), another head size (the two calls); rows past a
+    multiple of a workgroup's."""
+    from qwenasr_amd import kernels as K
+
+    r = np.random.default_rng([84, pos, nq])
+    d = lambda *s: torch.from_numpy(r.standard_normal(s).astype(np.float32).ravel()).to(dev)  # noqa: E731
+    kv, qd, rows = nk * hd, nq * hd, pos + 3
+    q, k, v, kc, vc = d(qd), d(kv), d(kv), d(rows * kv), d(rows * kv)
+    qw, kw = d(hd), d(hd)
+    w = K.QuantWeight(torch.from_numpy(r.integers(-127, 128, out_dim * qd).astype(np.int8)).to(dev), d(out_dim), out_dim,
+                      qd)
+    rope = K.RopeCache(dev)
+    rope.ensure(pos + 1, hd, 1e6)
+    got = []
+    for fused in (True, False):
+        out, y = torch.full((qd,), 9.0, device=dev), torch.full((out_dim,), 9.0, device=dev)
+        ws = K.attention_workspace(1, nq, hd, dev).fill_(float("nan"))
+        caches = kc.clone(), vc.clone()
+        args = (q.clone(), k, v, qw, kw, rope, pos, nq, nk, hd, 1e-6, hd ** -0.5, *caches, rows, ws)
+        if fused:
+            K.decode_attention_linear_int8(y, out, *args, w, out_dim)
+        else:
+            K.decode_attention(out, *args)
+            K.linear_nobias_int8(y, out, w.data, w.scales, 1, qd, out_dim)
+        got.append((y, *caches))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
