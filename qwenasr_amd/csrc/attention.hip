@@ -802,11 +802,11 @@ QASR_DEV void ld_v_block(float (&dst)[32], const float* vbase, size_t kv_stride,
 // SPLIT: workgroup (item, z) walks key tiles [z * tiles_per_split, ...) of its
 // item only and leaves its unnormalised row and (max, sum) in the workspace,
 // slot z of gridDim.y per (row, head), for attention_combine_kernel.
-template <int G, int NW, bool SPLIT = false>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_prefill_mfma_kernel(
+template <int G, int NW, bool SPLIT>
+QASR_DEV void attention_prefill_body(
     float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, int seq_q, int seq_k, int nk, float scale, int q_offset,
-    int tiles_per_split = 0, float* __restrict__ ws_o = nullptr, float* __restrict__ ws_ml = nullptr) {
+    int tiles_per_split, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
   constexpr int HD = 128;
   constexpr int R = 16 / G;  // query rows per block
   __shared__ float ml[NW][16][2];
@@ -1007,6 +1007,21 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
   }
 }
 
+template <int G, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_prefill_mfma_kernel(
+    float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k,
+    const float* __restrict__ v, int seq_q, int seq_k, int nk, float scale, int q_offset) {
+  attention_prefill_body<G, NW, false>(out, q, k, v, seq_q, seq_k, nk, scale, q_offset, 0, nullptr, nullptr);
+}
+
+template <int G, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_prefill_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, int seq_q, int seq_k, int nk,
+    float scale, int q_offset, int tiles_per_split, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
+  attention_prefill_body<G, NW, true>(nullptr, q, k, v, seq_q, seq_k, nk, scale, q_offset, tiles_per_split, ws_o,
+                                      ws_ml);
+}
+
 template <int HD, int G>
 void launch_attention(float* out, const float* q, const float* k, const float* v, int seq_q,
                       int seq_k, int nk, float scale, int q_offset, hipStream_t st) {
@@ -1069,8 +1084,8 @@ void launch_prefill_split(float* out, const float* q, const float* k, const floa
   const long long rows_heads = (long long)seq_q * nk * G;
   float* ws_ml = workspace + rows_heads * ps.nsplit * 128;
   const dim3 grid((unsigned)((seq_q + 16 / G - 1) / (16 / G)) * (unsigned)nk, (unsigned)ps.nsplit);
-  attention_prefill_mfma_kernel<G, kPrefillWaves, true><<<grid, 64 * kPrefillWaves, 0, st>>>(
-      out, q, k, v, seq_q, seq_k, nk, scale, q_offset, ps.tiles_per_split, workspace, ws_ml);
+  attention_prefill_split_kernel<G, kPrefillWaves><<<grid, 64 * kPrefillWaves, 0, st>>>(
+      q, k, v, seq_q, seq_k, nk, scale, q_offset, ps.tiles_per_split, workspace, ws_ml);
   attention_combine_kernel<128><<<(unsigned)rows_heads, 64, 0, st>>>(out, workspace, ws_ml, rows_heads, ps.nsplit);
 }
 
