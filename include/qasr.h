@@ -577,18 +577,24 @@ int qasr_decode_attention_linear_int8_f32(float* y, float* out, float* q, const 
  * No reference counterpart (its INT8 linears multiply in fp32). */
 int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
                         void* stream);
-/* x += delta (nullable), then the digit rows of its RMSNorm (kernels/mod.rs:897-918);
+/* x += delta (nullable; the sum of delta_parts slices [rows][cols], 1 to 4, as
+ * qasr_linear_digits_int8_f32 writes them), then the digit rows of its RMSNorm (kernels/mod.rs:897-918);
  * x_norm (nullable) receives the normalised rows too. */
-int qasr_add_rms_norm_digits_f32(float* x, const float* delta, const float* weight, float* x_norm,
-                                 int8_t* digits, int32_t* exps, size_t rows, size_t cols, float eps,
-                                 void* stream);
+int qasr_add_rms_norm_digits_f32(float* x, const float* delta, size_t delta_parts, const float* weight,
+                                 float* x_norm, int8_t* digits, int32_t* exps, size_t rows, size_t cols,
+                                 float eps, void* stream);
 /* W8A32 projections (kernels/mod.rs:650-661) of digit rows, 1 to 3 matrices of
- * the same input in one launch; residual != 0: y += projection. in_dim a
- * multiple of 256, out_dims multiples of 4, 16-byte aligned buffers. */
+ * the same input in one launch; residual != 0: y += projection. With parts > 1
+ * (at most 4, no residual, in_dim a multiple of 256 * parts) in_dim is cut into
+ * that many parts and y holds their slices, [parts][seq][out_dim], to be added:
+ * more workgroups for a small product; qasr_linear_digits_parts gives the
+ * number worth taking. in_dim a multiple of 256, out_dims multiples of 4,
+ * 16-byte aligned buffers. */
 int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
                                 const float* const* scales, const size_t* out_dims, const int8_t* digits,
                                 const int32_t* exps, size_t seq, size_t in_dim, size_t residual,
-                                void* stream);
+                                size_t parts, void* stream);
+size_t qasr_linear_digits_parts(size_t seq, size_t in_dim, size_t out_dim);
 /* The interleaved gate/up projection of digit rows with the SwiGLU: the decode
  * loop's (decoder.rs:916-921, libm exp) or, prefill != 0, swiglu_multiply's
  * (kernels/mod.rs:965-985). */

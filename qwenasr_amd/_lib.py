@@ -88,8 +88,8 @@ SIGNATURES: dict[str, list] = {
     "qasr_pack_w8a8_tiles": [P, P, Z, Z, P],
     "qasr_gate_up_swiglu_w8a8_packed": [P, P, P, P, P, Z, Z, Z, P],
     "qasr_digit_rows_f32": [P, P, P, Z, Z, P],
-    "qasr_add_rms_norm_digits_f32": [P, P, P, P, P, P, Z, Z, F, P],
-    "qasr_linear_digits_int8_f32": [Z, P, P, P, P, P, P, Z, Z, Z, P],
+    "qasr_add_rms_norm_digits_f32": [P, P, Z, P, P, P, P, Z, Z, F, P],
+    "qasr_linear_digits_int8_f32": [Z, P, P, P, P, P, P, Z, Z, Z, Z, P],
     "qasr_gate_up_swiglu_digits_int8_f32": [P, P, P, P, P, Z, Z, Z, Z, P],
     "qasr_qkv_heads_digits_int8_f32": [P, P, P, Z, P, P, P, P, P, P, P, P, Z, Z, Z, Z, Z, P, P, P, P, Z, Z, F, P],
     "qasr_linear_w8a8_packed": [P, P, P, P, P, Z, Z, Z, P],
@@ -111,6 +111,7 @@ SIZE_QUERIES = {
     "qasr_causal_attention_workspace_floats": [ctypes.c_size_t] * 3,
     "qasr_batched_decode_attention_workspace_floats": [ctypes.c_size_t] * 4,
     "qasr_batched_decode_attention_split_workspace_floats": [ctypes.c_size_t] * 4,
+    "qasr_linear_digits_parts": [ctypes.c_size_t] * 3,
     "qasr_lm_head_argmax_workspace_bytes": [ctypes.c_size_t],
 }
 

@@ -368,26 +368,28 @@ PyObject* py_norm_multi(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
-// (ys, ws, digits, n, exps, n, seq_len, in_dim, residual)
+// (ys, ws, digits, n, exps, n, seq_len, in_dim, residual, parts, rows); ys hold rows = parts * seq_len rows
 PyObject* py_digits(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     static const char* const names[] = {"digits", "exps"};
     const char* fn = "qasr_linear_digits_int8_f32";
     Args a{args, n, names, fn};
-    if (n != 9) {
-      PyErr_Format(PyExc_TypeError, "%s: takes 9 arguments", fn);
+    if (n != 11) {
+      PyErr_Format(PyExc_TypeError, "%s: takes 11 arguments", fn);
       throw PyError();
     }
-    const Mats m = take_mats(a, args[6], args[7]);
+    const Mats m = take_mats(a, args[10], args[7]);
     const int8_t* digits = take<const int8_t*, false>(a);
     const int32_t* exps = take<const int32_t*, false>(a);
     const size_t seq = size_arg(a.next()), in_dim = size_arg(a.next()), residual = size_arg(a.next());
+    const size_t parts = size_arg(a.next());
     void* st = take<void*, true>(a);
     int rc;
     {
       PyThreadState* ts = PyEval_SaveThread();
       rc = reinterpret_cast<decltype(&qasr_linear_digits_int8_f32)>(Entry<Tag_digits>::address)(
-          (size_t)m.n, m.y.data(), m.w.data(), m.s.data(), m.out.data(), digits, exps, seq, in_dim, residual, st);
+          (size_t)m.n, m.y.data(), m.w.data(), m.s.data(), m.out.data(), digits, exps, seq, in_dim, residual, parts,
+          st);
       PyEval_RestoreThread(ts);
     }
     return finish(fn, rc);

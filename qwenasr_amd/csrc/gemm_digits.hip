@@ -25,8 +25,8 @@ constexpr int kDigits = 4;
 constexpr int kDigitBits = 30;          // |I| <= 2^30
 constexpr int kBadRow = -0x40000000;    // exponent of a row with an infinity or NaN: its outputs are NaN
 
-// One workgroup per row of up to 1024 NV floats: h = x (+ delta, written back
-// to x), with NORM the RMSNorm (h * rinv) * gain of it (kernels/mod.rs:897-918)
+// One workgroup per row of up to 1024 NV floats: h = x (+ delta, the sum of
+// `parts` slices [rows][cols] in slice order, written back to x), with NORM the RMSNorm (h * rinv) * gain of it (kernels/mod.rs:897-918)
 // and optionally that row itself, then the row's digits and exponent.
 struct DigitArgs {
   int8_t* digits;  // [4][rows][cols]
@@ -35,7 +35,7 @@ struct DigitArgs {
   const float* delta;  // nullable
   const float* gain;   // NORM
   float* x_norm;       // nullable
-  int rows, cols;
+  int rows, cols, parts;
   float eps;
 };
 
@@ -56,7 +56,11 @@ __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
     for (int i = 0; i < NV; ++i) {
       const int c = threadIdx.x + 256 * i;
       if (c < n4) {
-        const float4 d = ld4(dr, c);
+        float4 d = ld4(dr, c);
+        for (int p = 1; p < a.parts; ++p) {  // uniform
+          const float4 e = ld4(dr + (size_t)p * a.rows * a.cols, c);
+          d.x += e.x; d.y += e.y; d.z += e.z; d.w += e.w;
+        }
         v[i].x += d.x; v[i].y += d.y; v[i].z += d.z; v[i].w += d.w;
         st4(xr, c, v[i]);
       }
@@ -167,6 +171,7 @@ struct DigitGemm {
   const int8_t* digits;  // [4][T][K]
   const int32_t* exps;
   int T, K;
+  int parts;             // K cut over this many workgroups: part p writes y + p * T * N (kDgPlain)
   unsigned cols, rows, split_cols;  // the tile grid, and how the XCDs share it
   DigitHeads heads;
 };
@@ -211,11 +216,12 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
   extern __shared__ __align__(16) int8_t dg_lds[];
 
   unsigned bx, by;
+  const unsigned part = EPI == kDgPlain ? blockIdx.x / (a.cols * a.rows) : 0, block = blockIdx.x - part * a.cols * a.rows;
   if (a.split_cols == 0) {
-    bx = blockIdx.x % a.cols;
-    by = blockIdx.x / a.cols;
+    bx = block % a.cols;
+    by = block / a.cols;
   } else {
-    const unsigned xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    const unsigned xcd = block % 8, slot = block / 8;
     const unsigned ca = a.cols / a.split_cols, rb = a.rows / (8 / a.split_cols);
     bx = (xcd % a.split_cols) * ca + slot % ca;
     by = (xcd / a.split_cols) * rb + slot / ca;
@@ -243,7 +249,8 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
   const int wr = wv % WR, wc = wv / WR;
   const int r = lane & 31, g = lane >> 5;
   const int gt = (int)threadIdx.x - kg * NTG;  // thread of its group
-  const int nch = a.K / (BK * KW);
+  const int nch = a.K / (BK * KW * a.parts);
+  if constexpr (EPI == kDgPlain) y += (size_t)part * a.T * N;
   int8_t* buf = dg_lds + kg * 2 * STAGE;
 
   // row of the digit block of a token tile: 128 (t / 32) + 32 d + t % 32
@@ -252,7 +259,7 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int row = u * RPU + gt / SL, slot = gt % SL;
-    const size_t k = (size_t)kg * nch * BK + 16 * slot;
+    const size_t k = (size_t)((int)part * KW + kg) * nch * BK + 16 * slot;
     if (u < UW) {
       src[u] = w + (size_t)min(n0 + row, N - 1) * a.K + k;  // rows and tokens past the end re-read the last one
     } else {
@@ -431,7 +438,7 @@ template <int BN, int BT, int MI, int BK, int KW, int EPI>
 bool run_digit_gemm(DigitGemm a, hipStream_t st) {
   constexpr size_t lds = digit_gemm_tile_bytes<BN, BT, BK, KW>() + (BN + BT) * 4;
   static_assert(lds <= 163840, "LDS of a CU");
-  if (a.K % (BK * KW) != 0) return false;
+  if (a.K % (BK * KW * a.parts) != 0) return false;
   if (!digit_lds_ok<&digit_gemm_kernel<BN, BT, MI, BK, KW, EPI>>(lds)) return false;
   unsigned c = 0;
   for (int m = 0; m < a.n; ++m) {
@@ -453,7 +460,7 @@ bool run_digit_gemm(DigitGemm a, hipStream_t st) {
     }
   }
   digit_gemm_kernel<BN, BT, MI, BK, KW, EPI>
-      <<<a.cols * a.rows, 64 * KW * (BN / (32 * MI)) * (BT / 32), lds, st>>>(a);
+      <<<a.cols * a.rows * (unsigned)a.parts, 64 * KW * (BN / (32 * MI)) * (BT / 32), lds, st>>>(a);
   return true;
 }
 
@@ -478,9 +485,9 @@ bool launch_digit_gemm(const DigitGemm& a, hipStream_t st) {
     auto tiles = [&](int bn, int bt) {
       long long c = 0;
       for (int m = 0; m < a.n; ++m) c += (a.N[m] + bn - 1) / bn;
-      return (double)(c * ((a.T + bt - 1) / bt)) / 256.0;
+      return (double)(c * ((a.T + bt - 1) / bt) * a.parts) / 256.0;
     };
-    const double k = a.K / 1024.0, t32 = tiles(32, 32), t64 = tiles(64, 32), t128 = tiles(128, 32), t256 = tiles(256, 64);
+    const double k = a.K / (1024.0 * a.parts), t32 = tiles(32, 32), t64 = tiles(64, 32), t128 = tiles(128, 32), t256 = tiles(256, 64);
     const double c256 = 2.5 + ceil(t256) * (5.2 + 12.7 * k);
     const double c128 = 5.0 + (t128 > 1.0 ? t128 : 1.0) * 5.2 * k;
     const double c64 = 2.5 + ceil(t64) * (2.6 + 3.6 * k);
@@ -491,6 +498,17 @@ bool launch_digit_gemm(const DigitGemm& a, hipStream_t st) {
     return c128 < c256 ? run_digit_gemm<128, 32, 1, 128, 1, EPI>(a, st)
                        : run_digit_gemm<256, 64, 2, 128, 1, EPI>(a, st);
   }
+}
+
+// Parts of K for a projection whose 32 x 32 tiles leave CUs idle (a few streams'
+// o and down projections): as many, up to 4, as still give each CU at most one
+// workgroup of at least 512 of K. Their slices are added by the norm that reads
+// them (qasr_add_rms_norm_digits_f32), so no launch is added.
+size_t digit_parts(size_t T, size_t K, size_t N) {
+  const size_t tiles = ((N + 31) / 32) * ((T + 31) / 32);
+  size_t p = 1;
+  while (p < 4 && 2 * p * tiles <= 256 && K % (512 * p) == 0 && K / (2 * p) >= 512) p *= 2;
+  return p;
 }
 
 int digit_gemm_checks(size_t T, size_t K, const int8_t* digits, const int32_t* exps, const char* what) {
@@ -524,22 +542,23 @@ extern "C" int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x
   QASR_REQUIRE(rows <= kMaxRows, "digit_rows: too many rows");
   if (cols == 0 || cols % 4 != 0 || cols > 8192 || !aligned16(x) || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED, "digit_rows: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
-  const DigitArgs a{digits, exps, const_cast<float*>(x), nullptr, nullptr, nullptr, (int)rows, (int)cols, 0.0f};
+  const DigitArgs a{digits, exps, const_cast<float*>(x), nullptr, nullptr, nullptr, (int)rows, (int)cols, 1, 0.0f};
   launch_digit_rows<false>(a, as_stream(stream));
   return launch_status("digit_rows");
 }
 
-extern "C" int qasr_add_rms_norm_digits_f32(float* x, const float* delta, const float* weight, float* x_norm,
-                                            int8_t* digits, int32_t* exps, size_t rows, size_t cols, float eps,
-                                            void* stream) {
+extern "C" int qasr_add_rms_norm_digits_f32(float* x, const float* delta, size_t delta_parts, const float* weight,
+                                            float* x_norm, int8_t* digits, int32_t* exps, size_t rows, size_t cols,
+                                            float eps, void* stream) {
   if (rows == 0) return QASR_OK;
   QASR_REQUIRE(x && weight && digits && exps, "add_rms_norm_digits: null pointer");
-  QASR_REQUIRE(rows <= kMaxRows, "add_rms_norm_digits: too many rows");
+  QASR_REQUIRE(rows <= kMaxRows && delta_parts >= 1 && delta_parts <= 4,
+               "add_rms_norm_digits: too many rows, or not 1 to 4 slices of delta");
   if (cols == 0 || cols % 4 != 0 || cols > 8192 || !aligned16(x) || !aligned16(delta) || !aligned16(weight) ||
       !aligned16(x_norm) || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED,
                 "add_rms_norm_digits: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
-  const DigitArgs a{digits, exps, x, delta, weight, x_norm, (int)rows, (int)cols, eps};
+  const DigitArgs a{digits, exps, x, delta, weight, x_norm, (int)rows, (int)cols, (int)delta_parts, eps};
   launch_digit_rows<true>(a, as_stream(stream));
   return launch_status("add_rms_norm_digits");
 }
@@ -547,15 +566,17 @@ extern "C" int qasr_add_rms_norm_digits_f32(float* x, const float* delta, const 
 extern "C" int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
                                            const float* const* scales, const size_t* out_dims,
                                            const int8_t* digits, const int32_t* exps, size_t seq, size_t in_dim,
-                                           size_t residual, void* stream) {
+                                           size_t residual, size_t parts, void* stream) {
   if (seq == 0 || n_mats == 0) return QASR_OK;
   QASR_REQUIRE(n_mats <= 3 && ys && ws && scales && out_dims, "linear_digits: 1 to 3 matrices");
+  QASR_REQUIRE(parts >= 1 && parts <= 4 && (parts == 1 || !residual),
+               "linear_digits: 1 to 4 parts, and only one with a residual");
   int rc = digit_gemm_checks(seq, in_dim, digits, exps, "linear_digits");
   if (rc != QASR_OK) return rc;
   DigitGemm a{};
   a.n = (int)n_mats;
   for (size_t m = 0; m < n_mats; ++m) {
-    rc = digit_mat_checks(ys[m], ws[m], scales[m], out_dims[m], seq, in_dim, "linear_digits");
+    rc = digit_mat_checks(ys[m], ws[m], scales[m], out_dims[m], parts * seq, in_dim, "linear_digits");
     if (rc != QASR_OK) return rc;
     a.y[m] = ys[m];
     a.w[m] = ws[m];
@@ -566,10 +587,16 @@ extern "C" int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, cons
   a.exps = exps;
   a.T = (int)seq;
   a.K = (int)in_dim;
+  a.parts = (int)parts;
   const bool ok = residual ? launch_digit_gemm<kDgResidual>(a, as_stream(stream))
                            : launch_digit_gemm<kDgPlain>(a, as_stream(stream));
   if (!ok) return fail(QASR_ERR_UNSUPPORTED, "linear_digits: no kernel for this shape");
   return launch_status("linear_digits");
+}
+
+extern "C" size_t qasr_linear_digits_parts(size_t seq, size_t in_dim, size_t out_dim) {
+  if (seq == 0 || seq > 0xffffffu || out_dim > 0x3fffffffu) return 1;
+  return digit_parts(seq, in_dim, out_dim);
 }
 
 extern "C" int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_gate_up, const float* scales,
@@ -590,6 +617,7 @@ extern "C" int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_g
   a.exps = exps;
   a.T = (int)seq;
   a.K = (int)in_dim;
+  a.parts = 1;
   const bool ok = prefill ? launch_digit_gemm<kDgSwiglu>(a, as_stream(stream))
                           : launch_digit_gemm<kDgSwigluLibm>(a, as_stream(stream));
   if (!ok) return fail(QASR_ERR_UNSUPPORTED, "gate_up_swiglu_digits: no kernel for this shape");
@@ -636,6 +664,7 @@ extern "C" int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v
   a.exps = exps;
   a.T = (int)seq;
   a.K = (int)in_dim;
+  a.parts = 1;
   a.heads = {k_cache, v_cache, q_norm_w, k_norm_w, cos_tab, sin_tab, (long long)start_pos, eps};
   if (!launch_digit_gemm<kDgHeads>(a, as_stream(stream)))
     return fail(QASR_ERR_UNSUPPORTED, "qkv_heads_digits: no kernel for this shape");

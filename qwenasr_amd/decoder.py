@@ -410,6 +410,10 @@ class DecoderInt8Batched:
         if self.digits:
             self.dg = torch.empty(4 * B * max(hidden, intermediate, q_dim), dtype=torch.int8, device=device)
             self.dg_exps = torch.empty(B, dtype=torch.int32, device=device)
+            self.o_parts = K.linear_digits_parts(B, q_dim, hidden)
+            self.down_parts = K.linear_digits_parts(B, intermediate, hidden)
+            self.proj = torch.empty(self.o_parts * B * hidden, **f32)  # the parts' slices
+            self.down = torch.empty(self.down_parts * B * hidden, **f32)
         fits = self.vocab % 128 == 0 and self.vocab == self.lm.out_dim and hidden in (1024, 2048, 3072, 4096, 6144)
         if lm_head_w8a8 is None:
             lm_head_w8a8 = w8a8 and fits
@@ -438,18 +442,19 @@ class DecoderInt8Batched:
     def _layer_digits(self, l: int, lw: dict, kb, vb) -> None:
         H, I, B, nq, nk, hd, eps = self.H, self.I, self.B, self.nq, self.nk, self.hd, self.eps
         dg, ex = self.dg, self.dg_exps
-        K.add_rms_norm_digits(self.x, None if l == 0 else self.down, lw["input_norm"], None, dg, ex, B, H, eps)
+        K.add_rms_norm_digits(self.x, None if l == 0 else self.down, lw["input_norm"], None, dg, ex, B, H, eps,
+                              self.down_parts)
         K.linear_digits_int8([self.q, self.kk, self.vv], [lw["wq"], lw["wk"], lw["wv"]], dg, ex, B, H)
         K.head_rms_norm_rope_kv(self.q, self.kk, self.vv, lw["q_norm"], lw["k_norm"], self.rope, self.positions, 0, B,
                                 nq, nk, hd, eps, kb, vb, self.rows)
         K.batched_decode_attention(self.attn, self.q, kb, vb, self.rows, self.positions, B, nq, nk, hd, self.scale,
                                    self.attn_ws, order=self.order)
         K.digit_rows(dg, ex, self.attn, B, nq * hd)
-        K.linear_digits_int8([self.proj], [lw["wo"]], dg, ex, B, nq * hd)
-        K.add_rms_norm_digits(self.x, self.proj, lw["post_attn_norm"], None, dg, ex, B, H, eps)
+        K.linear_digits_int8([self.proj], [lw["wo"]], dg, ex, B, nq * hd, parts=self.o_parts)
+        K.add_rms_norm_digits(self.x, self.proj, lw["post_attn_norm"], None, dg, ex, B, H, eps, self.o_parts)
         K.gate_up_swiglu_digits_int8(self.ffn, lw["gate_up"], dg, ex, B, H, I)
         K.digit_rows(dg, ex, self.ffn, B, I)
-        K.linear_digits_int8([self.down], [lw["down"]], dg, ex, B, I)
+        K.linear_digits_int8([self.down], [lw["down"]], dg, ex, B, I, parts=self.down_parts)
 
     def decode(self, embeds: torch.Tensor) -> None:
         """One token for every stream (``embeds``: [batch, hidden]) at its
@@ -489,10 +494,14 @@ class DecoderInt8Batched:
             K.linear_w8a8_packed(self.logits, self.lm_packed, self.xq, self.xs, B, H, self.vocab)
             K.argmax_rows(self.tokens, self.logits, B, self.vocab)
             return
-        if self.digits and self.vocab % 4 == 0:
-            K.add_rms_norm_digits(self.x, self.down, self.w["norm"], self.x_norm, self.dg, self.dg_exps, B, H, eps)
-            K.linear_digits_int8([self.logits], [self.lm], self.dg, self.dg_exps, B, H)
-            K.argmax_rows(self.tokens, self.logits, B, self.vocab)
+        if self.digits:
+            K.add_rms_norm_digits(self.x, self.down, self.w["norm"], self.x_norm, self.dg, self.dg_exps, B, H, eps,
+                                  self.down_parts)
+            if self.vocab % 4 == 0 and self.vocab == self.lm.out_dim:
+                K.linear_digits_int8([self.logits], [self.lm], self.dg, self.dg_exps, B, H)
+                K.argmax_rows(self.tokens, self.logits, B, self.vocab)
+            else:
+                K.lm_head_int8_argmax(self.tokens, self.logits, self.x_norm, self.lm, B, H, self.vocab)
             return
         K.add_rms_norm(self.x, self.down, self.w["norm"], self.x_norm, B, H, eps)
         K.lm_head_int8_argmax(self.tokens, self.logits, self.x_norm, self.lm, B, H, self.vocab)

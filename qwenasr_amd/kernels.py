@@ -530,19 +530,27 @@ def digit_rows(digits, exps, x, rows: int, cols: int) -> None:
     _call.qasr_digit_rows_f32(digits, 4 * rows * cols, exps, rows, x, rows * cols, rows, cols)
 
 
-def add_rms_norm_digits(x, delta, weight, x_norm, digits, exps, rows: int, cols: int, eps: float) -> None:
-    """x += delta (None: not), then the digit rows of its RMSNorm; ``x_norm`` (or None)
+def add_rms_norm_digits(x, delta, weight, x_norm, digits, exps, rows: int, cols: int, eps: float,
+                        delta_parts: int = 1) -> None:
+    """x += delta (None: not; ``delta_parts`` slices to be added), then the digit rows of its RMSNorm; ``x_norm`` (or None)
     receives the normalised rows too."""
     n = rows * cols
-    _call.qasr_add_rms_norm_digits_f32(x, n, delta, n, weight, cols, x_norm, n, digits, 4 * n, exps, rows, rows, cols,
+    _call.qasr_add_rms_norm_digits_f32(x, n, delta, delta_parts * n, delta_parts, weight, cols, x_norm, n, digits, 4 * n, exps, rows, rows, cols,
                                        eps)
 
 
-def linear_digits_int8(ys, ws: list, digits, exps, seq_len: int, in_dim: int, residual: bool = False) -> None:
+def linear_digits_parts(seq_len: int, in_dim: int, out_dim: int) -> int:
+    """The ``parts`` worth taking for a projection of this size."""
+    return _lib.lib().qasr_linear_digits_parts(seq_len, in_dim, out_dim)
+
+
+def linear_digits_int8(ys, ws: list, digits, exps, seq_len: int, in_dim: int, residual: bool = False,
+                       parts: int = 1) -> None:
     """W8A32 projections of the same digit rows in one launch (up to 3 QuantWeights);
-    with ``residual`` each is added to its y."""
+    with ``residual`` each is added to its y. ``parts`` > 1 cuts in_dim: each y holds that
+    many slices ``[parts, seq_len, out_dim]`` to be added (``add_rms_norm_digits``)."""
     _call.qasr_linear_digits_int8_f32(ys, ws, digits, 4 * seq_len * in_dim, exps, seq_len, seq_len, in_dim,
-                                      int(residual))
+                                      int(residual), parts, parts * seq_len)
 
 
 def gate_up_swiglu_digits_int8(out, w: QuantWeight, digits, exps, seq_len: int, in_dim: int, intermediate: int,

@@ -76,6 +76,11 @@ def test_linear_digits(dev, T, K_, N):
     K.linear_digits_int8([y], [w], dg, ex, T, K_)
     ref, bound = _product(x, w)
     _near(y.view(T, N), ref, bound)
+    for parts in (2, 3, 4):
+        if K_ % (256 * parts) == 0:
+            p = torch.full((parts * T * N,), 9.0, device=dev)
+            K.linear_digits_int8([p], [w], dg, ex, T, K_, parts=parts)
+            _near(p.view(parts, T, N).double().sum(0), ref, bound)
     z = torch.ones(T * N, device=dev)
     K.linear_digits_int8([z], [w], dg, ex, T, K_, residual=True)
     assert torch.equal(z, y + 1.0)
@@ -162,10 +167,23 @@ def test_add_rms_norm_digits(dev):
             else:
                 K.add_rms_norm(b, delta, g, ref, rows, cols, 1e-6)
             assert torch.equal(a, b)
+            if delta is not None:  # slices that add up to delta exactly
+                c, dg3, ex3 = x.clone(), torch.empty_like(dg), torch.empty_like(ex)
+                half = torch.cat([delta * 0.5, delta * 0.25, delta * 0.25])
+                K.add_rms_norm_digits(c, half, g, None, dg3, ex3, rows, cols, 1e-6, 3)
+                assert torch.equal(a, c) and torch.equal(dg, dg3) and torch.equal(ex, ex3)
             # each sums the squares through at most 42 additions (half of that in the row) and rounds 3 times
             torch.testing.assert_close(xn, ref, rtol=2 * 24 * 2.0 ** -24, atol=0)
             dg2, ex2 = _digits(xn.view(rows, cols), dev)
             assert torch.equal(dg, dg2) and torch.equal(ex, ex2)
+
+
+def test_parts_worth_taking(dev):
+    from qwenasr_amd import kernels as K
+
+    assert K.linear_digits_parts(11, 2048, 1024) == 4 and K.linear_digits_parts(11, 3072, 1024) == 4
+    assert K.linear_digits_parts(64, 6144, 2048) == 2 and K.linear_digits_parts(65, 2048, 2048) == 1
+    assert K.linear_digits_parts(2, 512, 256) == 1 and K.linear_digits_parts(2, 1024, 256) == 2
 
 
 def test_refusals(dev):
@@ -177,6 +195,7 @@ def test_refusals(dev):
     y = torch.zeros(64, device=dev)
     for call in (lambda: K.linear_digits_int8([y], [w], dg, ex, 4, 384),               # in_dim not a multiple of 256
                  lambda: K.linear_digits_int8([y], [K.QuantWeight(w.data, w.scales, 6, 512)], dg, ex, 4, 512),
+                 lambda: K.linear_digits_int8([y], [w], dg, ex, 1, 512, parts=4),
                  lambda: K.digit_rows(dg, ex, x, 4, 510),
                  lambda: K.digit_rows(dg[1:], ex, x, 1, 512)):
         with pytest.raises(K.QasrError) as e:
