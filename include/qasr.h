@@ -618,7 +618,8 @@ int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v_cache, siz
  * rotated) over rows 0..pos of k_cache/v_cache + m * cache_rows *
  * n_kv_heads * head_dim (the block qasr_head_rms_norm_rope_kv_f32 with
  * positions writes). With a workspace of at least
- * qasr_batched_decode_attention_workspace_floats() floats, each stream's keys
+ * qasr_batched_decode_attention_workspace_floats() floats (or, for a few
+ * streams, of qasr_batched_decode_attention_split_workspace_floats()), each stream's keys
  * are cut into chunks of 512 (streams at different positions then cost the
  * GPU evenly) and the chunks' partial results are merged in a second launch;
  * with workspace NULL one workgroup per (stream, kv head) walks all of its

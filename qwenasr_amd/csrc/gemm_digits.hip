@@ -4,7 +4,7 @@
 // own power of two, x = 2^ex * I with |I| <= 2^30, and each I four signed
 // base-256 digits: I = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3. The dot product with an
 // int8 weight row is then four int8 dot products with exact int32 sums
-// (|sum| <= 127 * 128 * in_dim), put together in fp32 at the end:
+// (|sum| <= 2^14 in_dim, in_dim at most 65536), put together in fp32 at the end:
 //   y = (s0 + 2^8 s1 + 2^16 s2 + 2^24 s3) * 2^ex * row_scale.
 // The only roundings are the row's fixed point (2^-31 of its largest element,
 // 128 times finer than fp32's rounding of that element) and the last few fp32
@@ -514,7 +514,7 @@ size_t digit_parts(size_t T, size_t K, size_t N) {
 int digit_gemm_checks(size_t T, size_t K, const int8_t* digits, const int32_t* exps, const char* what) {
   QASR_REQUIRE(digits && exps, std::string(what) + ": null pointer");
   size_t n;
-  QASR_REQUIRE(T <= 0xffffffu && K <= 131072 && mul_ok(T, 4 * K, &n), std::string(what) + ": size too large");
+  QASR_REQUIRE(T <= 0xffffffu && K <= 65536 && mul_ok(T, 4 * K, &n), std::string(what) + ": size too large");
   if (K == 0 || K % 256 != 0 || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED, std::string(what) + ": in_dim must be a multiple of 256, digits 16-byte aligned");
   return QASR_OK;

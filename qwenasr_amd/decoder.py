@@ -5,9 +5,10 @@ Per layer, in the reference's order:
   the previous layer's residual add + input RMSNorm + q/k/v projections (one
   launch), q/k head RMSNorm + RoPE, the K/V rows written into the cache and
   causal attention over the layer's cache block (one launch with the keys
-  split over workgroups, then the merge), o projection, residual add +
+  split over workgroups; past 8 splits a merge launch), o projection (which
+  merges up to 8 splits itself), residual add +
   post-attention RMSNorm + gate/up projection + SwiGLU (one launch), down
-  projection: 6 launches.
+  projection: 5 or 6 launches.
 The fused add + RMSNorm + projection launches normalise the row inside every
 workgroup, in the element order of the standalone add_rms_norm kernel, so the
 results equal the unfused sequence (``fuse_norms=False``: add_rms_norm, then
@@ -25,7 +26,12 @@ RMSNorm + RoPE with the chunk's K/V rows written into the cache (in the q/k/v
 GEMM's epilogue where that launch fills the chip, else a launch of its own),
 causal attention over the cache (matrix cores), o, residual add +
 post-attention RMSNorm, gate/up with the prefill SwiGLU (fast_exp form) in its
-epilogue, down: 7 or 8 launches per layer, then the last residual add.
+epilogue, down: 7 or 8 launches per layer, then the last residual add. From
+5 tokens on (``prefill_digits``) the projections run from digit rows instead:
+RMSNorm + digits, q/k/v with the heads in the epilogue, attention, its rows'
+digits, o with the residual add, RMSNorm + digits, gate/up + SwiGLU, digits,
+down with the residual add, all GEMMs on the int8 matrix cores with exact
+integer sums.
 
 Weights come from ``qint8.load_decoder_int8`` (or any dict of the same
 layout); ``DecoderInt8.decode`` runs one token and can be captured in a HIP
@@ -341,6 +347,11 @@ class DecoderInt8Batched:
     steps) makes the lm_head one too: the final add + RMSNorm quantizes the
     rows in the same launch, the logits are ((f32)dot * x_scale) * row_scale,
     each stream's argmax follows; otherwise the lm_head stays W8A32.
+
+    Without ``w8a8``, from two streams on, the projections run from digit rows
+    (``K.linear_digits_int8``: exact integer products, the activations in 31-bit
+    fixed point per row): the norms write the rows' digits, and a few streams' o
+    and down projections come in parts of K that the next norm adds.
 
     ``attn_chunked`` (default: when batch * n_kv_heads < 1024) also cuts each
     stream's keys into chunks for the attention, to give a small batch enough

@@ -210,7 +210,8 @@ def batched_decode_attention(out, q, k_cache, v_cache, cache_rows: int, position
     """Decode attention of ``batch`` streams, each over rows 0..positions[m] of its
     own cache block ``[batch, cache_rows, n_kv_heads * head_dim]`` (decoder.rs:900-903
     per stream). With ``workspace`` (batched_decode_workspace) every stream's
-    keys are cut into chunks of 512 and the chunk partials merged; without it
+    keys are cut into chunks of 512 (shorter ones for a few streams, with
+    batched_decode_split_workspace) and the chunk partials merged; without it
     one workgroup per (stream, kv head) walks all of its keys. ``out_q`` /
     ``out_scales`` (int8 [batch * n_heads * head_dim], f32 [batch]) also get each
     stream's row quantized per row, as quantize_rows_i8 would on ``out``."""
