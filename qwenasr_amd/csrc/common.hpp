@@ -10,6 +10,7 @@
 #include <stdint.h>
 #include <stddef.h>
 
+#include <atomic>
 #include <string>
 
 #include "../../include/qasr.h"
@@ -281,6 +282,29 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 inline bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
+
+// Raises kernel Fn's dynamic-LDS limit (64 KiB by default) to `bytes` on the
+// current device. The attribute is per device, so the outcome is remembered
+// per device (0 unknown, 1 set, -1 unavailable); concurrent first calls may
+// both set it, which is harmless. Returns false if the device cannot give a
+// workgroup that much LDS.
+template <auto Fn>
+bool raise_lds_limit(size_t bytes) {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<signed char> state[kMaxDevices];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
+  const signed char known = state[dev].load(std::memory_order_acquire);
+  if (known != 0) return known > 0;
+  int max_lds = 0;
+  const bool ok =
+      hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
+      (size_t)max_lds >= bytes &&
+      hipFuncSetAttribute(reinterpret_cast<const void*>(Fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)bytes) == hipSuccess;
+  state[dev].store(ok ? 1 : -1, std::memory_order_release);
+  return ok;
+}
 
 // Largest size any kernel indexes with 64-bit arithmetic; guards products of
 // dimensions against overflow.

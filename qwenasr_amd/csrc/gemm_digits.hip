@@ -426,20 +426,12 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
   }
 }
 
-template <auto Kernel>
-bool digit_lds_ok(size_t bytes) {
-  static const bool ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)bytes) == hipSuccess;
-  return ok;
-}
-
 template <int BN, int BT, int MI, int BK, int KW, int EPI>
 bool run_digit_gemm(DigitGemm a, hipStream_t st) {
   constexpr size_t lds = digit_gemm_tile_bytes<BN, BT, BK, KW>() + (BN + BT) * 4;
   static_assert(lds <= 163840, "LDS of a CU");
   if (a.K % (BK * KW * a.parts) != 0) return false;
-  if (!digit_lds_ok<&digit_gemm_kernel<BN, BT, MI, BK, KW, EPI>>(lds)) return false;
+  if (!raise_lds_limit<&digit_gemm_kernel<BN, BT, MI, BK, KW, EPI>>(lds)) return false;
   unsigned c = 0;
   for (int m = 0; m < a.n; ++m) {
     a.bx_begin[m] = c;
@@ -448,6 +440,8 @@ bool run_digit_gemm(DigitGemm a, hipStream_t st) {
   for (int m = a.n; m <= 3; ++m) a.bx_begin[m] = c;
   a.cols = c;
   a.rows = (unsigned)((a.T + BT - 1) / BT);
+  constexpr unsigned kThreads = 64 * KW * (BN / (32 * MI)) * (BT / 32);
+  if (!exact_grid_ok((size_t)a.cols * a.rows * (size_t)a.parts * kThreads)) return false;
   // the XCD map that reads least: cols / s weight blocks and rows / (8 / s) token blocks each
   a.split_cols = 0;
   double best = 0;
@@ -460,7 +454,7 @@ bool run_digit_gemm(DigitGemm a, hipStream_t st) {
     }
   }
   digit_gemm_kernel<BN, BT, MI, BK, KW, EPI>
-      <<<a.cols * a.rows * (unsigned)a.parts, 64 * KW * (BN / (32 * MI)) * (BT / 32), lds, st>>>(a);
+      <<<a.cols * a.rows * (unsigned)a.parts, kThreads, lds, st>>>(a);
   return true;
 }
 
@@ -539,7 +533,7 @@ extern "C" int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x
                                    void* stream) {
   if (rows == 0) return QASR_OK;
   QASR_REQUIRE(digits && exps && x, "digit_rows: null pointer");
-  QASR_REQUIRE(rows <= kMaxRows, "digit_rows: too many rows");
+  QASR_REQUIRE(rows < kMaxRows, "digit_rows: too many rows");
   if (cols == 0 || cols % 4 != 0 || cols > 8192 || !aligned16(x) || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED, "digit_rows: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
   const DigitArgs a{digits, exps, const_cast<float*>(x), nullptr, nullptr, nullptr, (int)rows, (int)cols, 1, 0.0f};
@@ -552,7 +546,7 @@ extern "C" int qasr_add_rms_norm_digits_f32(float* x, const float* delta, size_t
                                             float eps, void* stream) {
   if (rows == 0) return QASR_OK;
   QASR_REQUIRE(x && weight && digits && exps, "add_rms_norm_digits: null pointer");
-  QASR_REQUIRE(rows <= kMaxRows && delta_parts >= 1 && delta_parts <= 4,
+  QASR_REQUIRE(rows < kMaxRows && delta_parts >= 1 && delta_parts <= 4,
                "add_rms_norm_digits: too many rows, or not 1 to 4 slices of delta");
   if (cols == 0 || cols % 4 != 0 || cols > 8192 || !aligned16(x) || !aligned16(delta) || !aligned16(weight) ||
       !aligned16(x_norm) || !aligned16(digits) || !aligned4(exps))

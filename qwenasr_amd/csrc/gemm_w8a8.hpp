@@ -269,29 +269,6 @@ inline bool gemm_w8a8_lds_shape(size_t K, size_t inter) {
   return (K == 1024 || K == 2048) && (2 * inter) % kLdsBN == 0;
 }
 
-// Raises kernel Fn's dynamic-LDS limit (64 KiB by default) to `bytes` on the
-// current device. The attribute is per device, so the outcome is remembered
-// per device (0 unknown, 1 set, -1 unavailable); concurrent first calls may
-// both set it, which is harmless. Returns false if the device cannot give a
-// workgroup that much LDS.
-template <auto Fn>
-bool raise_lds_limit(size_t bytes) {
-  constexpr int kMaxDevices = 64;
-  static std::atomic<signed char> state[kMaxDevices];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
-  const signed char known = state[dev].load(std::memory_order_acquire);
-  if (known != 0) return known > 0;
-  int max_lds = 0;
-  const bool ok =
-      hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
-      (size_t)max_lds >= bytes &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(Fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)bytes) == hipSuccess;
-  state[dev].store(ok ? 1 : -1, std::memory_order_release);
-  return ok;
-}
-
 // The staged X tile needs up to 64 x 2064 bytes.
 template <int KSTEPS>
 bool lds_kernel_ready(size_t lds) {

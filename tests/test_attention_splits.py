@@ -31,6 +31,24 @@ def test_one_token_split_edges(dev, pos):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nq,nk,hd", [(8, 1, 128), (8, 8, 128), (16, 4, 128), (4, 4, 64), (8, 1, 64), (8, 2, 64)])
+def test_one_token_split_other_heads(dev, nq, nk, hd):
+    from qwenasr_amd import kernels as K
+
+    kv = nk * hd
+    for pos in (0, 5, 63, 64, 130, 255):
+        r = np.random.default_rng([85, pos, nq])
+        q = r.standard_normal(nq * hd).astype(np.float32)
+        k, v = (r.standard_normal((pos + 1) * kv).astype(np.float32) for _ in range(2))
+        d = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+        out = torch.full((nq * hd,), 9.0, device=dev)
+        K.causal_attention_split(out, d(q), d(k), d(v), 1, pos + 1, nq, nk, hd, hd ** -0.5, pos,
+                                 K.attention_workspace(1, nq, hd, dev))
+        ref = oracle.causal_attention(q, k, v, 1, pos + 1, nq, nk, hd, hd ** -0.5, pos)
+        np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=1e-5, err_msg=f"pos {pos}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,start,nq,nk", [(77, 610, 16, 8), (128, 385, 16, 8), (16, 1000, 16, 8), (9, 3000, 16, 8),
                                            (33, 400, 8, 8), (40, 2000, 16, 4), (20, 4200, 16, 2), (77, 179, 16, 8)])
 def test_prefill_key_splits(dev, T, start, nq, nk):
