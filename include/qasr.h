@@ -688,8 +688,10 @@ int qasr_argmax_rows_f32(int32_t* idx, const float* x, size_t rows, size_t cols,
  * workspace (8-byte aligned, may be NULL): with rows == 1 and at least
  * qasr_lm_head_argmax_workspace_bytes(vocab) bytes, the matvec reduces its
  * rows to per-workgroup candidates there and one small kernel merges them
- * (no second pass over the logits). Without it, or for rows > 1, the logits
- * are scanned after the matvec. Same idx either way. Calls that share a
+ * (no second pass over the logits). With rows > 1 and room for their digit rows
+ * (rows * (4 * in_dim + 4) bytes, 16-byte aligned; in_dim a multiple of 256 up
+ * to 8192) the logits come from qasr_linear_digits_int8_f32, which rounds less.
+ * Otherwise the logits are scanned after the matvec. Same idx for the same logits. Calls that share a
  * workspace must be ordered on one stream. */
 int qasr_lm_head_int8_argmax_f32(int32_t* idx, float* logits, const float* x,
                                  const int8_t* w, const float* scales, size_t rows,
@@ -705,7 +707,7 @@ size_t qasr_lm_head_argmax_workspace_bytes(size_t vocab);
  * The one-row candidates go to a 512 KiB array the library holds on each GPU
  * it runs on until the process ends (looked up once per device on the first
  * call there; nothing is allocated, no call here allocates). Same results as
- * qasr_lm_head_int8_argmax_f32 with a workspace. One row needs in_dim
+ * qasr_lm_head_int8_argmax_f32 with a workspace for one row, without one for several. One row needs in_dim
  * 1024..8192 in steps of 1024 and 16-byte aligned x and w (UNSUPPORTED
  * otherwise); vocab at most QASR_LM_HEAD_NOALLOC_MAX_VOCAB (INVALID_ARG
  * otherwise). rows > 1 writes the logits and scans them, as the workspace

@@ -281,7 +281,7 @@ def argmax_rows(idx, x, rows: int, cols: int) -> None:
 
 
 def lm_head_workspace(vocab: int, device="cuda") -> torch.Tensor:
-    """Workspace for the one-token lm_head argmax (bytes as a uint8 tensor)."""
+    """Workspace for the lm_head argmax (bytes as a uint8 tensor)."""
     n = _lib.lib().qasr_lm_head_argmax_workspace_bytes(vocab)
     return torch.empty(max(n, 8), dtype=torch.uint8, device=device)
 
@@ -289,7 +289,8 @@ def lm_head_workspace(vocab: int, device="cuda") -> torch.Tensor:
 def lm_head_int8_argmax(idx, logits, x, w: QuantWeight, rows: int, in_dim: int, vocab: int,
                         workspace: torch.Tensor | None = None) -> None:
     """INT8 lm_head logits + greedy argmax (decoder.rs:935-963). With a
-    ``lm_head_workspace`` and one row the argmax is reduced inside the matvec."""
+    ``lm_head_workspace`` and one row the argmax is reduced inside the matvec; several
+    rows that fit it as digit rows run on the int8 matrix cores."""
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     _call.qasr_lm_head_int8_argmax_f32(idx, rows, logits, rows * vocab, x, rows * in_dim, w.data, vocab * in_dim,
                                        w.scales, vocab, rows, in_dim, vocab, workspace, ws_bytes)

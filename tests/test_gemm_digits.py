@@ -178,6 +178,23 @@ def test_add_rms_norm_digits(dev):
             assert torch.equal(dg, dg2) and torch.equal(ex, ex2)
 
 
+@pytest.mark.parametrize("rows,K_,vocab", [(2, 1024, 4000), (7, 2048, 3004), (32, 1024, 33000), (40, 2048, 1000)])
+def test_lm_head_rows_from_digits(dev, rows, K_, vocab):
+    """Several rows with a workspace that holds their digits (the last one's does not, and
+    takes the general projection): logits against 64 bits, the first largest wins."""
+    from qwenasr_amd import kernels as K
+
+    x = torch.randn(rows, K_, device=dev)
+    w = _weight(vocab, K_, dev, rows)
+    ws = torch.empty(8 * 37984 if vocab > 1000 else 4096, dtype=torch.uint8, device=dev)
+    logits, idx = torch.empty(rows * vocab, device=dev), torch.empty(rows, dtype=torch.int32, device=dev)
+    K.lm_head_int8_argmax(idx, logits, x.view(-1), w, rows, K_, vocab, ws)
+    got = logits.view(rows, vocab)
+    ref, bound = _product(x, w)
+    _near(got, ref, bound if vocab > 1000 else 1e-5 * bound / (10 * 2.0 ** -24))
+    assert torch.equal(idx.long(), got.argmax(-1))
+
+
 def test_parts_worth_taking(dev):
     from qwenasr_amd import kernels as K
 
