@@ -571,18 +571,35 @@ int qasr_decode_attention_linear_int8_f32(float* y, float* out, float* q, const 
  * own power of two, x = 2^exps[r] * I with |I| <= 2^30, each I as four signed
  * base-256 digits: plane d of digits ([4][rows][cols] int8) holds digit d, the
  * lowest first. The *_digits_* projections take such rows: their int8 weights
- * meet the digits on the int8 matrix cores with exact integer sums, so they
- * round less than an fp32 accumulation of the same dot product. A row with an
- * infinity or NaN gives NaN outputs. cols a multiple of 4, at most 8192.
- * No reference counterpart (its INT8 linears multiply in fp32). */
+ * meet the digits on the int8 matrix cores with exact integer sums. What is
+ * left is the fixed step: at most 2^-30 of the row's largest element per
+ * element, so an output is within 2^-30 max|x| sum|w| scale of the exact one
+ * (and a few fp32 roundings). That is less than an fp32 accumulation of the same
+ * dot product rounds, unless its weights are 0 at elements far above the rest.
+ * A row with an infinity or NaN gives NaN outputs. cols a multiple of 4, at
+ * most 8192. No reference counterpart (its INT8 linears multiply in fp32).
+ *
+ * The _wide forms keep fp32 precision for every row: the writers mark a row
+ * whose largest magnitude is above 128 times its mean magnitude, or which holds
+ * an infinity or NaN (exps = QASR_DIGITS_WIDE_ROW, digits of no meaning), and the
+ * projections multiply marked rows in fp32 from x, the floats that the digits
+ * were made from ([seq][in_dim], 16-byte aligned; only marked rows are read).
+ * With x NULL a marked row gives NaN outputs. */
+#define QASR_DIGITS_WIDE_ROW (-0x40000001)
 int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
                         void* stream);
+int qasr_digit_rows_wide_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
+                             void* stream);
 /* x += delta (nullable; the sum of delta_parts slices [rows][cols], 1 to 4, as
- * qasr_linear_digits_int8_f32 writes them), then the digit rows of its RMSNorm (kernels/mod.rs:897-918);
- * x_norm (nullable) receives the normalised rows too. */
+ * qasr_linear_digits_int8_f32 writes them), then the digit rows of its RMSNorm
+ * (kernels/mod.rs:897-918); x_norm (nullable) receives the normalised rows too. */
 int qasr_add_rms_norm_digits_f32(float* x, const float* delta, size_t delta_parts, const float* weight,
                                  float* x_norm, int8_t* digits, int32_t* exps, size_t rows, size_t cols,
                                  float eps, void* stream);
+/* The same with wide rows marked; x_norm (not NULL) receives the marked rows, or all with all_rows != 0. */
+int qasr_add_rms_norm_digits_wide_f32(float* x, const float* delta, size_t delta_parts, const float* weight,
+                                      float* x_norm, size_t all_rows, int8_t* digits, int32_t* exps,
+                                      size_t rows, size_t cols, float eps, void* stream);
 /* W8A32 projections (kernels/mod.rs:650-661) of digit rows, 1 to 3 matrices of
  * the same input in one launch; residual != 0: y += projection. With parts > 1
  * (at most 4, no residual, in_dim a multiple of 256 * parts) in_dim is cut into
@@ -594,6 +611,10 @@ int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, const int8_t* c
                                 const float* const* scales, const size_t* out_dims, const int8_t* digits,
                                 const int32_t* exps, size_t seq, size_t in_dim, size_t residual,
                                 size_t parts, void* stream);
+int qasr_linear_digits_wide_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
+                                     const float* const* scales, const size_t* out_dims, const int8_t* digits,
+                                     const int32_t* exps, const float* x, size_t seq, size_t in_dim,
+                                     size_t residual, size_t parts, void* stream);
 size_t qasr_linear_digits_parts(size_t seq, size_t in_dim, size_t out_dim);
 /* The interleaved gate/up projection of digit rows with the SwiGLU: the decode
  * loop's (decoder.rs:916-921, libm exp) or, prefill != 0, swiglu_multiply's
@@ -601,6 +622,10 @@ size_t qasr_linear_digits_parts(size_t seq, size_t in_dim, size_t out_dim);
 int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_gate_up, const float* scales,
                                         const int8_t* digits, const int32_t* exps, size_t seq, size_t in_dim,
                                         size_t inter, size_t prefill, void* stream);
+int qasr_gate_up_swiglu_digits_wide_int8_f32(float* out, const int8_t* w_gate_up, const float* scales,
+                                             const int8_t* digits, const int32_t* exps, const float* x,
+                                             size_t seq, size_t in_dim, size_t inter, size_t prefill,
+                                             void* stream);
 /* As qasr_qkv_heads_int8_f32, from digit rows: the q/k/v projections of a
  * prefill chunk, q/k head RMSNorm + RoPE at start_pos + t, K/V rows into the
  * layer's cache blocks (decoder.rs:795-810). head_dim 128. */
@@ -611,6 +636,14 @@ int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v_cache, siz
                                    size_t n_kv_heads, size_t head_dim, const float* q_norm_w,
                                    const float* k_norm_w, const float* cos_tab, const float* sin_tab,
                                    size_t table_rows, size_t start_pos, float eps, void* stream);
+int qasr_qkv_heads_digits_wide_int8_f32(float* q, float* k_cache, float* v_cache, size_t cache_rows,
+                                        const int8_t* wq, const float* sq, const int8_t* wk, const float* sk,
+                                        const int8_t* wv, const float* sv, const int8_t* digits,
+                                        const int32_t* exps, const float* x, size_t seq, size_t in_dim,
+                                        size_t n_heads, size_t n_kv_heads, size_t head_dim,
+                                        const float* q_norm_w, const float* k_norm_w, const float* cos_tab,
+                                        const float* sin_tab, size_t table_rows, size_t start_pos, float eps,
+                                        void* stream);
 
 /* Decode attention of `batch` streams, each over its own cache block
  * (decoder.rs:900-903 per stream): for stream m at pos = positions[m], out[m]
@@ -690,7 +723,7 @@ int qasr_argmax_rows_f32(int32_t* idx, const float* x, size_t rows, size_t cols,
  * rows to per-workgroup candidates there and one small kernel merges them
  * (no second pass over the logits). With rows > 1 and room for their digit rows
  * (rows * (4 * in_dim + 4) bytes, 16-byte aligned; in_dim a multiple of 256 up
- * to 8192) the logits come from qasr_linear_digits_int8_f32, which rounds less.
+ * to 8192) the logits come from qasr_linear_digits_wide_int8_f32.
  * Otherwise the logits are scanned after the matvec. Same idx for the same logits. Calls that share a
  * workspace must be ordered on one stream. */
 int qasr_lm_head_int8_argmax_f32(int32_t* idx, float* logits, const float* x,

@@ -88,10 +88,16 @@ SIGNATURES: dict[str, list] = {
     "qasr_pack_w8a8_tiles": [P, P, Z, Z, P],
     "qasr_gate_up_swiglu_w8a8_packed": [P, P, P, P, P, Z, Z, Z, P],
     "qasr_digit_rows_f32": [P, P, P, Z, Z, P],
+    "qasr_digit_rows_wide_f32": [P, P, P, Z, Z, P],
     "qasr_add_rms_norm_digits_f32": [P, P, Z, P, P, P, P, Z, Z, F, P],
+    "qasr_add_rms_norm_digits_wide_f32": [P, P, Z, P, P, Z, P, P, Z, Z, F, P],
     "qasr_linear_digits_int8_f32": [Z, P, P, P, P, P, P, Z, Z, Z, Z, P],
+    "qasr_linear_digits_wide_int8_f32": [Z, P, P, P, P, P, P, P, Z, Z, Z, Z, P],
     "qasr_gate_up_swiglu_digits_int8_f32": [P, P, P, P, P, Z, Z, Z, Z, P],
+    "qasr_gate_up_swiglu_digits_wide_int8_f32": [P, P, P, P, P, P, Z, Z, Z, Z, P],
     "qasr_qkv_heads_digits_int8_f32": [P, P, P, Z, P, P, P, P, P, P, P, P, Z, Z, Z, Z, Z, P, P, P, P, Z, Z, F, P],
+    "qasr_qkv_heads_digits_wide_int8_f32": [P, P, P, Z, P, P, P, P, P, P, P, P, P, Z, Z, Z, Z, Z, P, P, P, P, Z, Z, F,
+                                            P],
     "qasr_linear_w8a8_packed": [P, P, P, P, P, Z, Z, Z, P],
     "qasr_batched_decode_attention_f32": [P, P, P, P, Z, P, Z, Z, Z, Z, F, P, Z, P, P, P, P],
     "qasr_batched_decode_order_i32": [P, P, Z, Z, P],

@@ -250,10 +250,12 @@ QASR_BIND(qasr_linear_w8a8_packed, "y", "w.data", "w.scales", "xq", "x_scales")
 QASR_BIND(qasr_qkv_heads_w8a8_packed, "q_out", "k_cache", "v_cache", "w.data", "w.scales", "xq", "x_scales",
           "q_norm_w", "k_norm_w", "cos", "sin", "positions")
 QASR_BIND(qasr_digit_rows_f32, "digits", "exps", "x")
+QASR_BIND(qasr_digit_rows_wide_f32, "digits", "exps", "x")
 QASR_BIND(qasr_add_rms_norm_digits_f32, "x", "?delta", "weight", "?x_norm", "digits", "exps")
-QASR_BIND(qasr_gate_up_swiglu_digits_int8_f32, "out", "w.data", "w.scales", "digits", "exps")
-QASR_BIND(qasr_qkv_heads_digits_int8_f32, "q", "k_cache", "v_cache", "wq", "wq.scales", "wk", "wk.scales", "wv",
-          "wv.scales", "digits", "exps", "q_norm_w", "k_norm_w", "cos", "sin")
+QASR_BIND(qasr_add_rms_norm_digits_wide_f32, "x", "?delta", "weight", "x_norm", "digits", "exps")
+QASR_BIND(qasr_gate_up_swiglu_digits_wide_int8_f32, "out", "w.data", "w.scales", "digits", "exps", "?x")
+QASR_BIND(qasr_qkv_heads_digits_wide_int8_f32, "q", "k_cache", "v_cache", "wq", "wq.scales", "wk", "wk.scales", "wv",
+          "wv.scales", "digits", "exps", "?x", "q_norm_w", "k_norm_w", "cos", "sin")
 QASR_BIND(qasr_causal_attention_f32, "out", "q", "?k", "?v")
 QASR_BIND(qasr_causal_attention_split_f32, "out", "q", "?k", "?v", "workspace")
 QASR_BIND(qasr_decode_attention_f32, "out", "q", "k", "v", "q_norm_w", "k_norm_w", "cos", "sin", "k_cache", "v_cache",
@@ -368,28 +370,29 @@ PyObject* py_norm_multi(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
-// (ys, ws, digits, n, exps, n, seq_len, in_dim, residual, parts, rows); ys hold rows = parts * seq_len rows
+// (ys, ws, digits, n, exps, n, x, n, seq_len, in_dim, residual, parts, rows); ys hold rows = parts * seq_len rows
 PyObject* py_digits(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
-    static const char* const names[] = {"digits", "exps"};
-    const char* fn = "qasr_linear_digits_int8_f32";
+    static const char* const names[] = {"digits", "exps", "?x"};
+    const char* fn = "qasr_linear_digits_wide_int8_f32";
     Args a{args, n, names, fn};
-    if (n != 11) {
-      PyErr_Format(PyExc_TypeError, "%s: takes 11 arguments", fn);
+    if (n != 13) {
+      PyErr_Format(PyExc_TypeError, "%s: takes 13 arguments", fn);
       throw PyError();
     }
-    const Mats m = take_mats(a, args[10], args[7]);
+    const Mats m = take_mats(a, args[12], args[9]);
     const int8_t* digits = take<const int8_t*, false>(a);
     const int32_t* exps = take<const int32_t*, false>(a);
+    const float* x = take<const float*, false>(a);
     const size_t seq = size_arg(a.next()), in_dim = size_arg(a.next()), residual = size_arg(a.next());
     const size_t parts = size_arg(a.next());
     void* st = take<void*, true>(a);
     int rc;
     {
       PyThreadState* ts = PyEval_SaveThread();
-      rc = reinterpret_cast<decltype(&qasr_linear_digits_int8_f32)>(Entry<Tag_digits>::address)(
-          (size_t)m.n, m.y.data(), m.w.data(), m.s.data(), m.out.data(), digits, exps, seq, in_dim, residual, parts,
-          st);
+      rc = reinterpret_cast<decltype(&qasr_linear_digits_wide_int8_f32)>(Entry<Tag_digits>::address)(
+          (size_t)m.n, m.y.data(), m.w.data(), m.s.data(), m.out.data(), digits, exps, x, seq, in_dim, residual,
+          parts, st);
       PyEval_RestoreThread(ts);
     }
     return finish(fn, rc);
@@ -442,9 +445,11 @@ Bound g_bound[] = {
     QASR_ENTRY(qasr_linear_w8a8_packed),
     QASR_ENTRY(qasr_qkv_heads_w8a8_packed),
     QASR_ENTRY(qasr_digit_rows_f32),
+    QASR_ENTRY(qasr_digit_rows_wide_f32),
     QASR_ENTRY(qasr_add_rms_norm_digits_f32),
-    QASR_ENTRY(qasr_gate_up_swiglu_digits_int8_f32),
-    QASR_ENTRY(qasr_qkv_heads_digits_int8_f32),
+    QASR_ENTRY(qasr_add_rms_norm_digits_wide_f32),
+    QASR_ENTRY(qasr_gate_up_swiglu_digits_wide_int8_f32),
+    QASR_ENTRY(qasr_qkv_heads_digits_wide_int8_f32),
     QASR_ENTRY(qasr_causal_attention_f32),
     QASR_ENTRY(qasr_causal_attention_split_f32),
     QASR_ENTRY(qasr_decode_attention_f32),
@@ -456,7 +461,7 @@ Bound g_bound[] = {
     {"qasr_linear_nobias_int8_multi_f32", (PyCFunction)(void (*)(void))py_multi, &Entry<Tag_multi>::address},
     {"qasr_add_rms_norm_linear_nobias_int8_multi_f32", (PyCFunction)(void (*)(void))py_norm_multi,
      &Entry<Tag_norm_multi>::address},
-    {"qasr_linear_digits_int8_f32", (PyCFunction)(void (*)(void))py_digits, &Entry<Tag_digits>::address},
+    {"qasr_linear_digits_wide_int8_f32", (PyCFunction)(void (*)(void))py_digits, &Entry<Tag_digits>::address},
 };
 constexpr size_t kBound = sizeof(g_bound) / sizeof(g_bound[0]);
 PyMethodDef g_defs[kBound];

@@ -153,6 +153,22 @@ QASR_DEV void st4_nt(float* p, size_t i, float4 v) {
 }
 
 // ---------------------------------------------------------------------------
+// Operands of the bf16 matrix cores
+// ---------------------------------------------------------------------------
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+QASR_DEV float bf16_trunc(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
+// bf16 bits of two floats, truncated, packed low element first
+QASR_DEV unsigned bf16_pair(float lo_elem, float hi_elem) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi_elem), __float_as_uint(lo_elem), 0x07060302u);
+}
+QASR_DEV unsigned bf16_pair_i8(int v, int byte) {  // bytes byte, byte + 1 of v as two bf16
+  return bf16_pair((float)(int8_t)((v >> (8 * byte)) & 0xff), (float)(int8_t)((v >> (8 * byte + 8)) & 0xff));
+}
+
+// ---------------------------------------------------------------------------
 // Scalar math shared by several kernels
 // ---------------------------------------------------------------------------
 

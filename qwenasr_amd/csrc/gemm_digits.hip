@@ -1,18 +1,31 @@
 // INT8-weight projections of fp32 activations on the int8 matrix cores.
 //
-// A row of activations becomes fixed-point numbers of 31 bits under the row's
-// own power of two, x = 2^ex * I with |I| <= 2^30, and each I four signed
-// base-256 digits: I = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3. The dot product with an
-// int8 weight row is then four int8 dot products with exact int32 sums
+// A row of activations becomes fixed-point numbers of 30 bits and a sign under
+// the row's own power of two, x = 2^ex * I with |I| <= 2^30, and each I four
+// signed base-256 digits: I = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3. The dot product
+// with an int8 weight row is then four int8 dot products with exact int32 sums
 // (|sum| <= 2^14 in_dim, in_dim at most 65536), put together in fp32 at the end:
 //   y = (s0 + 2^8 s1 + 2^16 s2 + 2^24 s3) * 2^ex * row_scale.
-// The only roundings are the row's fixed point (2^-31 of its largest element,
-// 128 times finer than fp32's rounding of that element) and the last few fp32
-// operations, against one per product for an fp32 accumulator. The int8
+// The only roundings are the row's fixed point (at most 2^-30 of its largest
+// element, 64 times finer than fp32's rounding of that element) and the last few
+// fp32 operations, against one per product for an fp32 accumulator. The int8
 // matrix cores run at twice the bf16 rate, so four digits cost two bf16
 // products where the three-way bf16 split costs three, and neither operand is
 // converted in the GEMM: weights and digits go from memory to LDS to the
 // matrix cores as they are. The digits take the bytes of the fp32 row.
+//
+// Wide rows. The fixed step is one for the whole row, so an element far below
+// the largest keeps fewer than fp32's 24 bits, and an output whose weights are 0
+// at the few largest elements would be off by more than an fp32 sum. The writers
+// of digit rows therefore mark (when asked, kWideRow) each row whose largest
+// magnitude is above kWideRange times its mean magnitude, or which holds an
+// infinity or NaN; the GEMMs then multiply that row in fp32 precision from its
+// floats (wide_rows below), in the token tiles that hold such a row alone. For
+// an unmarked row, leaving out its largest element leaves a row whose 2-norm is
+// at least max (cols / kWideRange - 1) / sqrt(cols), so the fixed point's error
+// in a dot product with the rest is at most about
+//   2^-29 / sqrt(12) kWideRange / (1 - kWideRange / cols) = 8e-8 (1024 columns)
+// of the product's size, at or below that of an fp32 accumulation.
 #include "common.hpp"
 
 namespace qasr {
@@ -24,10 +37,16 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int kDigits = 4;
 constexpr int kDigitBits = 30;          // |I| <= 2^30
 constexpr int kBadRow = -0x40000000;    // exponent of a row with an infinity or NaN: its outputs are NaN
+constexpr int kWideRow = -0x40000001;   // exponent of a row that the GEMMs take from its floats
+constexpr float kWideRange = 128.0f;    // largest over mean magnitude from which a row is wide
+
+// Which rows of x_norm the norm writes, and whether it marks wide rows.
+enum DigitWide { kNoWide = 0, kWideAllNorm = 1, kWideOwnNorm = 2 };
 
 // One workgroup per row of up to 1024 NV floats: h = x (+ delta, the sum of
-// `parts` slices [rows][cols] in slice order, written back to x), with NORM the RMSNorm (h * rinv) * gain of it (kernels/mod.rs:897-918)
-// and optionally that row itself, then the row's digits and exponent.
+// `parts` slices [rows][cols] in slice order, written back to x), with NORM the
+// RMSNorm (h * rinv) * gain of it (kernels/mod.rs:897-918) and optionally that
+// row itself, then the row's digits and exponent.
 struct DigitArgs {
   int8_t* digits;  // [4][rows][cols]
   int32_t* exps;   // [rows]
@@ -37,11 +56,32 @@ struct DigitArgs {
   float* x_norm;       // nullable
   int rows, cols, parts;
   float eps;
+  int wide;            // DigitWide; kWideOwnNorm: x_norm gets the wide rows alone
 };
+
+// The largest of `big` and the sum of `sum` over a workgroup of 256, in one pass
+// through LDS.
+QASR_DEV void block_max_sum(float& big, float& sum, float (&lds)[2][256 / kWave]) {
+  big = wave_max(big);
+  sum = wave_sum(sum);
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  if (lane == 0) {
+    lds[0][w] = big;
+    lds[1][w] = sum;
+  }
+  __syncthreads();
+  big = lds[0][0];
+  sum = lds[1][0];
+#pragma unroll
+  for (int i = 1; i < 256 / kWave; ++i) {
+    big = fmaxf(big, lds[0][i]);
+    sum += lds[1][i];
+  }
+}
 
 template <int NV, bool NORM>
 __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
-  __shared__ float red[256 / kWave];
+  __shared__ float red[2][256 / kWave];
   const int row = blockIdx.x, n4 = a.cols >> 2;
   float* xr = a.x + (size_t)row * a.cols;
   float4 v[NV];
@@ -81,7 +121,7 @@ __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
       ss += v[i].z * v[i].z;
       ss += v[i].w * v[i].w;
     }
-    ss = block_sum<256>(ss, red);
+    ss = block_sum<256>(ss, red[0]);
     const float rinv = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -90,7 +130,7 @@ __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
       v[i].y = (v[i].y * rinv) * g[i].y;
       v[i].z = (v[i].z * rinv) * g[i].z;
       v[i].w = (v[i].w * rinv) * g[i].w;
-      if (a.x_norm && c < n4) st4(a.x_norm + (size_t)row * a.cols, c, v[i]);
+      if (a.x_norm && a.wide != kWideOwnNorm && c < n4) st4(a.x_norm + (size_t)row * a.cols, c, v[i]);
     }
   }
   // the largest magnitude; an infinity or NaN counts as infinity
@@ -98,13 +138,27 @@ __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
     const float m = fabsf(f);
     return m <= 3.402823466e38f ? m : __builtin_inff();
   };
-  float big = 0.0f;
+  float big = 0.0f, sum = 0.0f;  // the sum scaled by 2^-13 (cols <= 2^13): it cannot overflow
 #pragma unroll
-  for (int i = 0; i < NV; ++i) big = fmaxf(big, fmaxf(fmaxf(mag(v[i].x), mag(v[i].y)), fmaxf(mag(v[i].z), mag(v[i].w))));
-  big = block_max<256>(big, red);
+  for (int i = 0; i < NV; ++i) {
+    const float m0 = mag(v[i].x), m1 = mag(v[i].y), m2 = mag(v[i].z), m3 = mag(v[i].w);
+    big = fmaxf(big, fmaxf(fmaxf(m0, m1), fmaxf(m2, m3)));
+    sum += (m0 * 0x1p-13f + m1 * 0x1p-13f) + (m2 * 0x1p-13f + m3 * 0x1p-13f);
+  }
+  block_max_sum(big, sum, red);
   const bool bad = big == __builtin_inff();
+  const bool wide = a.wide && (bad || big > sum * (kWideRange * 0x1p13f / (float)a.cols));
   const int up = bad ? 0 : kDigitBits - __builtin_amdgcn_frexp_expf(big);  // big < 2^exp (0 for a row of zeros)
-  if (threadIdx.x == 0) a.exps[row] = bad ? kBadRow : -up;
+  if (threadIdx.x == 0) a.exps[row] = wide ? kWideRow : bad ? kBadRow : -up;
+  if constexpr (NORM) {
+    if (a.wide == kWideOwnNorm && wide) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int c = threadIdx.x + 256 * i;
+        if (c < n4) st4(a.x_norm + (size_t)row * a.cols, c, v[i]);
+      }
+    }
+  }
   // byte d of (I + 0x00808080) ^ 0x00808080 is digit d: adding 128 to the lower
   // three bytes carries into the next one where a digit is negative
   auto digits_of = [&](float f) {
@@ -170,6 +224,7 @@ struct DigitGemm {
   int n;
   const int8_t* digits;  // [4][T][K]
   const int32_t* exps;
+  const float* x;        // [T][K], read for rows marked kWideRow; null: such rows give NaN
   int T, K;
   int parts;             // K cut over this many workgroups: part p writes y + p * T * N (kDgPlain)
   unsigned cols, rows, split_cols;  // the tile grid, and how the XCDs share it
@@ -182,6 +237,83 @@ constexpr size_t digit_gemm_tile_bytes() {
   constexpr size_t stages = (size_t)KW * 2 * (BN + kDigits * BT) * BK;
   constexpr size_t tiles = (size_t)KW * BT * (BN + 4) * sizeof(float);
   return stages > tiles ? stages : tiles;
+}
+
+// acc[i] = the dot products of a 32-token block's wide rows with MI 32-row weight
+// blocks over nk (a multiple of 64) of K, with the sums of the bf16 split
+// (int8.hip): an int8 weight is exact in bf16, an fp32 activation is
+// hi + mid + lo exactly, and the products are summed in fp32. The operands come
+// straight from memory (L2), a 64-wide chunk ahead: of every 32 of K, lane (r, g)
+// loads 16 weights of row r and 16 floats of a token, the first 8 of each for one
+// matrix instruction and the rest for the next (the same permutation of K for
+// both). xp and wp[i] point at the lane's first ones; lanes of other tokens pass
+// a wide one's xp, so that no load is conditional, and their columns mean
+// nothing. An infinity or NaN travels as in fp32: hi alone carries an infinity.
+// What a launch costs without, with one and with only wide rows, and the bf16
+// split on the same product (us): 64 tokens [2048 -> 12288] 14, 34, 51 and 20;
+// 77 [3072 -> 1024] 9, 17, 23 and 13; 8 [2048 -> 151936] 63, 140, 150 and 131.
+// Each wave converts its own operands and shares nothing through LDS, which is
+// what the split's launches are faster by where every row is wide.
+template <int MI>
+QASR_DEV void wide_rows(v16f (&acc)[MI], const int8_t* const (&wp)[MI], const float* xp, int nk) {
+  v16f low[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) acc[i] = low[i] = v16f{};
+  struct Chunk {
+    v4i w[MI][2];
+    v4f x[2][4];
+  };
+  auto load = [&](Chunk& c, int k) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i) c.w[i][h] = *reinterpret_cast<const v4i*>(wp[i] + k + 32 * h);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) c.x[h][q] = *reinterpret_cast<const v4f*>(xp + k + 32 * h + 4 * q);
+    }
+  };
+  auto multiply = [&](const Chunk& c) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {  // 16 of K: half h % 2 of the lane's 16 of 32-block h / 2
+      v4u b[3];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        float e[2], r1[2], r2[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          e[j] = c.x[h >> 1][2 * (h & 1) + (p >> 1)][2 * (p & 1) + j];
+          r1[j] = fabsf(e[j]) == __builtin_inff() ? 0.0f : e[j] - bf16_trunc(e[j]);
+          r2[j] = r1[j] - bf16_trunc(r1[j]);  // at most 8 significant bits
+        }
+        b[0][p] = bf16_pair(e[0], e[1]);
+        b[1][p] = bf16_pair(r1[0], r1[1]);
+        b[2][p] = bf16_pair(r2[0], r2[1]);
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const int w0 = c.w[i][h >> 1][2 * (h & 1)], w1 = c.w[i][h >> 1][2 * (h & 1) + 1];
+        const v8bf a = __builtin_bit_cast(v8bf, v4u{bf16_pair_i8(w0, 0), bf16_pair_i8(w0, 2), bf16_pair_i8(w1, 0),
+                                                    bf16_pair_i8(w1, 2)});
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(v8bf, b[0]), acc[i], 0, 0, 0);
+        low[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(v8bf, b[1]), low[i], 0, 0, 0);
+        low[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(v8bf, b[2]), low[i], 0, 0, 0);
+      }
+    }
+  };
+  Chunk c[2];
+  load(c[0], 0);
+  for (int k = 0; k < nk; k += 128) {
+    load(c[1], min(k + 64, nk - 64));  // past the end: the last chunk again, not multiplied
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(c[0]);
+    if (k + 64 < nk) {  // uniform
+      load(c[0], min(k + 128, nk - 64));
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(c[1]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MI; ++i) acc[i] += low[i];
 }
 
 // One BN x BT output tile (BT tokens, so 4 BT digit columns) per workgroup.
@@ -273,7 +405,11 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
   float* sc_lds = reinterpret_cast<float*>(dg_lds + TILE_BYTES);
   int* ex_lds = reinterpret_cast<int*>(sc_lds + BN);
   if ((int)threadIdx.x < BN) sc_lds[threadIdx.x] = scales[min(n0 + (int)threadIdx.x, N - 1)];
-  if ((int)threadIdx.x < BT) ex_lds[threadIdx.x] = a.exps[min(t0 + (int)threadIdx.x, a.T - 1)];
+  if ((int)threadIdx.x < BT) {
+    const int e = a.exps[min(t0 + (int)threadIdx.x, a.T - 1)];
+    ex_lds[threadIdx.x] = e == kWideRow && a.x ? 0 : e;  // a wide row's floats have no power of two
+  }
+  const int t_wave = min(t0 + 32 * wc + r, a.T - 1), e_wave = a.exps[t_wave];  // looked at after the loop
   v4i st[U];
   {
     v4i first[U];
@@ -347,8 +483,30 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
         }
         *reinterpret_cast<float4*>(mine + 32 * (MI * wr + i) + 8 * q + 4 * g) = make_float4(f[0], f[1], f[2], f[3]);
       }
+    // This wave's wide rows again, from the floats: its own part of the tile, its own part of K.
+    const unsigned wide_tokens = a.x ? (unsigned)__ballot(e_wave == kWideRow) : 0u;
+    if (wide_tokens) {
+      const size_t k = (size_t)((int)part * KW + kg) * nch * BK + 16 * g;
+      const int8_t* wp[MI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) wp[i] = w + (size_t)min(n0 + 32 * (MI * wr + i) + r, N - 1) * a.K + k;
+      const bool wide = wide_tokens >> r & 1;
+      const int t = wide ? t_wave : min(t0 + 32 * wc + __builtin_ctz(wide_tokens), a.T - 1);
+      v16f f[MI];
+      wide_rows<MI>(f, wp, a.x + (size_t)t * a.K + k, nch * BK);
+      if (wide) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4*>(mine + 32 * (MI * wr + i) + 8 * q + 4 * g) =
+                make_float4(f[i][4 * q], f[i][4 * q + 1], f[i][4 * q + 2], f[i][4 * q + 3]);
+      }
+    }
   }
   __syncthreads();
+  // a sum of products times the token's power of two
+  auto powered = [](float v, int ex) { return ex <= kBadRow ? qnan() : ldexpf(v, ex); };
   if constexpr (EPI == kDgHeads) {
     // 16 lanes a head: lane `sub` holds dims 4 sub.. and 64 + 4 sub..
     constexpr int L = 16, PER = NT / L;
@@ -372,8 +530,8 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
           f.x += q.x; f.y += q.y; f.z += q.z; f.w += q.w;
         }
         const float4 sc = *reinterpret_cast<const float4*>(sc_lds + c);
-        auto one = [&](float v, float s) { return ex == kBadRow ? qnan() : ldexpf(v * s, ex); };
-        return make_float4(one(f.x, sc.x), one(f.y, sc.y), one(f.z, sc.z), one(f.w, sc.w));
+        return make_float4(powered(f.x * sc.x, ex), powered(f.y * sc.y, ex), powered(f.z * sc.z, ex),
+                           powered(f.w * sc.w, ex));
       };
       float4 x1 = value(4 * sub), x2 = value(64 + 4 * sub);
       if (mat != 2) head_norm_rope<128, true, true>(x1, x2, w1, w2, c1, c2, s1, s2, true, he.eps);
@@ -408,7 +566,7 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
     const int ex = ex_lds[tt];
     float res[4] = {f.x * sc.x, f.y * sc.y, f.z * sc.z, f.w * sc.w};
 #pragma unroll
-    for (int v = 0; v < 4; ++v) res[v] = ex == kBadRow ? qnan() : ldexpf(res[v], ex);
+    for (int v = 0; v < 4; ++v) res[v] = powered(res[v], ex);
     if (t >= a.T || n >= N) continue;
     if constexpr (EPI == kDgSwiglu || EPI == kDgSwigluLibm) {
       const int inter = N >> 1, j = n >> 1, fast_end = EPI == kDgSwiglu ? inter & ~7 : 0;
@@ -505,12 +663,14 @@ size_t digit_parts(size_t T, size_t K, size_t N) {
   return p;
 }
 
-int digit_gemm_checks(size_t T, size_t K, const int8_t* digits, const int32_t* exps, const char* what) {
+int digit_gemm_checks(size_t T, size_t K, const int8_t* digits, const int32_t* exps, const float* x,
+                      const char* what) {
   QASR_REQUIRE(digits && exps, std::string(what) + ": null pointer");
   size_t n;
   QASR_REQUIRE(T <= 0xffffffu && K <= 65536 && mul_ok(T, 4 * K, &n), std::string(what) + ": size too large");
-  if (K == 0 || K % 256 != 0 || !aligned16(digits) || !aligned4(exps))
-    return fail(QASR_ERR_UNSUPPORTED, std::string(what) + ": in_dim must be a multiple of 256, digits 16-byte aligned");
+  if (K == 0 || K % 256 != 0 || !aligned16(digits) || !aligned4(exps) || !aligned16(x))
+    return fail(QASR_ERR_UNSUPPORTED,
+                std::string(what) + ": in_dim must be a multiple of 256, digits and x 16-byte aligned");
   return QASR_OK;
 }
 
@@ -529,43 +689,69 @@ int digit_mat_checks(const float* y, const int8_t* w, const float* s, size_t N, 
 
 using namespace qasr;
 
-extern "C" int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
-                                   void* stream) {
+static int digit_rows(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols, DigitWide wide,
+                      void* stream) {
   if (rows == 0) return QASR_OK;
   QASR_REQUIRE(digits && exps && x, "digit_rows: null pointer");
   QASR_REQUIRE(rows < kMaxRows, "digit_rows: too many rows");
   if (cols == 0 || cols % 4 != 0 || cols > 8192 || !aligned16(x) || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED, "digit_rows: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
-  const DigitArgs a{digits, exps, const_cast<float*>(x), nullptr, nullptr, nullptr, (int)rows, (int)cols, 1, 0.0f};
+  const DigitArgs a{digits, exps, const_cast<float*>(x), nullptr, nullptr, nullptr, (int)rows, (int)cols, 1, 0.0f,
+                    wide};
   launch_digit_rows<false>(a, as_stream(stream));
   return launch_status("digit_rows");
 }
 
-extern "C" int qasr_add_rms_norm_digits_f32(float* x, const float* delta, size_t delta_parts, const float* weight,
-                                            float* x_norm, int8_t* digits, int32_t* exps, size_t rows, size_t cols,
-                                            float eps, void* stream) {
+extern "C" int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
+                                   void* stream) {
+  return digit_rows(digits, exps, x, rows, cols, kNoWide, stream);
+}
+
+extern "C" int qasr_digit_rows_wide_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
+                                        void* stream) {
+  return digit_rows(digits, exps, x, rows, cols, kWideAllNorm, stream);
+}
+
+static int add_rms_norm_digits(float* x, const float* delta, size_t delta_parts, const float* weight, float* x_norm,
+                               DigitWide wide, int8_t* digits, int32_t* exps, size_t rows, size_t cols, float eps,
+                               void* stream) {
   if (rows == 0) return QASR_OK;
-  QASR_REQUIRE(x && weight && digits && exps, "add_rms_norm_digits: null pointer");
+  QASR_REQUIRE(x && weight && digits && exps && (x_norm || wide == kNoWide), "add_rms_norm_digits: null pointer");
   QASR_REQUIRE(rows < kMaxRows && delta_parts >= 1 && delta_parts <= 4,
                "add_rms_norm_digits: too many rows, or not 1 to 4 slices of delta");
   if (cols == 0 || cols % 4 != 0 || cols > 8192 || !aligned16(x) || !aligned16(delta) || !aligned16(weight) ||
       !aligned16(x_norm) || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED,
                 "add_rms_norm_digits: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
-  const DigitArgs a{digits, exps, x, delta, weight, x_norm, (int)rows, (int)cols, (int)delta_parts, eps};
+  const DigitArgs a{digits, exps, x, delta, weight, x_norm, (int)rows, (int)cols, (int)delta_parts, eps, wide};
   launch_digit_rows<true>(a, as_stream(stream));
   return launch_status("add_rms_norm_digits");
 }
 
-extern "C" int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
-                                           const float* const* scales, const size_t* out_dims,
-                                           const int8_t* digits, const int32_t* exps, size_t seq, size_t in_dim,
-                                           size_t residual, size_t parts, void* stream) {
+extern "C" int qasr_add_rms_norm_digits_f32(float* x, const float* delta, size_t delta_parts, const float* weight,
+                                            float* x_norm, int8_t* digits, int32_t* exps, size_t rows, size_t cols,
+                                            float eps, void* stream) {
+  return add_rms_norm_digits(x, delta, delta_parts, weight, x_norm, kNoWide, digits, exps, rows, cols, eps, stream);
+}
+
+extern "C" int qasr_add_rms_norm_digits_wide_f32(float* x, const float* delta, size_t delta_parts,
+                                                 const float* weight, float* x_norm, size_t all_rows,
+                                                 int8_t* digits, int32_t* exps, size_t rows, size_t cols, float eps,
+                                                 void* stream) {
+  return add_rms_norm_digits(x, delta, delta_parts, weight, x_norm, all_rows ? kWideAllNorm : kWideOwnNorm, digits,
+                             exps, rows, cols, eps, stream);
+}
+
+extern "C" int qasr_linear_digits_wide_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
+                                                const float* const* scales, const size_t* out_dims,
+                                                const int8_t* digits, const int32_t* exps, const float* x,
+                                                size_t seq, size_t in_dim, size_t residual, size_t parts,
+                                                void* stream) {
   if (seq == 0 || n_mats == 0) return QASR_OK;
   QASR_REQUIRE(n_mats <= 3 && ys && ws && scales && out_dims, "linear_digits: 1 to 3 matrices");
   QASR_REQUIRE(parts >= 1 && parts <= 4 && (parts == 1 || !residual),
                "linear_digits: 1 to 4 parts, and only one with a residual");
-  int rc = digit_gemm_checks(seq, in_dim, digits, exps, "linear_digits");
+  int rc = digit_gemm_checks(seq, in_dim, digits, exps, x, "linear_digits");
   if (rc != QASR_OK) return rc;
   DigitGemm a{};
   a.n = (int)n_mats;
@@ -579,6 +765,7 @@ extern "C" int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, cons
   }
   a.digits = digits;
   a.exps = exps;
+  a.x = x;
   a.T = (int)seq;
   a.K = (int)in_dim;
   a.parts = (int)parts;
@@ -588,16 +775,25 @@ extern "C" int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, cons
   return launch_status("linear_digits");
 }
 
+extern "C" int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
+                                           const float* const* scales, const size_t* out_dims,
+                                           const int8_t* digits, const int32_t* exps, size_t seq, size_t in_dim,
+                                           size_t residual, size_t parts, void* stream) {
+  return qasr_linear_digits_wide_int8_f32(n_mats, ys, ws, scales, out_dims, digits, exps, nullptr, seq, in_dim,
+                                          residual, parts, stream);
+}
+
 extern "C" size_t qasr_linear_digits_parts(size_t seq, size_t in_dim, size_t out_dim) {
   if (seq == 0 || seq > 0xffffffu || out_dim > 0x3fffffffu) return 1;
   return digit_parts(seq, in_dim, out_dim);
 }
 
-extern "C" int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_gate_up, const float* scales,
-                                                   const int8_t* digits, const int32_t* exps, size_t seq,
-                                                   size_t in_dim, size_t inter, size_t prefill, void* stream) {
+extern "C" int qasr_gate_up_swiglu_digits_wide_int8_f32(float* out, const int8_t* w_gate_up, const float* scales,
+                                                        const int8_t* digits, const int32_t* exps, const float* x,
+                                                        size_t seq, size_t in_dim, size_t inter, size_t prefill,
+                                                        void* stream) {
   if (seq == 0 || inter == 0) return QASR_OK;
-  int rc = digit_gemm_checks(seq, in_dim, digits, exps, "gate_up_swiglu_digits");
+  int rc = digit_gemm_checks(seq, in_dim, digits, exps, x, "gate_up_swiglu_digits");
   if (rc != QASR_OK) return rc;
   rc = digit_mat_checks(out, w_gate_up, scales, 2 * inter, seq, in_dim, "gate_up_swiglu_digits");
   if (rc != QASR_OK) return rc;
@@ -609,6 +805,7 @@ extern "C" int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_g
   a.N[0] = (int)(2 * inter);
   a.digits = digits;
   a.exps = exps;
+  a.x = x;
   a.T = (int)seq;
   a.K = (int)in_dim;
   a.parts = 1;
@@ -618,13 +815,19 @@ extern "C" int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_g
   return launch_status("gate_up_swiglu_digits");
 }
 
-extern "C" int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v_cache, size_t cache_rows,
-                                              const int8_t* wq, const float* sq, const int8_t* wk, const float* sk,
-                                              const int8_t* wv, const float* sv, const int8_t* digits,
-                                              const int32_t* exps, size_t seq, size_t in_dim, size_t n_heads,
-                                              size_t n_kv_heads, size_t head_dim, const float* q_norm_w,
-                                              const float* k_norm_w, const float* cos_tab, const float* sin_tab,
-                                              size_t table_rows, size_t start_pos, float eps, void* stream) {
+extern "C" int qasr_gate_up_swiglu_digits_int8_f32(float* out, const int8_t* w_gate_up, const float* scales,
+                                                   const int8_t* digits, const int32_t* exps, size_t seq,
+                                                   size_t in_dim, size_t inter, size_t prefill, void* stream) {
+  return qasr_gate_up_swiglu_digits_wide_int8_f32(out, w_gate_up, scales, digits, exps, nullptr, seq, in_dim, inter,
+                                                  prefill, stream);
+}
+
+extern "C" int qasr_qkv_heads_digits_wide_int8_f32(
+    float* q, float* k_cache, float* v_cache, size_t cache_rows, const int8_t* wq, const float* sq, const int8_t* wk,
+    const float* sk, const int8_t* wv, const float* sv, const int8_t* digits, const int32_t* exps, const float* x,
+    size_t seq, size_t in_dim, size_t n_heads, size_t n_kv_heads, size_t head_dim, const float* q_norm_w,
+    const float* k_norm_w, const float* cos_tab, const float* sin_tab, size_t table_rows, size_t start_pos, float eps,
+    void* stream) {
   if (seq == 0 || n_heads == 0) return QASR_OK;
   const char* what = "qkv_heads_digits";
   QASR_REQUIRE(q_norm_w && k_norm_w && cos_tab && sin_tab, "qkv_heads_digits: null pointer");
@@ -636,7 +839,7 @@ extern "C" int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v
                "qkv_heads_digits: rows start_pos..start_pos+seq exceed the cache or the RoPE table");
   if (head_dim != 128 || !aligned16(q_norm_w) || !aligned16(k_norm_w) || !aligned16(cos_tab) || !aligned16(sin_tab))
     return fail(QASR_ERR_UNSUPPORTED, "qkv_heads_digits: head_dim must be 128, tables and gains 16-byte aligned");
-  int rc = digit_gemm_checks(seq, in_dim, digits, exps, what);
+  int rc = digit_gemm_checks(seq, in_dim, digits, exps, x, what);
   if (rc != QASR_OK) return rc;
   size_t n;
   QASR_REQUIRE(mul_ok(cache_rows, n_kv_heads * 128, &n), "qkv_heads_digits: size overflows");
@@ -656,6 +859,7 @@ extern "C" int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v
   }
   a.digits = digits;
   a.exps = exps;
+  a.x = x;
   a.T = (int)seq;
   a.K = (int)in_dim;
   a.parts = 1;
@@ -663,4 +867,16 @@ extern "C" int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v
   if (!launch_digit_gemm<kDgHeads>(a, as_stream(stream)))
     return fail(QASR_ERR_UNSUPPORTED, "qkv_heads_digits: no kernel for this shape");
   return launch_status(what);
+}
+
+extern "C" int qasr_qkv_heads_digits_int8_f32(float* q, float* k_cache, float* v_cache, size_t cache_rows,
+                                              const int8_t* wq, const float* sq, const int8_t* wk, const float* sk,
+                                              const int8_t* wv, const float* sv, const int8_t* digits,
+                                              const int32_t* exps, size_t seq, size_t in_dim, size_t n_heads,
+                                              size_t n_kv_heads, size_t head_dim, const float* q_norm_w,
+                                              const float* k_norm_w, const float* cos_tab, const float* sin_tab,
+                                              size_t table_rows, size_t start_pos, float eps, void* stream) {
+  return qasr_qkv_heads_digits_wide_int8_f32(q, k_cache, v_cache, cache_rows, wq, sq, wk, sk, wv, sv, digits, exps,
+                                             nullptr, seq, in_dim, n_heads, n_kv_heads, head_dim, q_norm_w, k_norm_w,
+                                             cos_tab, sin_tab, table_rows, start_pos, eps, stream);
 }

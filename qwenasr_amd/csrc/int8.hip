@@ -718,9 +718,6 @@ bool matvec_shape(size_t in_dim) { return in_dim % 1024 == 0 && in_dim >= 1024 &
 // MFMA operands: A[i][k] (lane i + 16*(k/8), element k%8) = weight row i,
 // B[k][j] = token j; the result lane l holds rows 4*(l/16)+v of token l%16.
 // ---------------------------------------------------------------------------
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int kGmBK = 64;           // K granularity of the GEMM path
 // GEMM epilogues: y = acc * scale; + bias; or the SwiGLU of each interleaved
 // (gate, up) row pair, y[t, n/2] = swiglu(y[t, n], y[t, n + 1]), an output row
@@ -741,13 +738,6 @@ constexpr int kGemmXNorm = 8;
 constexpr int kGemmPrefetch = 1;
 constexpr int kGemmSets = 2;
 constexpr int kGemmPcSets = 4;  // the producer/consumer kernel's register sets (chunks in flight)
-
-QASR_DEV unsigned short bf16_bits_trunc(float v) { return (unsigned short)(__float_as_uint(v) >> 16); }
-QASR_DEV float bf16_trunc(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
-// bf16 bits of two floats, truncated, packed low element first
-QASR_DEV unsigned bf16_pair(float lo_elem, float hi_elem) {
-  return __builtin_amdgcn_perm(__float_as_uint(hi_elem), __float_as_uint(lo_elem), 0x07060302u);
-}
 
 // BN weight rows x BT tokens per workgroup (BN in {64, 128}, BT in {32, 64});
 // the 4 waves form a 2 x 2 grid of (BN/2) x (BT/2) tiles.
@@ -1560,10 +1550,6 @@ inline unsigned xcd_split_cols(unsigned cols, unsigned rows, int BN, int BT) {
 // gets its own accumulator (three independent chains for the matrix pipe),
 // added hi + mid + lo at the end. The KW partial tiles are added in LDS in
 // wave order.
-QASR_DEV unsigned bf16_pair_i8(int v, int byte) {  // bytes byte, byte + 1 of v as two bf16
-  return bf16_pair((float)(int8_t)((v >> (8 * byte)) & 0xff), (float)(int8_t)((v >> (8 * byte + 8)) & 0xff));
-}
-
 template <int MI, int MJ>
 struct KsplitRaw {
   v4i w[MI][2];          // per 32-wide chunk: 16 int8 of one weight row

@@ -180,9 +180,10 @@ extern "C" int qasr_lm_head_int8_argmax_f32(int32_t* idx, float* logits, const f
       aligned16(x) && aligned16(w) && aligned16(scales) && aligned16(logits)) {
     int8_t* digits = static_cast<int8_t*>(workspace);
     int32_t* exps = reinterpret_cast<int32_t*>(digits + 4 * plane);
-    int rc = qasr_digit_rows_f32(digits, exps, x, rows, in_dim, stream);
+    int rc = qasr_digit_rows_wide_f32(digits, exps, x, rows, in_dim, stream);
     if (rc == QASR_OK)
-      rc = qasr_linear_digits_int8_f32(1, &logits, &w, &scales, &vocab, digits, exps, rows, in_dim, 0, 1, stream);
+      rc = qasr_linear_digits_wide_int8_f32(1, &logits, &w, &scales, &vocab, digits, exps, x, rows, in_dim, 0, 1,
+                                            stream);
     if (rc == QASR_OK) return qasr_argmax_rows_f32(idx, logits, rows, vocab, stream);
     if (rc != QASR_ERR_UNSUPPORTED) return rc;
   }

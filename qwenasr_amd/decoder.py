@@ -164,21 +164,21 @@ class DecoderInt8:
 
     def _prefill_digits(self, T: int, start_pos: int) -> None:
         H, I, nq, nk, hd, eps = self.H, self.I, self.nq, self.nk, self.hd, self.eps
-        x, dg, ex, rows = self.px, self.pdigits, self.pexps, self.kv.max_seq
+        x, xn, dg, ex, rows = self.px, self.pxn, self.pdigits, self.pexps, self.kv.max_seq  # xn: the wide rows
         k_blocks, v_blocks = self.kv.layer_blocks()
         for l, lw in enumerate(self.w["layers"]):
             kb, vb = k_blocks[l], v_blocks[l]
-            K.add_rms_norm_digits(x, None, lw["input_norm"], None, dg, ex, T, H, eps)
+            K.add_rms_norm_digits(x, None, lw["input_norm"], xn, dg, ex, T, H, eps, 1, True, False)
             K.qkv_heads_digits_int8(self.pq, kb, vb, rows, lw["wq"], lw["wk"], lw["wv"], dg, ex, T, H, nq, nk, hd,
-                                    lw["q_norm"], lw["k_norm"], self.rope, start_pos, eps)
+                                    lw["q_norm"], lw["k_norm"], self.rope, start_pos, eps, xn)
             K.causal_attention_split(self.pattn, self.pq, kb, vb, T, start_pos + T, nq, nk, hd, self.scale, start_pos,
                                      self.pattn_ws)
-            K.digit_rows(dg, ex, self.pattn, T, nq * hd)
-            K.linear_digits_int8([x], [lw["wo"]], dg, ex, T, nq * hd, residual=True)
-            K.add_rms_norm_digits(x, None, lw["post_attn_norm"], None, dg, ex, T, H, eps)
-            K.gate_up_swiglu_digits_int8(self.pgate, lw["gate_up"], dg, ex, T, H, I, prefill=True)
-            K.digit_rows(dg, ex, self.pgate, T, I)
-            K.linear_digits_int8([x], [lw["down"]], dg, ex, T, I, residual=True)
+            K.digit_rows(dg, ex, self.pattn, T, nq * hd, True)
+            K.linear_digits_int8([x], [lw["wo"]], dg, ex, T, nq * hd, True, 1, self.pattn)
+            K.add_rms_norm_digits(x, None, lw["post_attn_norm"], xn, dg, ex, T, H, eps, 1, True, False)
+            K.gate_up_swiglu_digits_int8(self.pgate, lw["gate_up"], dg, ex, T, H, I, True, xn)
+            K.digit_rows(dg, ex, self.pgate, T, I, True)
+            K.linear_digits_int8([x], [lw["down"]], dg, ex, T, I, True, 1, self.pgate)
 
     def prefill(self, embeds: torch.Tensor, T: int, start_pos: int | None = None) -> None:
         """T tokens at positions start_pos.. (decoder.rs:751-847): writes cache rows
@@ -452,20 +452,21 @@ class DecoderInt8Batched:
 
     def _layer_digits(self, l: int, lw: dict, kb, vb) -> None:
         H, I, B, nq, nk, hd, eps = self.H, self.I, self.B, self.nq, self.nk, self.hd, self.eps
-        dg, ex = self.dg, self.dg_exps
-        K.add_rms_norm_digits(self.x, None if l == 0 else self.down, lw["input_norm"], None, dg, ex, B, H, eps,
-                              self.down_parts)
-        K.linear_digits_int8([self.q, self.kk, self.vv], [lw["wq"], lw["wk"], lw["wv"]], dg, ex, B, H)
+        xn, dg, ex = self.x_norm, self.dg, self.dg_exps  # xn: the wide rows
+        K.add_rms_norm_digits(self.x, None if l == 0 else self.down, lw["input_norm"], xn, dg, ex, B, H, eps,
+                              self.down_parts, True, False)
+        K.linear_digits_int8([self.q, self.kk, self.vv], [lw["wq"], lw["wk"], lw["wv"]], dg, ex, B, H, False, 1, xn)
         K.head_rms_norm_rope_kv(self.q, self.kk, self.vv, lw["q_norm"], lw["k_norm"], self.rope, self.positions, 0, B,
                                 nq, nk, hd, eps, kb, vb, self.rows)
         K.batched_decode_attention(self.attn, self.q, kb, vb, self.rows, self.positions, B, nq, nk, hd, self.scale,
                                    self.attn_ws, order=self.order)
-        K.digit_rows(dg, ex, self.attn, B, nq * hd)
-        K.linear_digits_int8([self.proj], [lw["wo"]], dg, ex, B, nq * hd, parts=self.o_parts)
-        K.add_rms_norm_digits(self.x, self.proj, lw["post_attn_norm"], None, dg, ex, B, H, eps, self.o_parts)
-        K.gate_up_swiglu_digits_int8(self.ffn, lw["gate_up"], dg, ex, B, H, I)
-        K.digit_rows(dg, ex, self.ffn, B, I)
-        K.linear_digits_int8([self.down], [lw["down"]], dg, ex, B, I, parts=self.down_parts)
+        K.digit_rows(dg, ex, self.attn, B, nq * hd, True)
+        K.linear_digits_int8([self.proj], [lw["wo"]], dg, ex, B, nq * hd, False, self.o_parts, self.attn)
+        K.add_rms_norm_digits(self.x, self.proj, lw["post_attn_norm"], xn, dg, ex, B, H, eps, self.o_parts, True,
+                              False)
+        K.gate_up_swiglu_digits_int8(self.ffn, lw["gate_up"], dg, ex, B, H, I, False, xn)
+        K.digit_rows(dg, ex, self.ffn, B, I, True)
+        K.linear_digits_int8([self.down], [lw["down"]], dg, ex, B, I, False, self.down_parts, self.ffn)
 
     def decode(self, embeds: torch.Tensor) -> None:
         """One token for every stream (``embeds``: [batch, hidden]) at its
@@ -507,9 +508,9 @@ class DecoderInt8Batched:
             return
         if self.digits:
             K.add_rms_norm_digits(self.x, self.down, self.w["norm"], self.x_norm, self.dg, self.dg_exps, B, H, eps,
-                                  self.down_parts)
+                                  self.down_parts, True)
             if self.vocab % 4 == 0 and self.vocab == self.lm.out_dim:
-                K.linear_digits_int8([self.logits], [self.lm], self.dg, self.dg_exps, B, H)
+                K.linear_digits_int8([self.logits], [self.lm], self.dg, self.dg_exps, B, H, x=self.x_norm)
                 K.argmax_rows(self.tokens, self.logits, B, self.vocab)
             else:
                 K.lm_head_int8_argmax(self.tokens, self.logits, self.x_norm, self.lm, B, H, self.vocab)

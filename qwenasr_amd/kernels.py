@@ -526,19 +526,28 @@ def linear_nobias_int8_multi(ys, ws: list, x, seq_len: int, in_dim: int) -> None
     _call.qasr_linear_nobias_int8_multi_f32(ys, ws, x, seq_len * in_dim, seq_len, in_dim)
 
 
-def digit_rows(digits, exps, x, rows: int, cols: int) -> None:
+def digit_rows(digits, exps, x, rows: int, cols: int, wide: bool = False) -> None:
     """Rows of x as four int8 digit planes (``digits`` [4 * rows * cols]) and a power of
-    two per row (``exps``, int32), for the ``*_digits`` projections."""
-    _call.qasr_digit_rows_f32(digits, 4 * rows * cols, exps, rows, x, rows * cols, rows, cols)
+    two per row (``exps``, int32), for the ``*_digits`` projections. The digits hold x to
+    2^-30 of the row's largest element; with ``wide`` a row whose elements range too far
+    for that is marked, and a projection given ``x`` multiplies it in fp32 instead."""
+    fn = _call.qasr_digit_rows_wide_f32 if wide else _call.qasr_digit_rows_f32
+    fn(digits, 4 * rows * cols, exps, rows, x, rows * cols, rows, cols)
 
 
 def add_rms_norm_digits(x, delta, weight, x_norm, digits, exps, rows: int, cols: int, eps: float,
-                        delta_parts: int = 1) -> None:
-    """x += delta (None: not; ``delta_parts`` slices to be added), then the digit rows of its RMSNorm; ``x_norm`` (or None)
-    receives the normalised rows too."""
+                        delta_parts: int = 1, wide: bool = False, all_rows: bool = True) -> None:
+    """x += delta (None: not; ``delta_parts`` slices to be added), then the digit rows of
+    its RMSNorm; ``x_norm`` (or None) receives the normalised rows too. ``wide`` as in
+    ``digit_rows``; then ``x_norm`` is needed, and without ``all_rows`` receives the marked
+    rows only."""
     n = rows * cols
-    _call.qasr_add_rms_norm_digits_f32(x, n, delta, delta_parts * n, delta_parts, weight, cols, x_norm, n, digits, 4 * n, exps, rows, rows, cols,
-                                       eps)
+    if wide:
+        _call.qasr_add_rms_norm_digits_wide_f32(x, n, delta, delta_parts * n, delta_parts, weight, cols, x_norm, n,
+                                                int(all_rows), digits, 4 * n, exps, rows, rows, cols, eps)
+    else:
+        _call.qasr_add_rms_norm_digits_f32(x, n, delta, delta_parts * n, delta_parts, weight, cols, x_norm, n, digits,
+                                           4 * n, exps, rows, rows, cols, eps)
 
 
 def linear_digits_parts(seq_len: int, in_dim: int, out_dim: int) -> int:
@@ -547,36 +556,38 @@ def linear_digits_parts(seq_len: int, in_dim: int, out_dim: int) -> int:
 
 
 def linear_digits_int8(ys, ws: list, digits, exps, seq_len: int, in_dim: int, residual: bool = False,
-                       parts: int = 1) -> None:
+                       parts: int = 1, x=None) -> None:
     """W8A32 projections of the same digit rows in one launch (up to 3 QuantWeights);
     with ``residual`` each is added to its y. ``parts`` > 1 cuts in_dim: each y holds that
-    many slices ``[parts, seq_len, out_dim]`` to be added (``add_rms_norm_digits``)."""
-    _call.qasr_linear_digits_int8_f32(ys, ws, digits, 4 * seq_len * in_dim, exps, seq_len, seq_len, in_dim,
-                                      int(residual), parts, parts * seq_len)
+    many slices ``[parts, seq_len, out_dim]`` to be added (``add_rms_norm_digits``). ``x``:
+    the rows' floats, for those marked wide (without it they give NaN)."""
+    _call.qasr_linear_digits_wide_int8_f32(ys, ws, digits, 4 * seq_len * in_dim, exps, seq_len, x, seq_len * in_dim,
+                                           seq_len, in_dim, int(residual), parts, parts * seq_len)
 
 
 def gate_up_swiglu_digits_int8(out, w: QuantWeight, digits, exps, seq_len: int, in_dim: int, intermediate: int,
-                               prefill: bool = False) -> None:
+                               prefill: bool = False, x=None) -> None:
     """The interleaved gate/up projection of digit rows with the decode loop's SwiGLU, or
-    swiglu_multiply's (``prefill``)."""
-    _call.qasr_gate_up_swiglu_digits_int8_f32(out, seq_len * intermediate, w.data, 2 * intermediate * in_dim, w.scales,
-                                              2 * intermediate, digits, 4 * seq_len * in_dim, exps, seq_len, seq_len,
-                                              in_dim, intermediate, int(prefill))
+    swiglu_multiply's (``prefill``); ``x`` as in ``linear_digits_int8``."""
+    _call.qasr_gate_up_swiglu_digits_wide_int8_f32(out, seq_len * intermediate, w.data, 2 * intermediate * in_dim,
+                                                   w.scales, 2 * intermediate, digits, 4 * seq_len * in_dim, exps,
+                                                   seq_len, x, seq_len * in_dim, seq_len, in_dim, intermediate,
+                                                   int(prefill))
 
 
 def qkv_heads_digits_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeight, wk: QuantWeight, wv: QuantWeight,
                           digits, exps, seq_len: int, in_dim: int, n_heads: int, n_kv_heads: int, head_dim: int,
-                          q_norm_w, k_norm_w, rope: "RopeCache", start_pos: int, eps: float) -> None:
-    """``qkv_heads_int8`` from digit rows."""
+                          q_norm_w, k_norm_w, rope: "RopeCache", start_pos: int, eps: float, x=None) -> None:
+    """``qkv_heads_int8`` from digit rows; ``x`` as in ``linear_digits_int8``."""
     qd, kv = n_heads * head_dim, n_kv_heads * head_dim
     if rope.head_dim != head_dim:
         raise ValueError("RopeCache head_dim does not match")
-    _call.qasr_qkv_heads_digits_int8_f32(q, seq_len * qd, k_cache, cache_rows * kv, v_cache, cache_rows * kv,
-                                         cache_rows, wq.data, qd * in_dim, wq.scales, qd, wk.data, kv * in_dim,
-                                         wk.scales, kv, wv.data, kv * in_dim, wv.scales, kv, digits,
-                                         4 * seq_len * in_dim, exps, seq_len, seq_len, in_dim, n_heads, n_kv_heads,
-                                         head_dim, q_norm_w, head_dim, k_norm_w, head_dim, rope.cos, 0, rope.sin, 0,
-                                         rope.cap, start_pos, eps)
+    _call.qasr_qkv_heads_digits_wide_int8_f32(q, seq_len * qd, k_cache, cache_rows * kv, v_cache, cache_rows * kv,
+                                              cache_rows, wq.data, qd * in_dim, wq.scales, qd, wk.data, kv * in_dim,
+                                              wk.scales, kv, wv.data, kv * in_dim, wv.scales, kv, digits,
+                                              4 * seq_len * in_dim, exps, seq_len, x, seq_len * in_dim, seq_len,
+                                              in_dim, n_heads, n_kv_heads, head_dim, q_norm_w, head_dim, k_norm_w,
+                                              head_dim, rope.cos, 0, rope.sin, 0, rope.cap, start_pos, eps)
 
 
 def qkv_heads_int8(q, k_cache, v_cache, cache_rows: int, wq: QuantWeight, wk: QuantWeight, wv: QuantWeight,

@@ -1,9 +1,11 @@
 """The digit-row projections (csrc/gemm_digits.hip): the digits themselves, and every
 tile and epilogue at its edges, against 64-bit evaluations.
 
-Bounds: a digit row is x to 2^-31 of its largest element, and the dot products are exact;
+Bounds: a digit row is x to 2^-30 of its largest element, and the dot products are exact;
 what is left are at most ten fp32 roundings of sums of the digits' size, so an output is
-within 10 * 2^-24 of sum |w| |x| * scale plus that fixed-point step."""
+within 10 * 2^-24 of sum |w| |x| * scale plus that fixed-point step, 2^-30 max |x| sum |w| *
+scale. Rows marked wide are sums of exact products in fp32, as the general W8A32 projection's
+are: its error against 64 bits, on the same inputs, is their yardstick."""
 from __future__ import annotations
 
 import numpy as np
@@ -35,7 +37,8 @@ def _product(x, w):
     q = w.data.view(w.out_dim, w.in_dim).double().cpu()
     s = w.scales.double().cpu()
     x = x.double().cpu()
-    return (x @ q.t()) * s, (x.abs() @ q.abs().t()) * s * (10 * 2.0 ** -24) + 1e-30
+    step = 2.0 ** -30 * x.abs().amax(-1, keepdim=True) * q.abs().sum(-1)
+    return (x @ q.t()) * s, ((x.abs() @ q.abs().t()) * (10 * 2.0 ** -24) + step) * s + 1e-30
 
 
 def _near(got, ref, bound):
@@ -193,6 +196,171 @@ def test_lm_head_rows_from_digits(dev, rows, K_, vocab):
     ref, bound = _product(x, w)
     _near(got, ref, bound if vocab > 1000 else 1e-5 * bound / (10 * 2.0 ** -24))
     assert torch.equal(idx.long(), got.argmax(-1))
+
+
+OUTLIERS = (7, 100, 200)  # columns whose weights are 0 in the tests of wide rows
+
+
+def _wide_case(T, K_, N, dev):
+    """Rows that range too far for the digits (one or three elements far above the rest) among
+    ordinary ones and ones just inside the line; the weights are 0 at those elements, so the
+    outputs are sums of the small ones. Last rows: an infinity and a NaN."""
+    x = torch.randn(T, K_, device=dev, generator=torch.Generator(device=dev).manual_seed(T + K_))
+    x[1::5, 7] = 1e4
+    x[2::5, 100] = -1e6
+    x[3::5, 7], x[3::5, 100], x[3::5, 200] = 1e5, 1e5, -1e5
+    x[4::5, 200] = 60.0  # at most 100 times the mean magnitude
+    x[T - 2, 17], x[T - 1, 18] = float("-inf"), float("nan")
+    w = _weight(N, K_, dev, N)
+    w.data.view(N, K_)[:, list(OUTLIERS)] = 0
+    mean = x.double().abs().mean(-1)
+    wide = ~((x.double().abs().amax(-1) <= 128 * mean) & mean.isfinite())
+    return x, w, wide
+
+
+def _digits_wide(x, dev):
+    from qwenasr_amd import kernels as K
+
+    rows, cols = x.shape
+    dg = torch.empty(4 * rows * cols, dtype=torch.int8, device=dev)
+    ex = torch.empty(rows, dtype=torch.int32, device=dev)
+    K.digit_rows(dg, ex, x.reshape(-1), rows, cols, wide=True)
+    return dg, ex
+
+
+def _error(got, ref):  # of each row, against 64 bits
+    return (got.double() - ref).norm(dim=-1) / ref.norm(dim=-1)
+
+
+# one shape per tile (32 x 32, 64 x 32, 128 x 32, 256 x 64), ragged in rows and tokens, and a long sum
+@pytest.mark.parametrize("T,K_,N", [(9, 512, 1028), (65, 1024, 4096), (70, 512, 33028), (300, 1024, 12292),
+                                    (12, 6144, 2048)])
+def test_wide_rows_keep_fp32_precision(dev, T, K_, N):
+    from qwenasr_amd import kernels as K
+
+    x, w, wide = _wide_case(T, K_, N, dev)
+    dg, ex = _digits_wide(x, dev)
+    assert ((ex == -0x40000001) == wide).all() and wide[1::5].all() and not wide[4:T - 2:5].any()
+    flat = x.reshape(-1)
+    y, old = (torch.full((T * N,), 9.0, device=dev) for _ in range(2))
+    K.linear_digits_int8([y], [w], dg, ex, T, K_, x=flat)
+    K.linear_nobias_int8(old, flat, w.data, w.scales, T, K_, N)
+    ref = (x.double() @ w.data.view(N, K_).double().t().contiguous()) * w.scales.double()
+    fin = slice(0, T - 2)
+    limit = 1.25 * _error(old.view(T, N)[fin], ref[fin])  # a quarter for another order of the sums
+    assert (_error(y.view(T, N)[fin], ref[fin]) <= limit).all()
+    for parts in (2, 3, 4):
+        if K_ % (256 * parts) == 0:
+            p = torch.full((parts * T * N,), 9.0, device=dev)
+            K.linear_digits_int8([p], [w], dg, ex, T, K_, parts=parts, x=flat)
+            assert (_error(p.view(parts, T, N).double().sum(0)[fin], ref[fin]) <= limit).all()
+    z = torch.ones(T * N, device=dev)
+    K.linear_digits_int8([z], [w], dg, ex, T, K_, residual=True, x=flat)
+    assert torch.equal(z.view(T, N)[fin], (y + 1.0).view(T, N)[fin])
+    # an infinity and a NaN travel as in fp32: NaN only where a weight of 0 meets the infinity
+    got = y.view(T, N)[T - 2:]
+    assert torch.equal(got.isnan(), ref[T - 2:].isnan()) and torch.equal(got[0].isinf(), ref[T - 2].isinf())
+    keep = ~got[0].isnan()
+    assert torch.equal(got[0][keep].double(), ref[T - 2][keep]) and got[1].isnan().all()
+    K.linear_digits_int8([y], [w], dg, ex, T, K_)  # without the floats a marked row gives NaN
+    assert torch.equal(y.view(T, N).isnan().all(-1), wide) and torch.equal(y.view(T, N).isnan().any(-1), wide)
+
+
+def test_wide_rows_in_the_other_epilogues(dev):
+    """gate/up + SwiGLU and q/k/v + heads, whose marked rows equal the plain projection's followed
+    by the separate launches (their tiles may add K in another number of parts)."""
+    from qwenasr_amd import kernels as K
+
+    T, H, inter, nq, nk, hd = 45, 1024, 3072, 16, 8, 128
+    x, w, _ = _wide_case(T, H, 2 * inter, dev)
+    x = x[:T - 2].contiguous()
+    T -= 2
+    flat = x.view(-1)
+    w.scales.mul_(2e-4)
+    dg, ex = _digits_wide(x, dev)
+    gu, out, ref = torch.empty(T * 2 * inter, device=dev), torch.empty(T * inter, device=dev), torch.empty(T * inter, device=dev)
+    K.linear_digits_int8([gu], [w], dg, ex, T, H, x=flat)
+    K.swiglu_multiply(ref, gu, T, inter)
+    K.gate_up_swiglu_digits_int8(out, w, dg, ex, T, H, inter, prefill=True, x=flat)
+    torch.testing.assert_close(out, ref, rtol=1e-6, atol=1e-6)
+    K.gate_up_swiglu_digits_int8(out, w, dg, ex, T, H, inter, x=flat)
+    g, u = gu.view(T, inter, 2).double().unbind(-1)
+    torch.testing.assert_close(out.view(T, inter).double(), g / (1 + (-g).exp()) * u, rtol=1e-6, atol=1e-6)
+    ws = [_weight(n * hd, H, dev, n + i) for i, n in enumerate((nq, nk, nk))]
+    for m in ws:
+        m.scales.mul_(1e-3)
+        m.data.view(-1, H)[:, list(OUTLIERS)] = 0
+    qw, kw = torch.rand(hd, device=dev) + 0.5, torch.rand(hd, device=dev) + 0.5
+    rope = K.RopeCache(dev)
+    rope.ensure(T, hd, 1e6)
+    q1, k1, v1 = (torch.empty(T * n * hd, device=dev) for n in (nq, nk, nk))
+    caches = [torch.full((T * nk * hd,), 5.0, device=dev) for _ in range(4)]
+    q2 = torch.empty_like(q1)
+    K.qkv_heads_digits_int8(q2, caches[2], caches[3], T, *ws, dg, ex, T, H, nq, nk, hd, qw, kw, rope, 0, 1e-6, flat)
+    K.linear_digits_int8([q1, k1, v1], ws, dg, ex, T, H, x=flat)
+    K.head_rms_norm_rope_kv(q1, k1, v1, qw, kw, rope, None, 0, T, nq, nk, hd, 1e-6, caches[0], caches[1], T)
+    for a, b in ((q1, q2), (caches[0], caches[2]), (caches[1], caches[3])):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
+def test_add_rms_norm_digits_marks_wide_rows(dev):
+    from qwenasr_amd import kernels as K
+
+    for rows, cols in ((7, 1024), (6, 8192)):
+        x = torch.randn(rows, cols, device=dev)
+        x[2, 5], x[4, 1], x[5, 9] = 1e6, float("inf"), 30.0
+        g = torch.rand(cols, device=dev) + 0.5
+        a, b, c = (x.reshape(-1).clone() for _ in range(3))
+        xn, own, plain = torch.empty_like(a), torch.full_like(a, 7.0), torch.empty_like(a)
+        dg, dg2 = (torch.empty(4 * rows * cols, dtype=torch.int8, device=dev) for _ in range(2))
+        ex, ex2, ex3 = (torch.empty(rows, dtype=torch.int32, device=dev) for _ in range(3))
+        K.add_rms_norm_digits(a, None, g, plain, dg, ex, rows, cols, 1e-6)
+        K.add_rms_norm_digits(b, None, g, xn, dg2, ex2, rows, cols, 1e-6, wide=True)
+        K.add_rms_norm_digits(c, None, g, own, dg2, ex3, rows, cols, 1e-6, wide=True, all_rows=False)
+        marked = [2, 4]
+        rest = [i for i in range(rows) if i not in marked]
+        assert (ex2[marked] == -0x40000001).all() and torch.equal(ex2, ex3) and torch.equal(ex[rest], ex2[rest])
+        assert torch.equal(dg.view(4, rows, cols)[:, rest], dg2.view(4, rows, cols)[:, rest])
+        torch.testing.assert_close(xn, plain, rtol=0, atol=0, equal_nan=True)
+        own = own.view(rows, cols)
+        torch.testing.assert_close(own[marked], plain.view(rows, cols)[marked], rtol=0, atol=0, equal_nan=True)
+        assert (own[rest] == 7.0).all()
+
+
+@pytest.mark.parametrize("outlier", [1e4, 1e6])
+def test_lm_head_rows_keep_fp32_precision_beside_an_outlier(dev, outlier):
+    """With a workspace (digit rows) the logits are no further from 64 bits than without."""
+    from qwenasr_amd import kernels as K
+
+    rows, K_, vocab = 9, 2048, 4000
+    x = torch.randn(rows, K_, device=dev, generator=torch.Generator(device=dev).manual_seed(5))
+    x[::2, 7] = outlier
+    w = _weight(vocab, K_, dev, 3)
+    w.data.view(vocab, K_)[:, 7] = 0
+    ref = (x.double() @ w.data.view(vocab, K_).double().t().contiguous()) * w.scales.double()
+    idx, errors = torch.empty(rows, dtype=torch.int32, device=dev), []
+    for ws in (torch.empty(1 << 20, dtype=torch.uint8, device=dev), None):
+        logits = torch.empty(rows * vocab, device=dev)
+        K.lm_head_int8_argmax(idx, logits, x.view(-1), w, rows, K_, vocab, ws)
+        errors.append(_error(logits.view(rows, vocab), ref))
+    assert (errors[0] <= 1.25 * errors[1]).all()
+
+
+@pytest.mark.parametrize("rows", [2, 7])
+def test_lm_head_row_with_an_infinity(dev, rows):
+    """2 to 7 rows: an infinity gives infinite logits and the first positive one wins, as in fp32."""
+    from qwenasr_amd import kernels as K
+
+    K_, vocab = 1024, 3000
+    x = torch.randn(rows, K_, device=dev)
+    x[1, 3] = float("inf")
+    w = _weight(vocab, K_, dev, 8)
+    col = w.data.view(vocab, K_)[:, 3]
+    col[col == 0] = -1
+    idx, logits = torch.empty(rows, dtype=torch.int32, device=dev), torch.empty(rows * vocab, device=dev)
+    K.lm_head_int8_argmax(idx, logits, x.view(-1), w, rows, K_, vocab, torch.empty(1 << 20, dtype=torch.uint8, device=dev))
+    assert torch.equal(logits.view(rows, vocab)[1], torch.where(col > 0, float("inf"), float("-inf")))
+    assert int(idx[1]) == int((col > 0).nonzero()[0])
 
 
 def test_parts_worth_taking(dev):
