@@ -606,7 +606,7 @@ int qasr_add_rms_norm_digits_wide_f32(float* x, const float* delta, size_t delta
  * that many parts and y holds their slices, [parts][seq][out_dim], to be added:
  * more workgroups for a small product; qasr_linear_digits_parts gives the
  * number worth taking. in_dim a multiple of 256, out_dims multiples of 4,
- * 16-byte aligned buffers. */
+ * 16-byte aligned buffers (scales of any alignment). */
 int qasr_linear_digits_int8_f32(size_t n_mats, float* const* ys, const int8_t* const* ws,
                                 const float* const* scales, const size_t* out_dims, const int8_t* digits,
                                 const int32_t* exps, size_t seq, size_t in_dim, size_t residual,

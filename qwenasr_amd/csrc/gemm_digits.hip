@@ -679,8 +679,9 @@ int digit_mat_checks(const float* y, const int8_t* w, const float* s, size_t N, 
   QASR_REQUIRE(y && w && s, std::string(what) + ": null pointer");
   size_t n;
   QASR_REQUIRE(N <= 0x3fffffffu && mul_ok(N, K, &n) && mul_ok(T, N, &n), std::string(what) + ": size too large");
-  if (N == 0 || N % 4 != 0 || !aligned16(y) || !aligned16(w) || !aligned16(s))
-    return fail(QASR_ERR_UNSUPPORTED, std::string(what) + ": out_dim must be a multiple of 4, buffers 16-byte aligned");
+  if (N == 0 || N % 4 != 0 || !aligned16(y) || !aligned16(w) || !aligned4(s))
+    return fail(QASR_ERR_UNSUPPORTED,
+                std::string(what) + ": out_dim must be a multiple of 4, outputs and weights 16-byte aligned");
   return QASR_OK;
 }
 

@@ -47,6 +47,18 @@ import torch
 from . import kernels as K
 
 
+def _aligned16(*tensors: torch.Tensor) -> bool:
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _digit_weights(w: dict) -> bool:
+    """Whether the digit-row launches take these layers' weights and norm gains: 16-byte
+    aligned, which views into a larger buffer need not be (the general projections take
+    any alignment)."""
+    return all(_aligned16(*(lw[n].data for n in ("wq", "wk", "wv", "wo", "gate_up", "down")),
+                          lw["input_norm"], lw["post_attn_norm"]) for lw in w["layers"])
+
+
 class DecoderInt8:
     def __init__(self, weights: dict, hidden: int, intermediate: int, n_layers: int, n_heads: int = 16,
                  n_kv_heads: int = 8, head_dim: int = 128, eps: float = 1e-6, theta: float = 1e6,
@@ -90,6 +102,8 @@ class DecoderInt8:
         self.attn_ws = K.attention_workspace(1, n_heads, head_dim, dev)
         self.lm_ws = K.lm_head_workspace(self.vocab, dev)
         self.scale = 1.0 / math.sqrt(head_dim)
+        self.digit_weights = _digit_weights(weights) and all(_aligned16(lw["q_norm"], lw["k_norm"])
+                                                             for lw in weights["layers"])
 
     def _ensure_prefill(self, T: int) -> None:
         if getattr(self, "_pcap", 0) >= T:
@@ -159,8 +173,8 @@ class DecoderInt8:
         fits = (self.hd == 128 and max(self.H, self.I, q_dim) <= 8192
                 and self.H % 256 == 0 and self.I % 256 == 0 and q_dim % 256 == 0)
         one_wave = self.H <= 1024 and (self.nq + 2 * self.nk) * ((T + 63) // 64) == 256
-        return (fits and self.fuse_prefill_heads is None and self.fuse_prefill_norms is None and T >= 5
-                and not one_wave)
+        return (fits and self.digit_weights and self.fuse_prefill_heads is None and self.fuse_prefill_norms is None
+                and T >= 5 and not one_wave)
 
     def _prefill_digits(self, T: int, start_pos: int) -> None:
         H, I, nq, nk, hd, eps = self.H, self.I, self.nq, self.nk, self.hd, self.eps
@@ -417,7 +431,10 @@ class DecoderInt8Batched:
         # 151 us, 64 streams 292 -> 279; 1.7B, 5 streams 603 -> 237, 64 streams 412 -> 370
         q_dim = n_heads * head_dim
         self.digits = (not w8a8 and B >= 2 and max(hidden, intermediate, q_dim) <= 8192
-                       and hidden % 256 == 0 and intermediate % 256 == 0 and q_dim % 256 == 0)
+                       and hidden % 256 == 0 and intermediate % 256 == 0 and q_dim % 256 == 0
+                       and _digit_weights(weights) and _aligned16(weights["norm"]))
+        self.lm_digits = (self.digits and self.vocab % 4 == 0 and self.vocab == self.lm.out_dim
+                          and _aligned16(self.lm.data))
         if self.digits:
             self.dg = torch.empty(4 * B * max(hidden, intermediate, q_dim), dtype=torch.int8, device=device)
             self.dg_exps = torch.empty(B, dtype=torch.int32, device=device)
@@ -509,7 +526,7 @@ class DecoderInt8Batched:
         if self.digits:
             K.add_rms_norm_digits(self.x, self.down, self.w["norm"], self.x_norm, self.dg, self.dg_exps, B, H, eps,
                                   self.down_parts, True)
-            if self.vocab % 4 == 0 and self.vocab == self.lm.out_dim:
+            if self.lm_digits:
                 K.linear_digits_int8([self.logits], [self.lm], self.dg, self.dg_exps, B, H, x=self.x_norm)
                 K.argmax_rows(self.tokens, self.logits, B, self.vocab)
             else:

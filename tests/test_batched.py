@@ -727,3 +727,27 @@ def test_batched_decode_attention_bad_position_and_graph_replay(dev, rows):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.isnan(), eager.isnan()) and torch.equal(out.nan_to_num(), eager.nan_to_num()), rep
+
+
+@pytest.mark.parametrize("B", [3, 9])
+def test_batched_decode_takes_weights_of_any_alignment(tmp_path, dev, B):
+    """The W8A32 step with weights and scales of any alignment (the general projections) gives
+    what aligned ones (digit rows) give."""
+    from qwenasr_amd.decoder import DecoderInt8Batched
+    from tests.test_decoder_step import _load, unaligned
+    from tests.test_oracle import small_decoder
+
+    H, I, L, rows, vocab = 1024, 3072, 2, 64, 1000
+    weights = _load(tmp_path, small_decoder(np.random.default_rng([57, B]), H, I, L, NQ, NK, HD, vocab), L, dev)
+    e, got = torch.randn(B * H, device=dev), []
+    for w in (weights, unaligned(weights)):
+        dec = DecoderInt8Batched(w, H, I, L, B, rows, device=dev)
+        assert dec.digits == (w is weights)
+        dec.positions.zero_()
+        for step in range(2):
+            dec.decode(e)
+            got.append((dec.x_norm.clone(), dec.logits.clone()))
+            dec.finish()
+    for a, b in zip(got[:2], got[2:]):
+        for x, y in zip(a, b):
+            torch.testing.assert_close(x, y, rtol=1e-4, atol=1e-4)

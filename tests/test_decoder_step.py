@@ -367,3 +367,43 @@ def test_graph_replays_equal_the_eager_calls(tmp_path, dev):
 
         check(d, prefill_at_0, ("px",), slice(0, T),
               f"prefill fuse_prefill_heads={fuse_heads} fuse_prefill_norms={fuse_norms}")
+
+
+def unaligned(weights, data=True, scales=True):
+    """The same weights as views into larger buffers, weights a byte and scales a float past
+    16-byte alignment: what a loader that maps one buffer hands over."""
+    from qwenasr_amd import kernels as K
+
+    def shift(t, by):
+        buf = torch.empty(t.numel() + by, dtype=t.dtype, device=t.device)
+        buf[by:] = t.reshape(-1)
+        return buf[by:]
+
+    def quant(w):
+        return K.QuantWeight(shift(w.data, 1) if data else w.data, shift(w.scales, 1) if scales else w.scales,
+                             w.out_dim, w.in_dim)
+
+    return {**{k: quant(v) if isinstance(v, K.QuantWeight) else v for k, v in weights.items()},
+            "layers": [{k: quant(v) if isinstance(v, K.QuantWeight) else v for k, v in lw.items()}
+                       for lw in weights["layers"]]}
+
+
+@pytest.mark.parametrize("T,data", [(5, True), (7, True), (7, False), (37, False)])
+def test_prefill_takes_weights_of_any_alignment(tmp_path, dev, T, data):
+    """5 to 7 tokens with weights and scales of any alignment, longer prefills with such scales
+    (37 tokens: the q/k/v launch is a plain GEMM there) give what aligned ones give."""
+    from qwenasr_amd.decoder import DecoderInt8
+
+    H, I, L, nq, nk, hd, vocab = 1024, 3072, 2, 16, 8, 128, 100
+    r = np.random.default_rng([40, T])
+    weights = _load(tmp_path, small_decoder(r, H, I, L, nq, nk, hd, vocab), L, dev)
+    e = torch.randn(T * H, device=dev)
+    got = []
+    for w in (weights, unaligned(weights, data)):
+        dec = DecoderInt8(w, H, I, L, nq, nk, hd, max_seq=64, device=dev)
+        dec.prepare_prefill(0, T)
+        dec.prefill(e, T, 0)
+        got.append((dec.px[:T * H].clone(), dec.kv.k.clone(), dec.kv.v.clone()))
+        assert dec.prefill_digits(T) == (w is weights or not data)
+    for a, b in zip(*got):
+        torch.testing.assert_close(a, b, rtol=TOL, atol=TOL)
