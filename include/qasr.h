@@ -555,9 +555,8 @@ int qasr_decode_attention_f32(float* out, float* q, const float* k, const float*
 /* qasr_decode_attention_f32 followed by the o projection of its row
  * (qasr_linear_nobias_int8_f32: y[out_dim] from w [out_dim][n_heads *
  * head_dim], decoder.rs:906-907), bit for bit. Up to 512 cached keys of heads of
- * 128 (n_heads * 128 = 1024 or 2048) the projection merges the attention's key
- * splits itself and `out` is not written: treat it as scratch. w 16-byte
- * aligned. */
+ * 128 (n_heads * 128 = 1024 or 2048, w 16-byte aligned) the projection merges the
+ * attention's key splits itself and `out` is not written: treat it as scratch. */
 int qasr_decode_attention_linear_int8_f32(float* y, float* out, float* q, const float* k, const float* v,
                                           const float* q_norm_w, const float* k_norm_w,
                                           const float* cos_tab, const float* sin_tab, size_t table_rows,

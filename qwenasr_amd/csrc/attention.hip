@@ -1251,7 +1251,8 @@ static int decode_attention(float* out, float* q, const float* k, const float* v
     // every one of its 256 workgroups 8 KB of reads a split (all 16 heads), the
     // launch it replaces 2.7 us and as much again on the host.
     const size_t q_dim = n_heads * head_dim;
-    const bool fold = lin && sp.nsplit <= kMergeSplits && head_dim == 128 && (q_dim == 1024 || q_dim == 2048);
+    const bool fold = lin && sp.nsplit <= kMergeSplits && head_dim == 128 && (q_dim == 1024 || q_dim == 2048) &&
+                      aligned16(lin->w);
 #define QASR_PRE(HD, GG)                                                                         \
   if (head_dim == HD && G == GG) {                                                               \
     launch_attention_split<HD, GG>(out, q, k_cache, v_cache, 1, sk, nk, scale, qo, sp.nsplit,    \
@@ -1305,8 +1306,6 @@ extern "C" int qasr_decode_attention_linear_int8_f32(float* y, float* out, float
                    mul_ok(out_dim, n_heads * head_dim, &n),
                "decode_attention_linear: size too large");
   const DecodeLinear lin{y, w, scales, out_dim};
-  if (!aligned16(w))  // the unaligned projection's own kernel
-    return fail(QASR_ERR_UNSUPPORTED, "decode_attention_linear: w must be 16-byte aligned");
   return decode_attention(out, q, k, v, q_norm_w, k_norm_w, cos_tab, sin_tab, table_rows, pos, n_heads, n_kv_heads,
                           head_dim, eps, scale, k_cache, v_cache, cache_rows, workspace, workspace_floats, &lin,
                           stream);

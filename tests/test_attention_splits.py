@@ -160,3 +160,28 @@ def test_decode_attention_linear_equals_the_two_calls(dev, pos, nq, nk, hd, out_
         got.append((y, *caches))
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pos", [0, 70, 511, 600])
+def test_decode_attention_linear_takes_weights_of_any_alignment(dev, pos):
+    """The o projection's weights and scales as views off 16-byte alignment: decode_attention
+    followed by linear_nobias_int8, bit for bit; the decode step runs with them."""
+    from qwenasr_amd import kernels as K
+
+    nq, nk, hd, H, rows = 16, 8, 128, 1024, 640
+    g = torch.Generator(device=dev).manual_seed(pos)
+    r = lambda n: torch.randn(n, generator=g, device=dev)  # noqa: E731
+    q, k, v, qw, kw = r(nq * hd), r(nk * hd), r(nk * hd), r(hd), r(hd)
+    kc, vc = r(rows * nk * hd), r(rows * nk * hd)
+    rope = K.RopeCache(dev)
+    rope.ensure(rows, hd, 1e6)
+    ws = K.attention_workspace(1, nq, hd, dev)
+    data = torch.randint(-128, 128, (H * nq * hd + 1,), generator=g, device=dev, dtype=torch.int32).to(torch.int8)[1:]
+    w = K.QuantWeight(data, (r(H + 1).abs() + 0.1)[1:], H, nq * hd)
+    a, b, y, z = (torch.full((n,), 9.0, device=dev) for n in (nq * hd, nq * hd, H, H))
+    K.decode_attention(a, q.clone(), k, v, qw, kw, rope, pos, nq, nk, hd, 1e-6, 0.1, kc.clone(), vc.clone(), rows, ws)
+    K.linear_nobias_int8(y, a, w.data, w.scales, 1, nq * hd, H)
+    K.decode_attention_linear_int8(z, b, q.clone(), k, v, qw, kw, rope, pos, nq, nk, hd, 1e-6, 0.1, kc, vc, rows, ws,
+                                   w, H)
+    assert torch.equal(y, z)
