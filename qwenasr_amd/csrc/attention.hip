@@ -1257,9 +1257,9 @@ static int decode_attention(float* out, float* q, const float* k, const float* v
   if (head_dim == HD && G == GG) {                                                               \
     launch_attention_split<HD, GG>(out, q, k_cache, v_cache, 1, sk, nk, scale, qo, sp.nsplit,    \
                                    sp.keys_per_split, sp.ws_o, sp.ws_ml, st, &pre, !fold);       \
-    if (fold)                                                                                    \
-      launch_w8a32_merge(lin->y, sp.ws_o, sp.ws_ml, sp.nsplit, q_dim, lin->w, lin->scales,       \
-                         lin->out_dim, st);                                                      \
+    if (fold && !launch_w8a32_merge(lin->y, sp.ws_o, sp.ws_ml, sp.nsplit, q_dim, lin->w,         \
+                                    lin->scales, lin->out_dim, st))                              \
+      return fail(QASR_ERR_UNSUPPORTED, "decode_attention_linear: no merging kernel");           \
     const int rc = launch_status("decode_attention");                                            \
     if (rc != QASR_OK || !lin || fold) return rc;                                                \
     return qasr_linear_nobias_int8_f32(lin->y, out, lin->w, lin->scales, 1, q_dim, lin->out_dim, \

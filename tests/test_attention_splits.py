@@ -185,3 +185,11 @@ def test_decode_attention_linear_takes_weights_of_any_alignment(dev, pos):
     K.decode_attention_linear_int8(z, b, q.clone(), k, v, qw, kw, rope, pos, nq, nk, hd, 1e-6, 0.1, kc, vc, rows, ws,
                                    w, H)
     assert torch.equal(y, z)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nq,out_dim", [(8, 500), (8, 2500), (8, 8200), (16, 300), (16, 4100)])
+def test_every_row_count_of_the_projection_has_a_merging_kernel(dev, nq, out_dim):
+    """1, 2, 4 and 8 rows a wave at 1024 inputs, 1, 2 and 4 at 2048: the merging launch runs for
+    each (a size without one raises instead of leaving y as it was)."""
+    test_decode_attention_linear_equals_the_two_calls(dev, 130, nq, 8, 128, out_dim)
