@@ -721,17 +721,20 @@ int qasr_argmax_rows_f32(int32_t* idx, const float* x, size_t rows, size_t cols,
  * qasr_lm_head_argmax_workspace_bytes(vocab) bytes, the matvec reduces its
  * rows to per-workgroup candidates there and one small kernel merges them
  * (no second pass over the logits). With rows > 1 and room for their digit rows
- * (rows * (4 * in_dim + 4) bytes, 16-byte aligned; in_dim a multiple of 256 up
- * to 8192) the logits come from qasr_linear_digits_wide_int8_f32.
- * Otherwise the logits are scanned after the matvec. Same idx for the same logits. Calls that share a
- * workspace must be ordered on one stream. */
+ * (qasr_lm_head_argmax_rows_workspace_bytes(vocab, rows, in_dim) bytes, 16-byte
+ * aligned; in_dim a multiple of 256 up to 8192) the logits come from
+ * qasr_linear_digits_wide_int8_f32. Otherwise the logits are scanned after the
+ * matvec. Same idx for the same logits. Calls that share a workspace must be
+ * ordered on one stream. */
 int qasr_lm_head_int8_argmax_f32(int32_t* idx, float* logits, const float* x,
                                  const int8_t* w, const float* scales, size_t rows,
                                  size_t in_dim, size_t vocab, void* workspace,
                                  size_t workspace_bytes, void* stream);
 
-/* Workspace bytes qasr_lm_head_int8_argmax_f32 can use for this vocab. */
+/* Workspace bytes qasr_lm_head_int8_argmax_f32 can use for one row of this vocab,
+ * and for any number of rows up to `rows`. */
 size_t qasr_lm_head_argmax_workspace_bytes(size_t vocab);
+size_t qasr_lm_head_argmax_rows_workspace_bytes(size_t vocab, size_t rows, size_t in_dim);
 
 /* qasr_lm_head_int8_argmax_f32 without a workspace and without allocating:
  * no counterpart in the reference. For callers that cannot allocate device
@@ -739,7 +742,8 @@ size_t qasr_lm_head_argmax_workspace_bytes(size_t vocab);
  * The one-row candidates go to a 512 KiB array the library holds on each GPU
  * it runs on until the process ends (looked up once per device on the first
  * call there; nothing is allocated, no call here allocates). Same results as
- * qasr_lm_head_int8_argmax_f32 with a workspace for one row, without one for several. One row needs in_dim
+ * qasr_lm_head_int8_argmax_f32 with a workspace for one row, without one for
+ * several. One row needs in_dim
  * 1024..8192 in steps of 1024 and 16-byte aligned x and w (UNSUPPORTED
  * otherwise); vocab at most QASR_LM_HEAD_NOALLOC_MAX_VOCAB (INVALID_ARG
  * otherwise). rows > 1 writes the logits and scans them, as the workspace

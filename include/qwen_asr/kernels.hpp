@@ -700,8 +700,8 @@ inline void argmax_rows(DevSlice<int32_t> idx, CF x, size_t rows, size_t cols) {
   detail::check(qasr_argmax_rows_f32(idx.ptr, x.ptr, rows, cols, detail::st()), "argmax_rows");
 }
 
-inline size_t lm_head_workspace_bytes(size_t vocab) {
-  return qasr_lm_head_argmax_workspace_bytes(vocab);
+inline size_t lm_head_workspace_bytes(size_t vocab, size_t rows = 1, size_t in_dim = 0) {
+  return qasr_lm_head_argmax_rows_workspace_bytes(vocab, rows, in_dim);
 }
 
 inline void lm_head_int8_argmax(DevSlice<int32_t> idx, F logits, CF x, DevSlice<const int8_t> w,

@@ -119,6 +119,7 @@ SIZE_QUERIES = {
     "qasr_batched_decode_attention_split_workspace_floats": [ctypes.c_size_t] * 4,
     "qasr_linear_digits_parts": [ctypes.c_size_t] * 3,
     "qasr_lm_head_argmax_workspace_bytes": [ctypes.c_size_t],
+    "qasr_lm_head_argmax_rows_workspace_bytes": [ctypes.c_size_t] * 3,
 }
 
 _LIB = None

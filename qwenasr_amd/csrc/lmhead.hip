@@ -25,6 +25,7 @@ namespace {
 
 constexpr int kArgmaxBlock = 1024;
 constexpr int kArgmaxLoads = 8;  // loads in flight per thread
+constexpr size_t kLmDigitPlanes = 4;  // of qasr_digit_rows_f32
 
 template <int M>
 QASR_DEV void wave_argmax(float& bv, int& bi) {
@@ -147,6 +148,19 @@ extern "C" size_t qasr_lm_head_argmax_workspace_bytes(size_t vocab) {
   return lm_head_partials_max(vocab) * sizeof(float2);
 }
 
+// Bytes of the digit rows of several rows, 0 where the lm_head does not run from them.
+static size_t lm_head_digit_bytes(size_t rows, size_t in_dim, size_t vocab) {
+  if (rows < 2 || rows > 65536 || in_dim == 0 || in_dim > 8192 || in_dim % 256 != 0 || vocab % 4 != 0 ||
+      vocab > 0x3fffffffu)
+    return 0;
+  return rows * (kLmDigitPlanes * in_dim + sizeof(int32_t));
+}
+
+extern "C" size_t qasr_lm_head_argmax_rows_workspace_bytes(size_t vocab, size_t rows, size_t in_dim) {
+  const size_t one = qasr_lm_head_argmax_workspace_bytes(vocab), digits = lm_head_digit_bytes(rows, in_dim, vocab);
+  return one > digits ? one : digits;
+}
+
 extern "C" int qasr_lm_head_int8_argmax_f32(int32_t* idx, float* logits, const float* x,
                                             const int8_t* w, const float* scales, size_t rows,
                                             size_t in_dim, size_t vocab, void* workspace,
@@ -169,17 +183,17 @@ extern "C" int qasr_lm_head_int8_argmax_f32(int32_t* idx, float* logits, const f
       return launch_status("lm_head_int8_argmax");
     }
   }
-  // Several rows whose digit rows fit the workspace (32 rows of 2048 in that of a
-  // 151936 vocabulary): exact int8 products on the matrix cores instead of a
-  // conversion of every weight per token tile, or of a pass over the weights
-  // per token below 8 rows (151936 x 2048, one MI355X: 2 rows 159 -> 79 us, 7 rows
-  // 526 -> 79, 32 rows 158 -> 86; x 1024, 32 rows 87 -> 50).
-  const size_t plane = rows * in_dim;  // used once both are bounded
-  if (rows > 1 && rows <= 65536 && workspace && in_dim > 0 && in_dim <= 8192 && in_dim % 256 == 0 && vocab % 4 == 0 &&
-      vocab <= 0x3fffffffu && 4 * plane + rows * sizeof(int32_t) <= workspace_bytes && aligned16(workspace) &&
-      aligned16(x) && aligned16(w) && aligned16(scales) && aligned16(logits)) {
+  // Several rows whose digit rows fit the workspace (the one-row workspace of a
+  // 151936 vocabulary holds 37 rows of 2048; a caller asks for its own rows'):
+  // exact int8 products on the matrix cores instead of a conversion of every
+  // weight per token tile, or of a pass over the weights per token below 8 rows
+  // (151936 x 2048, one MI355X: 2 rows 159 -> 79 us, 7 rows 526 -> 79, 32 rows
+  // 158 -> 86; x 1024, 32 rows 87 -> 50).
+  const size_t digit_bytes = lm_head_digit_bytes(rows, in_dim, vocab);
+  if (digit_bytes && workspace && digit_bytes <= workspace_bytes && aligned16(workspace) && aligned16(x) &&
+      aligned16(w) && aligned4(scales) && aligned16(logits)) {
     int8_t* digits = static_cast<int8_t*>(workspace);
-    int32_t* exps = reinterpret_cast<int32_t*>(digits + 4 * plane);
+    int32_t* exps = reinterpret_cast<int32_t*>(digits + kLmDigitPlanes * rows * in_dim);
     int rc = qasr_digit_rows_wide_f32(digits, exps, x, rows, in_dim, stream);
     if (rc == QASR_OK)
       rc = qasr_linear_digits_wide_int8_f32(1, &logits, &w, &scales, &vocab, digits, exps, x, rows, in_dim, 0, 1,

@@ -280,9 +280,11 @@ def argmax_rows(idx, x, rows: int, cols: int) -> None:
     _call.qasr_argmax_rows_f32(idx, rows, x, rows * cols, rows, cols)
 
 
-def lm_head_workspace(vocab: int, device="cuda") -> torch.Tensor:
-    """Workspace for the lm_head argmax (bytes as a uint8 tensor)."""
-    n = _lib.lib().qasr_lm_head_argmax_workspace_bytes(vocab)
+def lm_head_workspace(vocab: int, device="cuda", rows: int = 1, in_dim: int = 0) -> torch.Tensor:
+    """Workspace for the lm_head argmax of up to ``rows`` rows of ``in_dim`` (bytes as a uint8
+    tensor). One made for fewer rows is taken too; rows that do not fit it then run on the
+    general projection."""
+    n = _lib.lib().qasr_lm_head_argmax_rows_workspace_bytes(vocab, rows, in_dim)
     return torch.empty(max(n, 8), dtype=torch.uint8, device=device)
 
 

@@ -443,3 +443,15 @@ def test_probe_read_validation():
     assert call(mode=0, buf_bytes=8 * 512 * kb - 1) == inv
     assert call(priv=4096) == inv
     assert b"probe_read" in so.qasr_last_error()
+
+
+def test_lm_head_workspace_sizes():
+    one = _lib.lib().qasr_lm_head_argmax_workspace_bytes
+    rows = _lib.lib().qasr_lm_head_argmax_rows_workspace_bytes
+    assert rows(151936, 1, 2048) == rows(151936, 37, 2048) == one(151936)  # 37 rows' digits fit it
+    assert rows(151936, 38, 2048) == 38 * (4 * 2048 + 4)
+    assert rows(1000, 65536, 8192) == 65536 * (4 * 8192 + 4)
+    # sizes that do not run from digit rows, and ones that would overflow
+    for vocab, n, k in ((1000, 65537, 1024), (1002, 40, 1024), (1000, 40, 1000), (1000, 40, 8448), (1000, 40, 0),
+                        (1000, 1 << 62, 1 << 62), (1 << 40, 40, 1024)):
+        assert rows(vocab, n, k) == one(vocab)

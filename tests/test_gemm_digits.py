@@ -363,6 +363,29 @@ def test_lm_head_row_with_an_infinity(dev, rows):
     assert int(idx[1]) == int((col > 0).nonzero()[0])
 
 
+@pytest.mark.parametrize("rows", [7, 8, 38])
+def test_lm_head_workspace_for_rows(dev, rows):
+    """A workspace asked for with the rows holds their digits (38 rows of 2048 do not fit the
+    one-row workspace of this vocabulary): the digit projection's logits, bit for bit; one
+    made for a row less gives the general projection's."""
+    from qwenasr_amd import kernels as K
+
+    K_, vocab = 2048, 4000
+    x = torch.randn(rows, K_, device=dev)
+    w = _weight(vocab, K_, dev, rows)
+    dg, ex = _digits_wide(x, dev)
+    digits, plain, logits = (torch.empty(rows * vocab, device=dev) for _ in range(3))
+    idx = torch.empty(rows, dtype=torch.int32, device=dev)
+    K.linear_digits_int8([digits], [w], dg, ex, rows, K_, x=x.view(-1))
+    K.linear_nobias_int8(plain, x.view(-1), w.data, w.scales, rows, K_, vocab)
+    assert not torch.equal(digits, plain)
+    for have, want in ((rows, digits), (rows - 1, plain)):
+        ws = K.lm_head_workspace(vocab, dev, have, K_)
+        K.lm_head_int8_argmax(idx, logits, x.view(-1), w, rows, K_, vocab, ws)
+        assert torch.equal(logits, want)
+        assert torch.equal(idx.long(), logits.view(rows, vocab).argmax(-1))
+
+
 def test_parts_worth_taking(dev):
     from qwenasr_amd import kernels as K
 
