@@ -148,7 +148,10 @@ class DecoderInt8:
         self._ensure_prefill(T)
 
     def prefill_heads_fused(self, T: int) -> bool:
-        """Whether a prefill of T tokens runs q/k/v with the heads in one launch."""
+        """Whether a prefill of T tokens runs q/k/v with the heads in one launch (from
+        digit rows: always)."""
+        if self.prefill_digits(T):
+            return True
         fits = self.hd == 128 and self.H % 64 == 0 and T >= 8
         if self.fuse_prefill_heads is None:
             return fits and (self.nq + 2 * self.nk) * ((T + 63) // 64) >= 256
@@ -157,7 +160,9 @@ class DecoderInt8:
     def prefill_norms_folded(self, T: int) -> bool:
         """Whether a prefill of T tokens folds the residual adds into the o / down
         GEMMs and the RMSNorms into the following GEMMs (the GEMM path: T >= 8,
-        every in_dim a multiple of 64)."""
+        every in_dim a multiple of 64). From digit rows the norms are launches of their own."""
+        if self.prefill_digits(T):
+            return False
         fits = T >= 8 and self.H % 64 == 0 and (self.nq * self.hd) % 64 == 0 and self.I % 64 == 0
         return fits and self.fuse_prefill_norms is not False
 
@@ -165,10 +170,14 @@ class DecoderInt8:
         """Whether a prefill of T tokens runs its projections from digit rows (exact
         integer products on the int8 matrix cores; ``K.linear_digits_int8``), the default
         wherever it is the faster one: from 5 tokens on, except where a hidden size of
-        1024 meets a q/k/v grid of exactly one workgroup per CU (449 to 512 tokens),
-        for which the folded bf16-split launches are tuned (two 0.6B layers, 512 tokens
-        213 us against 224; 430 tokens 240 against 217, 64 tokens 143 against 123, 2
-        tokens 89 against 99; 1.7B, 1473 tokens 1377 against 1099)."""
+        1024 meets a q/k/v grid of exactly one workgroup per CU (449 to 512 tokens with
+        16 and 8 heads), for which the folded bf16-split launches are tuned; their next
+        full grid (961 to 1024 tokens) has lost again. Two layers, split against digit
+        rows (us): 0.6B 4 tokens 107 and 99, 5 114 and 99, 64 143 and 122, 430 242 and
+        219, 448 243 and 221, 449 211 and 228, 480 212 and 228, 512 214 and 222, 513 299
+        and 273, 961 450 and 422, 1024 462 and 429; 1.7B 2 tokens 120 and 128, 5 194 and
+        128, 449 467 and 384, 512 472 and 397. The line at 5 is on the safe side: the two
+        cross between 3 and 4 tokens (0.6B 3 tokens 95 and 99; 1.7B 3 146 and 127)."""
         q_dim = self.nq * self.hd
         fits = (self.hd == 128 and max(self.H, self.I, q_dim) <= 8192
                 and self.H % 256 == 0 and self.I % 256 == 0 and q_dim % 256 == 0)
@@ -202,14 +211,14 @@ class DecoderInt8:
         H, I, nq, nk, hd, eps = self.H, self.I, self.nq, self.nk, self.hd, self.eps
         q_dim = nq * hd
         total = start_pos + T
-        fused_heads = self.prefill_heads_fused(T)
-        fold = self.prefill_norms_folded(T)
         x = self.px
         x[:T * H].copy_(embeds[:T * H])
         if self.prefill_digits(T):
             self._prefill_digits(T, start_pos)
             self.kv.len = total
             return
+        fused_heads = self.prefill_heads_fused(T)
+        fold = self.prefill_norms_folded(T)
         layers = self.w["layers"]
         k_blocks, v_blocks = self.kv.layer_blocks()
         for l, lw in enumerate(layers):

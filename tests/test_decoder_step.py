@@ -407,3 +407,32 @@ def test_prefill_takes_weights_of_any_alignment(tmp_path, dev, T, data):
         assert dec.prefill_digits(T) == (w is weights or not data)
     for a, b in zip(*got):
         torch.testing.assert_close(a, b, rtol=TOL, atol=TOL)
+
+
+def test_prefill_predicates_tell_the_path(tmp_path, dev, monkeypatch):
+    """prefill_digits, prefill_heads_fused and prefill_norms_folded against the calls that a
+    prefill makes: digit rows from 5 tokens on except in 449 to 512 (hidden 1024), and the
+    forms that the arguments ask for."""
+    from qwenasr_amd import kernels as K
+    from qwenasr_amd.decoder import DecoderInt8
+
+    H, I, L, nq, nk, hd, vocab = 1024, 3072, 1, 16, 8, 128, 100
+    weights = _load(tmp_path, small_decoder(np.random.default_rng(41), H, I, L, nq, nk, hd, vocab), L, dev)
+    made = set()
+    for name in ("qkv_heads_digits_int8", "qkv_heads_int8", "rms_norm_qkv_heads_int8", "linear_int8_residual",
+                 "linear_digits_int8"):
+        monkeypatch.setattr(K, name, lambda *a, _n=name, _f=getattr(K, name), **k: (made.add(_n), _f(*a, **k))[1])
+    for heads, norms, sizes in ((None, None, (1, 4, 5, 37, 448, 449, 512, 513)), (True, False, (37, 449)),
+                                (False, True, (37,)), (None, True, (37, 512))):
+        dec = DecoderInt8(weights, H, I, L, nq, nk, hd, max_seq=520, device=dev, fuse_prefill_heads=heads,
+                          fuse_prefill_norms=norms)
+        for T in sizes:
+            made.clear()
+            dec.kv.len = 0
+            dec.prepare_prefill(0, T)
+            dec.prefill(torch.zeros(T * H, device=dev), T, 0)
+            assert dec.prefill_digits(T) == ("linear_digits_int8" in made), T
+            assert dec.prefill_heads_fused(T) == any("heads" in n for n in made), (T, made)
+            assert dec.prefill_norms_folded(T) == ("linear_int8_residual" in made), (T, made)
+            if heads is None and norms is None:
+                assert dec.prefill_digits(T) == (T >= 5 and not 449 <= T <= 512), T
