@@ -4,7 +4,8 @@ Compiles every ``csrc/*.hip`` with hipcc for gfx950 and produces, in-tree:
 
 * ``qwenasr_amd/libqasr_hip.so`` -- shared library the Python and C++ hosts load;
 * ``qwenasr_amd/_binding.so``     -- the Python extension through which ``kernels.py``
-  calls it (host code only, against torch's headers);
+  calls it (host code only, against torch's and Python's headers; without these the
+  libraries are built alone, and a line says so);
 * ``qwenasr_amd/libqasr_hip.a``  -- static archive for a host that links it
   statically (a Rust ``build.rs`` would add ``cargo:rustc-link-lib=static=qasr_hip``
   plus ``amdhip64``).
@@ -63,18 +64,55 @@ def _run(cmd: list[str]) -> None:
         raise RuntimeError(f"command failed ({r.returncode}): {' '.join(cmd)}")
 
 
+def _binding_includes() -> list[Path]:
+    import torch
+
+    t = Path(torch.__file__).resolve().parent
+    return [t / "include", t / "include" / "torch" / "csrc" / "api" / "include", ROCM / "include",
+            Path(sysconfig.get_paths()["include"])]
+
+
+def binding_missing() -> str:
+    """What keeps the Python binding from being built here ('' for nothing): it needs torch
+    and its C++ headers, Python's headers and g++, which a C or Rust host has no use for."""
+    try:
+        incs = _binding_includes()
+    except ImportError as e:
+        return f"torch cannot be imported ({e})"
+    for header in ("torch/csrc/autograd/python_variable.h", "c10/hip/HIPStream.h", "Python.h"):
+        if not any((i / header).exists() for i in incs):
+            return f"no {header}"
+    return "" if shutil.which("g++") else "no g++"
+
+
 def binding_command(out: Path) -> list[str]:
     """The compile line of the Python binding: plain host C++ that calls the
     entry points by address, so it links torch but not the kernel library."""
     import torch
 
-    t = Path(torch.__file__).resolve().parent
-    incs = [t / "include", t / "include" / "torch" / "csrc" / "api" / "include", ROCM / "include",
-            Path(sysconfig.get_paths()["include"])]
+    lib = Path(torch.__file__).resolve().parent / "lib"
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-            f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *[f"-I{i}" for i in incs], str(CSRC / "binding.cpp"), "-o", str(out),
-            f"-L{t / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+            f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *[f"-I{i}" for i in _binding_includes()], str(CSRC / "binding.cpp"),
+            "-o", str(out), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+
+
+def build_binding(verbose: bool = False) -> Path | None:
+    """Builds ``_binding.so``. Where its prerequisites are missing, says so and leaves none
+    (an old one may not match the library): the libraries serve C and Rust hosts all the
+    same, and ``kernels.py`` names the reason on its first call."""
+    missing = binding_missing()
+    if missing:
+        print(f"the Python binding is not built: {missing}", file=sys.stderr, flush=True)
+        BINDING.unlink(missing_ok=True)
+        return None
+    tmp = BUILD / "_binding.so"
+    cmd = binding_command(tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    _run(cmd)
+    os.replace(tmp, BINDING)
+    return BINDING
 
 
 def sources() -> list[Path]:
@@ -82,7 +120,8 @@ def sources() -> list[Path]:
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile all kernels and link the shared and static libraries."""
+    """Compile all kernels and link the shared and static libraries; then the Python
+    binding, where it can be built."""
     hipcc = _hipcc()
     BUILD.mkdir(exist_ok=True)
     srcs = sources()
@@ -95,18 +134,10 @@ def build(verbose: bool = False) -> Path:
             print(" ".join(cmd), flush=True)
         _run(cmd)
 
-    binding = BUILD / "_binding.so"
-
-    def compile_binding(_):
-        _run(binding_command(binding))
-
     workers = min(len(srcs), max(1, (os.cpu_count() or 4)))
     with ThreadPoolExecutor(max_workers=workers) as ex:
-        jobs = [ex.submit(compile_binding, None)]
-        jobs += [ex.submit(compile_one, pair) for pair in zip(srcs, objs)]
-        for j in jobs:
-            j.result()
-    os.replace(binding, BINDING)
+        binding = ex.submit(build_binding, verbose)  # beside the kernels; its outcome is looked at last
+        list(ex.map(compile_one, zip(srcs, objs)))
 
     tmp_so = SO.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp_so),
@@ -117,6 +148,7 @@ def build(verbose: bool = False) -> Path:
         ARCHIVE.unlink()
     _run(["ar", "rcs", str(ARCHIVE), *map(str, objs)])
     build_cpp_tests(hipcc, verbose)
+    binding.result()
     return SO
 
 

@@ -30,6 +30,31 @@ def test_cpu_tensors_and_wrong_objects_are_refused():
         K._call.qasr_add_inplace_f32()
 
 
+def test_a_host_without_the_headers_gets_the_libraries(monkeypatch, tmp_path, capsys):
+    """Without torch, its headers, Python's or g++ the build leaves the binding out and says
+    why; with them a failing compile is still an error."""
+    import sys
+
+    from qwenasr_amd import build
+
+    assert build.binding_missing() == ""
+    so = tmp_path / "_binding.so"
+    monkeypatch.setattr(build, "BINDING", so)
+    monkeypatch.setattr(build, "BUILD", tmp_path)
+    for change, text in ((lambda m: m.setitem(sys.modules, "torch", None), "torch cannot be imported"),
+                         (lambda m: m.setattr(build, "_binding_includes", lambda: [tmp_path]), "no torch/csrc"),
+                         (lambda m: m.setattr(build.shutil, "which", lambda _: None), "no g++")):
+        so.write_bytes(b"old")
+        with monkeypatch.context() as m:
+            change(m)
+            assert build.build_binding() is None
+        assert not so.exists() and "not built: " + text in capsys.readouterr().err
+    with monkeypatch.context() as m:
+        m.setattr(build, "CSRC", tmp_path)  # no source there
+        with pytest.raises(RuntimeError, match="command failed"):
+            build.build_binding()
+
+
 @pytest.mark.gpu
 def test_checks_on_device_tensors(dev):
     x, w = torch.ones(64, device=dev), torch.ones(16, device=dev)
