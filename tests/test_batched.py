@@ -217,10 +217,9 @@ def test_batched_decode_step_matches_the_oracle_per_stream(tmp_path, dev, H, I, 
     """DecoderInt8Batched (B streams, each at its own position over its own
     cache) against the oracle's decode step (decoder.rs:848-965) run stream
     by stream: final hidden state, logits, the new K/V rows of every layer and
-    the token, over two consecutive steps. B = 9 takes the matrix-core paths
-    (8+ rows), B = 3 the per-row ones; the attention with its keys cut into
-    chunks (the small-batch default) and walked whole (the large-batch one),
-    both in longest-first order. Tolerance as for the single-stream decode
+    the token, over two consecutive steps. The projections run from digit rows;
+    the attention with its keys cut into chunks (the small-batch default) and
+    walked whole (the large-batch one), both in longest-first order. Tolerance as for the single-stream decode
     step (chained kernels, rel/abs 1e-4)."""
     from oracle.decoder import decode_int8_step
     from qwenasr_amd.decoder import DecoderInt8Batched
@@ -751,3 +750,14 @@ def test_batched_decode_takes_weights_of_any_alignment(tmp_path, dev, B):
     for a, b in zip(got[:2], got[2:]):
         for x, y in zip(a, b):
             torch.testing.assert_close(x, y, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("H,I,B", [(2048, 6144, 9), (1024, 3072, 3), (1024, 3072, 1)])
+def test_batched_decode_step_on_the_general_projections(tmp_path, dev, monkeypatch, H, I, B):
+    """The same step where the digit rows do not run (one stream, other dimensions, weights off
+    alignment): B = 9 takes the matrix-core W8A32 projections (8+ rows), B = 3 and 1 the
+    per-row ones."""
+    from qwenasr_amd import decoder
+
+    monkeypatch.setattr(decoder, "_digit_weights", lambda w: False)
+    test_batched_decode_step_matches_the_oracle_per_stream(tmp_path, dev, H, I, B, None)

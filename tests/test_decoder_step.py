@@ -168,8 +168,8 @@ def test_fused_norm_decode_equals_unfused(tmp_path, dev):
     """The decode step with the add + RMSNorm folded into the projections and
     the head norm + cache store folded into attention (fuse_norms=True)
     equals the unfused sequence bit for bit: hidden state, logits, token and
-    cache rows, at positions where attention runs unsplit (0, 1) and split
-    (300-302)."""
+    cache rows, at positions where attention runs in one key split (0, 1) and in
+    several (300-302)."""
     from qwenasr_amd import qint8
     from qwenasr_amd.decoder import DecoderInt8
 
@@ -436,3 +436,118 @@ def test_prefill_predicates_tell_the_path(tmp_path, dev, monkeypatch):
             assert dec.prefill_norms_folded(T) == ("linear_int8_residual" in made), (T, made)
             if heads is None and norms is None:
                 assert dec.prefill_digits(T) == (T >= 5 and not 449 <= T <= 512), T
+
+
+@pytest.mark.parametrize("H,I,L,start,sizes", [
+    (1024, 3072, 2, 0, (37, 20)), (2048, 6144, 2, 0, (37, 20)),  # ragged token tiles, a second chunk
+    (1024, 3072, 2, 0, (4, 5, 8)),                               # the last size of the general path and the first after
+    (1024, 3072, 2, 300, (33, 40)), (2048, 6144, 1, 700, (77,)),  # the attention's keys in splits
+    (1024, 3072, 1, 0, (448,)), (1024, 3072, 1, 0, (449,)),      # both sides of the one-workgroup-per-CU band
+])
+def test_default_prefill_matches_the_oracle(tmp_path, dev, H, I, L, start, sizes):
+    """The prefill that a decoder built without options runs (digit rows wherever
+    prefill_digits says so), chunk after chunk over an earlier context of `start` rows, then a
+    decode step over the cache: the residual stream, every cache row, the final hidden state,
+    the logits and the token against the oracle, at the tolerance of the other forms. One row
+    of each chunk holds an element far above the rest, so that its projections take the floats
+    in place of the digits."""
+    from qwenasr_amd.decoder import DecoderInt8
+
+    nq, nk, hd, vocab = 16, 8, 128, 1000
+    kv, rows = nk * hd, start + sum(sizes) + 1
+    r = np.random.default_rng([42, H, start, sizes[0]])
+    w = small_decoder(r, H, I, L, nq, nk, hd, vocab)
+    dec = DecoderInt8(_load(tmp_path, w, L, dev), H, I, L, nq, nk, hd, max_seq=rows, device=dev)
+    kc, vc = np.zeros((L, rows, kv), np.float32), np.zeros((L, rows, kv), np.float32)
+    for c, block in ((kc, dec.kv.k_layer_block), (vc, dec.kv.v_layer_block)):
+        c[:, :start] = r.standard_normal((L, start, kv)).astype(np.float32)
+        for l in range(L):
+            block(l).view(-1, kv)[:start] = torch.from_numpy(c[l, :start]).to(dev)
+    dec.kv.len = start
+    for T in sizes:
+        X = r.standard_normal((T, H)).astype(np.float32)
+        X[T // 2, 11] = 2e3
+        x_ref = prefill_int8(w, kc, vc, start, X.ravel(), T, nq, nk, hd, threads=8)
+        assert dec.prefill_digits(T) == (T >= 5 and T != 449)
+        dec.prepare_prefill(start, T)
+        dec.prefill(torch.from_numpy(X.ravel()).to(dev), T, start)
+        torch.cuda.synchronize()
+        np.testing.assert_allclose(dec.px[:T * H].cpu().numpy(), x_ref, rtol=TOL, atol=TOL, err_msg=f"chunk at {start}")
+        start += T
+        assert dec.kv.len == start
+        for l in range(L):
+            np.testing.assert_allclose(dec.kv.k_layer(l).cpu().numpy().reshape(start, kv), kc[l, :start], rtol=TOL,
+                                       atol=TOL, err_msg=f"k rows layer {l}")
+            np.testing.assert_allclose(dec.kv.v_layer(l).cpu().numpy().reshape(start, kv), vc[l, :start], rtol=TOL,
+                                       atol=TOL, err_msg=f"v rows layer {l}")
+    e = r.standard_normal(H).astype(np.float32)
+    tok, xn, logits = decode_int8_step(w, kc, vc, start, e, nq, nk, hd, threads=8)
+    dec.prepare(start)
+    dec.decode(torch.from_numpy(e).to(dev), start)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(dec.x_norm.cpu().numpy(), xn, rtol=TOL, atol=TOL)
+    np.testing.assert_allclose(dec.logits.cpu().numpy(), logits, rtol=TOL, atol=TOL)
+    top2 = np.sort(logits)[-2:]
+    if top2[1] - top2[0] > 10 * TOL * max(1.0, abs(top2[1])):
+        assert int(dec.token.cpu()[0]) == tok
+
+
+@pytest.mark.parametrize("H,I,start,T", [(1024, 3072, 0, 64), (2048, 6144, 0, 64), (1024, 3072, 400, 77)])
+def test_default_prefill_graph_replays_equal_the_eager_call(dev, H, I, start, T):
+    """As test_graph_replays_equal_the_eager_calls, for the default prefill's digit rows: the
+    digits and exponents, one buffer for every launch, are rewritten by each; the marks of a
+    row that ranges too far come and go between the replays with the input."""
+    from qwenasr_amd import kernels as K
+    from qwenasr_amd.decoder import DecoderInt8
+
+    L, nq, nk, hd = 2, 16, 8, 128
+    g = torch.Generator(device=dev).manual_seed(43)
+
+    def randn(n, scale=1.0, mean=0.0):
+        return torch.randn(n, generator=g, device=dev) * scale + mean
+
+    def qw(o, i):
+        return K.QuantWeight(torch.randint(-127, 128, (o * i,), generator=g, device=dev, dtype=torch.int8),
+                             randn(o, 1e-4, 1e-3).abs_(), o, i)
+
+    layers = [{"wq": qw(nq * hd, H), "wk": qw(nk * hd, H), "wv": qw(nk * hd, H), "wo": qw(H, nq * hd),
+               "gate_up": qw(2 * I, H), "down": qw(H, I), "q_norm": randn(hd, 0.1, 1.0), "k_norm": randn(hd, 0.1, 1.0),
+               "input_norm": randn(H, 0.1, 1.0), "post_attn_norm": randn(H, 0.1, 1.0)} for _ in range(L)]
+    d = DecoderInt8({"layers": layers, "norm": randn(H, 0.1, 1.0), "lm_head": qw(100, H)}, H, I, L, nq, nk, hd,
+                    max_seq=start + T, device=dev)
+    d.kv.k.normal_(generator=g)
+    d.kv.v.normal_(generator=g)
+    assert d.prefill_digits(T)
+    d.kv.len = start
+    d.prepare_prefill(start, T)
+    plain = randn(T * H)
+    wide = plain.clone()
+    wide.view(T, H)[T // 2, 11] = 2e3
+    e = plain.clone()
+
+    def run():
+        d.kv.len = start
+        d.prefill(e, T, start)
+
+    def result():
+        torch.cuda.synchronize()
+        return [t.clone() for t in (d.px[:T * H], d.kv.k, d.kv.v)]
+
+    want = []
+    for x in (plain, wide):
+        e.copy_(x)
+        run()
+        want.append(result())
+        assert (d.pexps[:T] > -0x40000000).all()  # the last launch's rows: SwiGLU, within range
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for rep in range(4):
+        d.px.fill_(float("nan"))
+        for c in (d.kv.k, d.kv.v):
+            c.view(L, start + T, -1)[:, start:] = float("nan")
+        e.copy_((plain, wide)[rep % 2])
+        torch.cuda.synchronize()
+        graph.replay()
+        for a, b in zip(result(), want[rep % 2]):
+            assert torch.equal(a, b), f"replay {rep}"
