@@ -580,10 +580,10 @@ int qasr_decode_attention_linear_int8_f32(float* y, float* out, float* q, const 
  *
  * The _wide forms keep fp32 precision for every row: the writers mark a row
  * whose largest magnitude is above 128 times its mean magnitude, or which holds
- * an infinity or NaN (exps = QASR_DIGITS_WIDE_ROW, digits of no meaning), and the
+ * an infinity (exps = QASR_DIGITS_WIDE_ROW, digits of no meaning), and the
  * projections multiply marked rows in fp32 from x, the floats that the digits
- * were made from ([seq][in_dim], 16-byte aligned; only marked rows are read).
- * With x NULL a marked row gives NaN outputs. */
+ * were made from ([seq][in_dim], 16-byte aligned; only marked rows count). With x
+ * NULL a marked row gives NaN outputs. A row with a NaN gives NaN outputs. */
 #define QASR_DIGITS_WIDE_ROW (-0x40000001)
 int qasr_digit_rows_f32(int8_t* digits, int32_t* exps, const float* x, size_t rows, size_t cols,
                         void* stream);

@@ -19,7 +19,7 @@
 // at the few largest elements would be off by more than an fp32 sum. The writers
 // of digit rows therefore mark (when asked, kWideRow) each row whose largest
 // magnitude is above kWideRange times its mean magnitude, or which holds an
-// infinity or NaN; the GEMMs then multiply that row in fp32 precision from its
+// infinity and no NaN; the GEMMs then multiply that row in fp32 precision from its
 // floats (wide_rows below), in the token tiles that hold such a row alone. For
 // an unmarked row, leaving out its largest element leaves a row whose 2-norm is
 // at least max (cols / kWideRange - 1) / sqrt(cols), so the fixed point's error
@@ -36,7 +36,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kDigits = 4;
 constexpr int kDigitBits = 30;          // |I| <= 2^30
-constexpr int kBadRow = -0x40000000;    // exponent of a row with an infinity or NaN: its outputs are NaN
+constexpr int kBadRow = -0x40000000;    // exponent of a row with an infinity (unless marked wide) or NaN: NaN outputs
 constexpr int kWideRow = -0x40000001;   // exponent of a row that the GEMMs take from its floats
 constexpr float kWideRange = 128.0f;    // largest over mean magnitude from which a row is wide
 
@@ -138,16 +138,18 @@ __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
     const float m = fabsf(f);
     return m <= 3.402823466e38f ? m : __builtin_inff();
   };
-  float big = 0.0f, sum = 0.0f;  // the sum scaled by 2^-13 (cols <= 2^13): it cannot overflow
+  // the sum of magnitudes scaled by 2^-13 (cols <= 2^13) cannot overflow: NaN only from a NaN
+  float big = 0.0f, sum = 0.0f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const float m0 = mag(v[i].x), m1 = mag(v[i].y), m2 = mag(v[i].z), m3 = mag(v[i].w);
-    big = fmaxf(big, fmaxf(fmaxf(m0, m1), fmaxf(m2, m3)));
-    sum += (m0 * 0x1p-13f + m1 * 0x1p-13f) + (m2 * 0x1p-13f + m3 * 0x1p-13f);
+    big = fmaxf(big, fmaxf(fmaxf(mag(v[i].x), mag(v[i].y)), fmaxf(mag(v[i].z), mag(v[i].w))));
+    sum += (fabsf(v[i].x) * 0x1p-13f + fabsf(v[i].y) * 0x1p-13f) +
+           (fabsf(v[i].z) * 0x1p-13f + fabsf(v[i].w) * 0x1p-13f);
   }
   block_max_sum(big, sum, red);
   const bool bad = big == __builtin_inff();
-  const bool wide = a.wide && (bad || big > sum * (kWideRange * 0x1p13f / (float)a.cols));
+  // a NaN gives NaN outputs whatever the weights: not worth the floats
+  const bool wide = a.wide && sum == sum && (bad || big > sum * (kWideRange * 0x1p13f / (float)a.cols));
   const int up = bad ? 0 : kDigitBits - __builtin_amdgcn_frexp_expf(big);  // big < 2^exp (0 for a row of zeros)
   if (threadIdx.x == 0) a.exps[row] = wide ? kWideRow : bad ? kBadRow : -up;
   if constexpr (NORM) {
