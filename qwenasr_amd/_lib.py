@@ -52,7 +52,8 @@ SIGNATURES: dict[str, list] = {
     "qasr_causal_attention_f32": [P, P, P, P, Z, Z, Z, Z, Z, F, Z, P],
     "qasr_causal_attention_split_f32": [P, P, P, P, Z, Z, Z, Z, Z, F, Z, P, Z, P],
     "qasr_decode_attention_f32": [P, P, P, P, P, P, P, P, Z, Z, Z, Z, Z, F, F, P, P, Z, P, Z, P],
-    "qasr_decode_attention_linear_int8_f32": [P, P, P, P, P, P, P, P, P, Z, Z, Z, Z, Z, F, F, P, P, Z, P, Z, P, P, Z, P],
+    "qasr_decode_attention_linear_int8_f32": [P, P, P, P, P, P, P, P, P, Z, Z, Z, Z, Z, F, F, P, P, Z, P, Z, P, P, Z,
+                                              P],
     "qasr_lm_head_int8_argmax_f32": [P, P, P, P, P, Z, Z, Z, P, Z, P],
     "qasr_lm_head_int8_argmax_noalloc_f32": [P, P, P, P, P, Z, Z, Z, P],
     "qasr_probe_read": [c_int, c_int, ctypes.c_uint, P, Z, P, Z, Z, Z, Z, P],

@@ -1214,14 +1214,11 @@ struct DecodeLinear {
   size_t out_dim;
 };
 
-static int decode_attention(float* out, float* q, const float* k, const float* v,
-                                         const float* q_norm_w, const float* k_norm_w,
-                                         const float* cos_tab, const float* sin_tab,
-                                         size_t table_rows, size_t pos, size_t n_heads,
-                                         size_t n_kv_heads, size_t head_dim, float eps, float scale,
-                                         float* k_cache, float* v_cache, size_t cache_rows,
-                                         float* workspace, size_t workspace_floats,
-                                         const DecodeLinear* lin, void* stream) {
+static int decode_attention(float* out, float* q, const float* k, const float* v, const float* q_norm_w,
+                            const float* k_norm_w, const float* cos_tab, const float* sin_tab,
+                            size_t table_rows, size_t pos, size_t n_heads, size_t n_kv_heads, size_t head_dim,
+                            float eps, float scale, float* k_cache, float* v_cache, size_t cache_rows,
+                            float* workspace, size_t workspace_floats, const DecodeLinear* lin, void* stream) {
   if (n_heads == 0) return QASR_OK;
   QASR_REQUIRE(out && q && k && v && q_norm_w && k_norm_w && cos_tab && sin_tab && k_cache && v_cache,
                "decode_attention: null pointer");
@@ -1310,7 +1307,6 @@ extern "C" int qasr_decode_attention_linear_int8_f32(float* y, float* out, float
                           head_dim, eps, scale, k_cache, v_cache, cache_rows, workspace, workspace_floats, &lin,
                           stream);
 }
-
 
 // Keys per chunk of the batched decode attention: 512 (a 2 MB stream-head
 // walk becomes at most 4 workgroups, which evens out streams at different

@@ -350,7 +350,8 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
   extern __shared__ __align__(16) int8_t dg_lds[];
 
   unsigned bx, by;
-  const unsigned part = EPI == kDgPlain ? blockIdx.x / (a.cols * a.rows) : 0, block = blockIdx.x - part * a.cols * a.rows;
+  const unsigned part = EPI == kDgPlain ? blockIdx.x / (a.cols * a.rows) : 0;
+  const unsigned block = blockIdx.x - part * a.cols * a.rows;
   if (a.split_cols == 0) {
     bx = block % a.cols;
     by = block / a.cols;
@@ -623,7 +624,12 @@ bool run_digit_gemm(DigitGemm a, hipStream_t st) {
 //   256 x 64, one workgroup a CU   2.5 + ceil(n / 256) (5.2 + 12.7 K')
 //   128 x 32, two a CU             5   + max(1, n / 256) 5.2 K'
 //   64 x 32, K over 4 wave groups  2.5 + ceil(n / 256) (2.6 + 3.6 K')
-//   32 x 32, K over 4 waves        3.5 + max(1, n / 256) 3.6 K' (half of it when a CU has one)
+//   32 x 32, K over 4 waves        3.5 + 1.8 K' up to n = 256, then 3.5 + n / 256 3.6 K'
+// A CU holds one 32 x 32 workgroup (82 KB of LDS): 256 tiles are one round, 257 two.
+// That tile measured at 64 tokens and K' = 1, 2 and 6: 64 tiles 5.7, 7.3 and 14.0 us,
+// 256 7.0, 9.1 and 21.6, 320 10.7, 14.7 and 35.8, 512 11.9, 16.1 and 44.4 (64 x 32 on
+// the same products, half the tiles: 6.3, 8.4, 17.5; 6.6, 8.8, 21.9; 6.9, 9.1, 22.9;
+// 7.9, 10.8, 26.1).
 // Measured on one MI355X against the bf16 three-way split kernels (int8.hip)
 // for the same product: 1473 tokens [2048 -> 12288] 163 us against 242 (1.8e15
 // int8 operations a second, 74% of what the same matrix instructions reach
@@ -641,7 +647,8 @@ bool launch_digit_gemm(const DigitGemm& a, hipStream_t st) {
       for (int m = 0; m < a.n; ++m) c += (a.N[m] + bn - 1) / bn;
       return (double)(c * ((a.T + bt - 1) / bt) * a.parts) / 256.0;
     };
-    const double k = a.K / (1024.0 * a.parts), t32 = tiles(32, 32), t64 = tiles(64, 32), t128 = tiles(128, 32), t256 = tiles(256, 64);
+    const double k = a.K / (1024.0 * a.parts);
+    const double t32 = tiles(32, 32), t64 = tiles(64, 32), t128 = tiles(128, 32), t256 = tiles(256, 64);
     const double c256 = 2.5 + ceil(t256) * (5.2 + 12.7 * k);
     const double c128 = 5.0 + (t128 > 1.0 ? t128 : 1.0) * 5.2 * k;
     const double c64 = 2.5 + ceil(t64) * (2.6 + 3.6 * k);
@@ -701,7 +708,8 @@ static int digit_rows(int8_t* digits, int32_t* exps, const float* x, size_t rows
     return fail(QASR_ERR_UNSUPPORTED, "digit_rows: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
   const DigitArgs a{digits, exps, const_cast<float*>(x), nullptr, nullptr, nullptr, (int)rows, (int)cols, 1, 0.0f,
                     wide};
-  launch_digit_rows<false>(a, as_stream(stream));
+  if (!launch_digit_rows<false>(a, as_stream(stream)))
+    return fail(QASR_ERR_UNSUPPORTED, "digit_rows: no kernel for this row length");
   return launch_status("digit_rows");
 }
 
@@ -727,7 +735,8 @@ static int add_rms_norm_digits(float* x, const float* delta, size_t delta_parts,
     return fail(QASR_ERR_UNSUPPORTED,
                 "add_rms_norm_digits: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
   const DigitArgs a{digits, exps, x, delta, weight, x_norm, (int)rows, (int)cols, (int)delta_parts, eps, wide};
-  launch_digit_rows<true>(a, as_stream(stream));
+  if (!launch_digit_rows<true>(a, as_stream(stream)))
+    return fail(QASR_ERR_UNSUPPORTED, "add_rms_norm_digits: no kernel for this row length");
   return launch_status("add_rms_norm_digits");
 }
 

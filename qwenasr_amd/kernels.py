@@ -677,8 +677,8 @@ def add_rms_norm_linear_nobias_int8_multi(ys, ws: list, h_out, x, delta, norm_w,
     then 881-886). ``h_out`` (None: not written) gets h and must be a different
     buffer from x and delta; ``ys[m]`` equals add_rms_norm + linear_nobias_int8_multi
     bit for bit."""
-    _call.qasr_add_rms_norm_linear_nobias_int8_multi_f32(ys, ws, h_out, in_dim, x, in_dim, delta, in_dim, norm_w, in_dim,
-                                                         in_dim, eps)
+    _call.qasr_add_rms_norm_linear_nobias_int8_multi_f32(ys, ws, h_out, in_dim, x, in_dim, delta, in_dim, norm_w,
+                                                         in_dim, in_dim, eps)
 
 
 def add_rms_norm_gate_up_swiglu_int8(out, h_out, x, delta, norm_w, w: QuantWeight, in_dim: int,

@@ -281,7 +281,7 @@ def test_wide_rows_in_the_other_epilogues(dev):
     flat = x.view(-1)
     w.scales.mul_(2e-4)
     dg, ex = _digits_wide(x, dev)
-    gu, out, ref = torch.empty(T * 2 * inter, device=dev), torch.empty(T * inter, device=dev), torch.empty(T * inter, device=dev)
+    gu, out, ref = (torch.empty(T * n, device=dev) for n in (2 * inter, inter, inter))
     K.linear_digits_int8([gu], [w], dg, ex, T, H, x=flat)
     K.swiglu_multiply(ref, gu, T, inter)
     K.gate_up_swiglu_digits_int8(out, w, dg, ex, T, H, inter, prefill=True, x=flat)
@@ -322,7 +322,8 @@ def test_add_rms_norm_digits_marks_wide_rows(dev):
         K.add_rms_norm_digits(c, None, g, own, dg2, ex3, rows, cols, 1e-6, wide=True, all_rows=False)
         marked = [2]  # an infinity's row is normalised to NaN
         rest = [i for i in range(rows) if i not in marked]
-        assert (ex2[marked] == -0x40000001).all() and int(ex2[4]) == -0x40000000 and torch.equal(ex2, ex3) and torch.equal(ex[rest], ex2[rest])
+        assert (ex2[marked] == -0x40000001).all() and int(ex2[4]) == -0x40000000
+        assert torch.equal(ex2, ex3) and torch.equal(ex[rest], ex2[rest])
         assert torch.equal(dg.view(4, rows, cols)[:, rest], dg2.view(4, rows, cols)[:, rest])
         torch.testing.assert_close(xn, plain, rtol=0, atol=0, equal_nan=True)
         own = own.view(rows, cols)
@@ -361,7 +362,8 @@ def test_lm_head_row_with_an_infinity(dev, rows):
     col = w.data.view(vocab, K_)[:, 3]
     col[col == 0] = -1
     idx, logits = torch.empty(rows, dtype=torch.int32, device=dev), torch.empty(rows * vocab, device=dev)
-    K.lm_head_int8_argmax(idx, logits, x.view(-1), w, rows, K_, vocab, torch.empty(1 << 20, dtype=torch.uint8, device=dev))
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device=dev)
+    K.lm_head_int8_argmax(idx, logits, x.view(-1), w, rows, K_, vocab, ws)
     assert torch.equal(logits.view(rows, vocab)[1], torch.where(col > 0, float("inf"), float("-inf")))
     assert int(idx[1]) == int((col > 0).nonzero()[0])
 
