@@ -57,6 +57,7 @@ struct DigitArgs {
   int rows, cols, parts;
   float eps;
   int wide;            // DigitWide; kWideOwnNorm: x_norm gets the wide rows alone
+  float wide_sum;      // kWideRange / cols: times a row's sum of magnitudes, the line
 };
 
 // The largest of `big` and the sum of `sum` over a workgroup of 256, in one pass
@@ -138,29 +139,20 @@ __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
     const float m = fabsf(f);
     return m <= 3.402823466e38f ? m : __builtin_inff();
   };
-  // the sum of magnitudes scaled by 2^-13 (cols <= 2^13) cannot overflow: NaN only from a NaN
-  float big = 0.0f, sum = 0.0f;
+  float big = 0.0f, sum = 0.0f;  // of the magnitudes
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     big = fmaxf(big, fmaxf(fmaxf(mag(v[i].x), mag(v[i].y)), fmaxf(mag(v[i].z), mag(v[i].w))));
-    sum += (fabsf(v[i].x) * 0x1p-13f + fabsf(v[i].y) * 0x1p-13f) +
-           (fabsf(v[i].z) * 0x1p-13f + fabsf(v[i].w) * 0x1p-13f);
+    sum += (fabsf(v[i].x) + fabsf(v[i].y)) + (fabsf(v[i].z) + fabsf(v[i].w));
   }
   block_max_sum(big, sum, red);
   const bool bad = big == __builtin_inff();
-  // a NaN gives NaN outputs whatever the weights: not worth the floats
-  const bool wide = a.wide && sum == sum && (bad || big > sum * (kWideRange * 0x1p13f / (float)a.cols));
+  // The sum is infinite for a row with an infinity and for one of floats so large
+  // that it overflows (marked too: its range is not known), NaN only for a row with
+  // a NaN, whose outputs are NaN whatever the weights: not worth the floats.
+  const bool wide = a.wide && (sum == __builtin_inff() || big > sum * a.wide_sum) && sum == sum;
   const int up = bad ? 0 : kDigitBits - __builtin_amdgcn_frexp_expf(big);  // big < 2^exp (0 for a row of zeros)
   if (threadIdx.x == 0) a.exps[row] = wide ? kWideRow : bad ? kBadRow : -up;
-  if constexpr (NORM) {
-    if (a.wide == kWideOwnNorm && wide) {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int c = threadIdx.x + 256 * i;
-        if (c < n4) st4(a.x_norm + (size_t)row * a.cols, c, v[i]);
-      }
-    }
-  }
   // byte d of (I + 0x00808080) ^ 0x00808080 is digit d: adding 128 to the lower
   // three bytes carries into the next one where a digit is negative
   auto digits_of = [&](float f) {
@@ -181,6 +173,15 @@ __global__ __launch_bounds__(256) void digit_rows_kernel(DigitArgs a) {
     *reinterpret_cast<unsigned*>(out + plane) = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
     *reinterpret_cast<unsigned*>(out + 2 * plane) = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
     *reinterpret_cast<unsigned*>(out + 3 * plane) = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+  }
+  if constexpr (NORM) {
+    if (a.wide == kWideOwnNorm && wide) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int c = threadIdx.x + 256 * i;
+        if (c < n4) st4(a.x_norm + (size_t)row * a.cols, c, v[i]);
+      }
+    }
   }
 }
 
@@ -408,11 +409,9 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
   float* sc_lds = reinterpret_cast<float*>(dg_lds + TILE_BYTES);
   int* ex_lds = reinterpret_cast<int*>(sc_lds + BN);
   if ((int)threadIdx.x < BN) sc_lds[threadIdx.x] = scales[min(n0 + (int)threadIdx.x, N - 1)];
-  if ((int)threadIdx.x < BT) {
-    const int e = a.exps[min(t0 + (int)threadIdx.x, a.T - 1)];
-    ex_lds[threadIdx.x] = e == kWideRow && a.x ? 0 : e;  // a wide row's floats have no power of two
-  }
-  const int t_wave = min(t0 + 32 * wc + r, a.T - 1), e_wave = a.exps[t_wave];  // looked at after the loop
+  if ((int)threadIdx.x < BT) ex_lds[threadIdx.x] = a.exps[min(t0 + (int)threadIdx.x, a.T - 1)];
+  const int t_wave = min(t0 + 32 * wc + r, a.T - 1);
+  int e_wave;  // of this lane's token, looked at after the loop
   v4i st[U];
   {
     v4i first[U];
@@ -421,6 +420,7 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
     const int k = min(1, nch - 1) * BK;
 #pragma unroll
     for (int u = 0; u < U; ++u) st[u] = *reinterpret_cast<const v4i*>(src[u] + k);
+    e_wave = a.exps[t_wave];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < U; ++u) *reinterpret_cast<v4i*>(buf + dst[u]) = first[u];
@@ -508,7 +508,8 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
     }
   }
   __syncthreads();
-  // a sum of products times the token's power of two
+  // a token's power of two (a wide row's floats have none), and a sum of products times it
+  auto power = [&](int tt) { return ex_lds[tt] == kWideRow && a.x ? 0 : ex_lds[tt]; };
   auto powered = [](float v, int ex) { return ex <= kBadRow ? qnan() : ldexpf(v, ex); };
   if constexpr (EPI == kDgHeads) {
     // 16 lanes a head: lane `sub` holds dims 4 sub.. and 64 + 4 sub..
@@ -524,7 +525,7 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
       const size_t pos = (size_t)(he.start_pos + min(t, a.T - 1)), trow = pos * 128;
       const float4 c1 = ld4(he.cos_tab + trow, sub), c2 = ld4(he.cos_tab + trow + 64, sub);
       const float4 s1 = ld4(he.sin_tab + trow, sub), s2 = ld4(he.sin_tab + trow + 64, sub);
-      const int ex = ex_lds[tt];
+      const int ex = power(tt);
       auto value = [&](int c) {
         float4 f = *reinterpret_cast<const float4*>(tile + (size_t)tt * PITCH + c);
 #pragma unroll
@@ -566,7 +567,7 @@ __global__ __launch_bounds__(64 * KW * (BN / (32 * MI)) * (BT / 32), 2) void dig
       f.x += p.x; f.y += p.y; f.z += p.z; f.w += p.w;
     }
     const float4 sc = *reinterpret_cast<const float4*>(sc_lds + c);
-    const int ex = ex_lds[tt];
+    const int ex = power(tt);
     float res[4] = {f.x * sc.x, f.y * sc.y, f.z * sc.z, f.w * sc.w};
 #pragma unroll
     for (int v = 0; v < 4; ++v) res[v] = powered(res[v], ex);
@@ -707,7 +708,7 @@ static int digit_rows(int8_t* digits, int32_t* exps, const float* x, size_t rows
   if (cols == 0 || cols % 4 != 0 || cols > 8192 || !aligned16(x) || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED, "digit_rows: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
   const DigitArgs a{digits, exps, const_cast<float*>(x), nullptr, nullptr, nullptr, (int)rows, (int)cols, 1, 0.0f,
-                    wide};
+                    wide, kWideRange / (float)cols};
   if (!launch_digit_rows<false>(a, as_stream(stream)))
     return fail(QASR_ERR_UNSUPPORTED, "digit_rows: no kernel for this row length");
   return launch_status("digit_rows");
@@ -734,7 +735,8 @@ static int add_rms_norm_digits(float* x, const float* delta, size_t delta_parts,
       !aligned16(x_norm) || !aligned16(digits) || !aligned4(exps))
     return fail(QASR_ERR_UNSUPPORTED,
                 "add_rms_norm_digits: cols must be a multiple of 4 up to 8192, buffers 16-byte aligned");
-  const DigitArgs a{digits, exps, x, delta, weight, x_norm, (int)rows, (int)cols, (int)delta_parts, eps, wide};
+  const DigitArgs a{digits, exps, x, delta, weight, x_norm, (int)rows, (int)cols, (int)delta_parts, eps, wide,
+                    kWideRange / (float)cols};
   if (!launch_digit_rows<true>(a, as_stream(stream)))
     return fail(QASR_ERR_UNSUPPORTED, "add_rms_norm_digits: no kernel for this row length");
   return launch_status("add_rms_norm_digits");

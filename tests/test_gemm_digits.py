@@ -232,6 +232,21 @@ def _error(got, ref):  # of each row, against 64 bits
     return (got.double() - ref).norm(dim=-1) / ref.norm(dim=-1)
 
 
+def test_which_rows_are_marked(dev):
+    x = torch.randn(7, 1024, device=dev)
+    x[1] = 3e38                    # the sum of magnitudes overflows: marked
+    x[2] = 0.0
+    x[3, 1:] = 0.0                 # one element: 1024 times the mean
+    x[4] *= 1e-42                  # subnormal, no outlier
+    x[5] = 1.0
+    x[5, 9] = 128 * 1023 / 896.0   # 128 times the mean, to rounding
+    x[5, 9] *= 1.001
+    x[6] = 1.0
+    x[6, 9] = 128 * 1023 / 896.0 * 0.999
+    _, ex = _digits_wide(x, dev)
+    assert (ex == -0x40000001).tolist() == [False, True, False, True, False, True, False]
+
+
 # one shape per tile (32 x 32, 64 x 32, 128 x 32, 256 x 64), ragged in rows and tokens, and a long sum
 @pytest.mark.parametrize("T,K_,N", [(9, 512, 1028), (65, 1024, 4096), (70, 512, 33028), (300, 1024, 12292),
                                     (12, 6144, 2048)])
