@@ -31,8 +31,9 @@ alone, K of them), and its algorithmic bytes per launch give
 roofline.achieved.
 
 Prints ONE JSON line: the headline workload's value, roofline and CPU
-baseline, and under "configs" the other workloads measured in the same run,
-each with its per-kernel figures and its own CPU baseline. The CPU baseline is
+baseline, and under "configs" the step time, rate, tokens/s and CPU tokens/s of
+the other workloads measured in the same run (their per-kernel figures go to
+stderr, and with their CPU samples to the file of --details). The CPU baseline is
 the oracle (a C restatement of the reference Rust kernels, compiled here with
 -march=native) timed on this host for a bounded sample.
 """
@@ -1567,6 +1568,16 @@ def summary(wl, m: dict, cpu) -> dict:
     return out
 
 
+def brief(c: dict) -> dict:
+    """A config's figures for the printed line, which has to survive a log that keeps its
+    last few KB (the kernels are on stderr and under --details)."""
+    out = {k: c[k] for k in ("us_per_step", "GB/s", "tokens_per_s", "dtype")}
+    cpu = c.get("cpu_baseline")
+    if cpu:
+        out["cpu_tokens_per_s"] = cpu.get("tokens_per_s")
+    return out
+
+
 def free(torch, wl) -> None:
     import gc
 
@@ -1586,6 +1597,8 @@ def main() -> int:
     ap.add_argument("--configs", default=DEFAULT_CONFIGS,
                     help="comma-separated workloads also measured in this run, each reported under "
                          "'configs' with its own CPU baseline ('none' for none)")
+    ap.add_argument("--details", metavar="FILE",
+                    help="also write the line with every config's workload, kernels and CPU sample (20 KB) here")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-seconds", type=float, default=10.0, help="CPU sample of the headline workload")
     ap.add_argument("--config-cpu-seconds", type=float, default=4.0, help="CPU sample of each other config")
@@ -1690,7 +1703,7 @@ def main() -> int:
         configs[name] = summary(cw, cm, ccpu)
         free(torch, cw)
     if configs:
-        out["configs"] = configs
+        out["configs"] = {n: brief(c) for n, c in configs.items()}
     if "decode_step" in configs:
         out["decode_tokens_per_s"] = configs["decode_step"]["tokens_per_s"]
     if "decode_step_b256" in configs:
@@ -1699,6 +1712,8 @@ def main() -> int:
         out["batched_decode_w8a8_tokens_per_s"] = configs["decode_step_b256_w8a8"]["tokens_per_s"]
     if "prefill_step" in configs:
         out["prefill_tokens_per_s"] = configs["prefill_step"]["tokens_per_s"]
+    if args.details:
+        Path(args.details).write_text(json.dumps({**out, "configs": configs}))
     print(json.dumps(out), flush=True)
     return 0
 
